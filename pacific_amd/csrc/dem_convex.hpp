@@ -26,6 +26,18 @@ namespace dem {
 constexpr double kEps2 = 1.e-15;  // Basic.hh EPSILON2
 constexpr double kEps3 = 1.e-20;  // Basic.hh EPSILON3
 
+// Work area of one distance search: the simplex of up to four points of the
+// Minkowski difference by slot -- y (entries 0-11), the support points p and q
+// in the local frames (12-23, 24-35) and the weight of each kept slot (36-39)
+// -- with entry e at a[e * st].  On the device it lies in LDS, one column per
+// lane, so that slots are addressed at run time without scratch memory or a
+// copy of the code per slot.
+constexpr int kGjkWork = 40;
+struct GjkWork {
+  double* a;
+  int st;
+};
+
 // A rigid body with crust as ClosestPoint sees it
 struct ConvexGeo {
   int type, nv;
@@ -39,6 +51,7 @@ struct ConvexGeo {
   double crust, circR;
   d3 obb;         // OBB half extents at the identity (bounding-volume pre-test)
   GjkOpts opt;    // the system's narrow-phase options
+  GjkWork work{nullptr, 1};  // body A's: the search's work area (device)
 };
 
 struct Tf {
@@ -68,6 +81,16 @@ DEM_HD Tf tf_scaled(const ConvexGeo& g, d3 sc) {
   return t;
 }
 
+// norm(v) < 1e-10 and norm(v) > 1e-10 without the square root: the squares
+// at which the correctly rounded root crosses the bound.
+DEM_HD bool norm_below_eps(d3 v) { return v.x * v.x + v.y * v.y + v.z * v.z < 0x1.79ca10c924223p-67; }
+DEM_HD bool norm_above_eps(d3 v) { return v.x * v.x + v.y * v.y + v.z * v.z > 0x1.79ca10c924224p-67; }
+
+// Vertices of a polyhedron are scanned in groups of this many; the vertex
+// table holds each shape's vertices filled up to whole groups with copies of
+// the last one (never the first maximum).
+constexpr int kVertGroup = 4;
+
 DEM_HD d3 support(const ConvexGeo& g, d3 v) {
   if (g.type == kShapeSphere) {
     double s = norm(v);
@@ -78,45 +101,40 @@ DEM_HD d3 support(const ConvexGeo& g, d3 v) {
     return d3{0., 0., 0.};
   }
   if (g.type == kShapeBox) {
-    double n = norm(v);
-    if (n < kEps) return d3{0., 0., 0.};
+    if (norm_below_eps(v)) return d3{0., 0., 0.};
     return d3{v.x < 0. ? -g.e.x : g.e.x, v.y < 0. ? -g.e.y : g.e.y, v.z < 0. ? -g.e.z : g.e.z};
   }
-  double n = norm(v);
-  if (!(n > kEps)) return d3{0., 0., 0.};
+  if (!norm_above_eps(v)) return d3{0., 0., 0.};
+  // the first maximum; a group's loads overlap
   const double* p = g.verts;
-  d3 best{p[0], p[1], p[2]};
-  double h = dot(best, v);
-  for (int i = 1; i < g.nv; ++i) {
-    d3 c{p[3 * i], p[3 * i + 1], p[3 * i + 2]};
-    double d = dot(c, v);
-    if (d > h) {
-      h = d;
-      best = c;
+  int best = 0;
+  double h = -INFINITY;
+  for (int i = 0; i < g.nv; i += kVertGroup) {
+    double d[kVertGroup];
+#pragma unroll
+    for (int u = 0; u < kVertGroup; ++u) {
+      const double* c = p + 3 * (i + u);
+      d[u] = dot(d3{c[0], c[1], c[2]}, v);
+    }
+#pragma unroll
+    for (int u = 0; u < kVertGroup; ++u) {
+      const bool more = d[u] > h;
+      h = more ? d[u] : h;
+      best = more ? i + u : best;
     }
   }
-  return best;
+  return d3{p[3 * best], p[3 * best + 1], p[3 * best + 2]};
 }
 
 // --- Johnson sub-distance algorithm -----------------------------------------
-// The simplex of up to four points of the Minkowski difference and the
-// determinant cache of Convex.cpp:219-435, with the same arithmetic in the
-// same order.  Every table index below is a compile-time constant -- the
-// slot of the point being added is a template argument, the subsets are
-// enumerated by unrolled loops -- so that the tables live in registers; the
-// run-time masks only pick which of the constant-indexed branches runs.
-// Only the 32 entries det[s][i] with i in s and the upper triangle of the
-// symmetric dot-product table are ever read.
-struct Simplex {
-  d3 y[4], p[4], q[4];
-  double det[16][4];
-  double dp[10];  // y_i . y_j for i <= j
-};
-
-// index of y_i . y_j in Simplex::dp, a constant expression (the tables are
-// addressed at compile time only)
-template <int I, int J>
-constexpr int kDp = I <= J ? I * 4 - I * (I - 1) / 2 + (J - I) : J * 4 - J * (J - 1) / 2 + (I - J);
+DEM_HD d3 work_get(const GjkWork& W, int e) { return d3{W.a[e * W.st], W.a[(e + 1) * W.st], W.a[(e + 2) * W.st]}; }
+DEM_HD void work_put(const GjkWork& W, int e, d3 v) {
+  W.a[e * W.st] = v.x;
+  W.a[(e + 1) * W.st] = v.y;
+  W.a[(e + 2) * W.st] = v.z;
+}
+DEM_HD d3 work_y(const GjkWork& W, int slot) { return work_get(W, 3 * slot); }
+DEM_HD double& work_w(const GjkWork& W, int slot) { return W.a[(36 + slot) * W.st]; }
 
 // f(integral_constant<int, i>) for i = B, B+1, ..., E-1
 template <int B, int E, class F>
@@ -126,186 +144,235 @@ DEM_HD void sfor(F&& f) {
     sfor<B + 1, E>(f);
   }
 }
-// f(integral_constant<int, i>) for i = B, B-1, ..., E+1
-template <int B, int E, class F>
-DEM_HD void sfor_down(F&& f) {
-  if constexpr (B > E) {
-    f(std::integral_constant<int, B>{});
-    sfor_down<B - 1, E>(f);
+
+// The determinants of computeDet (Convex.cpp:219-268) for subsets picked at
+// run time, from the points in the work area; f is the slot just added, and
+// the triple without it is the one kept by the last step, whose determinants
+// are the weights in the work area.  Only the backup procedure below needs
+// subsets by number; it runs once per search at most.
+DEM_HD double j_det3(const GjkWork& W, unsigned s, int i, int f) {
+  if (!(s & (1u << f))) return work_w(W, i);
+  // k < j the other two
+  const unsigned o = s & ~(1u << f);
+  const int k = __builtin_ctz(o), j = __builtin_ctz(o & (o - 1));
+  const d3 yk = work_y(W, k), yj = work_y(W, j), yl = work_y(W, f);
+  const double kk = dot(yk, yk), jj = dot(yj, yj), ll = dot(yl, yl), jk = dot(yk, yj), lk = dot(yk, yl), lj = dot(yj, yl);
+  if (i == k) return (ll - lj) * (jj - jk) + (jj - lj) * (lj - lk);
+  if (i == j) return (ll - lk) * (kk - jk) + (kk - lk) * (lk - lj);
+  return (jj - jk) * (kk - lk) + (kk - jk) * (jk - lj);
+}
+DEM_HD double j_det_of(const GjkWork& W, unsigned s, int i, int f) {
+  const int c = __builtin_popcount(s);
+  if (c == 1) return 1.;
+  const unsigned rest = s & ~(1u << i);
+  if (c == 2) {
+    const d3 yi = work_y(W, i), yo = work_y(W, __builtin_ctz(rest));
+    return dot(yo, yo) - dot(yi, yo);
   }
+  if (c == 3) return j_det3(W, s, i, f);
+  const int r = __builtin_ctz(rest);
+  double det = 0.;
+  bool first = true;
+  for (unsigned m = rest; m; m &= m - 1) {
+    const int j = __builtin_ctz(m);
+    const d3 yj = work_y(W, j);
+    const double t = j_det3(W, rest, j, f) * (dot(yj, work_y(W, r)) - dot(yj, work_y(W, i)));
+    det = first ? t : det + t;
+    first = false;
+  }
+  return det;
 }
 
-// computeDet (Convex.cpp:219-268) for the point just added in slot LAST
-template <int LAST>
-DEM_HD void j_det(Simplex& S, unsigned bits, unsigned all_bits) {
-  constexpr unsigned last_bit = 1u << LAST;
-  sfor<0, 4>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    if constexpr (i != LAST)
-      if (bits & (1u << i)) S.dp[kDp<i, LAST>] = dot(S.y[i], S.y[LAST]);
-  });
-  S.dp[kDp<LAST, LAST>] = dot(S.y[LAST], S.y[LAST]);
-  S.det[last_bit][LAST] = 1.;
-  sfor<0, 4>([&](auto J) {
-    constexpr int j = decltype(J)::value;
-    if constexpr (j != LAST) {
-      constexpr unsigned sj = 1u << j, s2 = sj | last_bit;
-      if (bits & sj) {
-        S.det[s2][j] = S.dp[kDp<LAST, LAST>] - S.dp[kDp<LAST, j>];
-        S.det[s2][LAST] = S.dp[kDp<j, j>] - S.dp[kDp<j, LAST>];
-        sfor<0, j>([&](auto K) {
-          constexpr int k = decltype(K)::value;
-          if constexpr (k != LAST) {
-            constexpr unsigned sk = 1u << k, s3 = sk | s2;
-            if (bits & sk) {
-              S.det[s3][k] = S.det[s2][j] * (S.dp[kDp<j, j>] - S.dp[kDp<j, k>]) +
-                             S.det[s2][LAST] * (S.dp[kDp<LAST, j>] - S.dp[kDp<LAST, k>]);
-              S.det[s3][j] = S.det[sk | last_bit][k] * (S.dp[kDp<k, k>] - S.dp[kDp<k, j>]) +
-                             S.det[sk | last_bit][LAST] * (S.dp[kDp<LAST, k>] - S.dp[kDp<LAST, j>]);
-              S.det[s3][LAST] = S.det[sk | sj][k] * (S.dp[kDp<k, k>] - S.dp[kDp<k, LAST>]) +
-                                S.det[sk | sj][j] * (S.dp[kDp<j, k>] - S.dp[kDp<j, LAST>]);
-            }
-          }
-        });
+// The backup procedure of closest (Convex.cpp:389-414): the subset of
+// all_bits with positive determinants whose point is nearest to the origin.
+DEM_HD void j_backup(const GjkWork& W, unsigned& bits, unsigned all_bits, int f, d3& v) {
+  double min_dist2 = INFINITY, w[4] = {0., 0., 0., 0.};
+  unsigned best = 0u;
+#pragma nounroll
+  for (unsigned s = 15u; s > 0u; --s) {
+    if ((s & all_bits) != s) continue;
+    bool proper = true;
+    double sum = 0., det[4] = {0., 0., 0., 0.};
+    d3 u{0., 0., 0.};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s & (1u << i)) {
+        det[i] = j_det_of(W, s, i, f);
+        if (det[i] <= kEps3) proper = false;
+        sum += det[i];
+        u += det[i] * work_y(W, i);
       }
+    if (!proper) continue;
+    u *= 1. / sum;
+    const double d2 = dot(u, u);
+    if (d2 < min_dist2) {
+      min_dist2 = d2;
+      best = s;
+      v = u;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = det[i];
     }
-  });
-  if (all_bits == 15) {
-    const double* dp = S.dp;
-    S.det[15][0] = S.det[14][1] * (dp[kDp<1, 1>] - dp[kDp<1, 0>]) + S.det[14][2] * (dp[kDp<2, 1>] - dp[kDp<2, 0>]) +
-                   S.det[14][3] * (dp[kDp<3, 1>] - dp[kDp<3, 0>]);
-    S.det[15][1] = S.det[13][0] * (dp[kDp<0, 0>] - dp[kDp<0, 1>]) + S.det[13][2] * (dp[kDp<2, 0>] - dp[kDp<2, 1>]) +
-                   S.det[13][3] * (dp[kDp<3, 0>] - dp[kDp<3, 1>]);
-    S.det[15][2] = S.det[11][0] * (dp[kDp<0, 0>] - dp[kDp<0, 2>]) + S.det[11][1] * (dp[kDp<1, 0>] - dp[kDp<1, 2>]) +
-                   S.det[11][3] * (dp[kDp<3, 0>] - dp[kDp<3, 2>]);
-    S.det[15][3] = S.det[7][0] * (dp[kDp<0, 0>] - dp[kDp<0, 3>]) + S.det[7][1] * (dp[kDp<1, 0>] - dp[kDp<1, 3>]) +
-                   S.det[7][2] * (dp[kDp<2, 0>] - dp[kDp<2, 3>]);
   }
+  if (!best) return;
+  bits = best;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (best & (1u << i)) work_w(W, i) = w[i];
 }
-// valid (Convex.cpp:272-290) for the subset SS
-template <unsigned SS>
-DEM_HD bool j_valid(const Simplex& S, unsigned all_bits) {
-  bool ok = true;
-  sfor<0, 4>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    constexpr unsigned bit = 1u << i;
-    if (!ok || !(all_bits & bit)) return;
-    if constexpr ((SS & bit) != 0u) {
-      if (S.det[SS][i] <= kEps3) ok = false;
-    } else {
-      if (S.det[SS | bit][i] > 0.) ok = false;
-    }
-  });
-  return ok;
-}
-// computeVector (Convex.cpp:294-306)
-template <unsigned SS>
-DEM_HD d3 j_vector(const Simplex& S) {
-  double sum = 0.;
-  d3 v{0., 0., 0.};
-  sfor<0, 4>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    if constexpr ((SS & (1u << i)) != 0u) {
-      sum += S.det[SS][i];
-      v += S.det[SS][i] * S.y[i];
-    }
-  });
-  v *= 1. / sum;
-  return v;
-}
-// computePoints (Convex.cpp:310-327)
-template <unsigned SS>
-DEM_HD void j_points_t(const Simplex& S, d3& p1, d3& p2) {
-  double sum = 0.;
-  p1 = d3{0., 0., 0.};
-  p2 = d3{0., 0., 0.};
-  sfor<0, 4>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    if constexpr ((SS & (1u << i)) != 0u) {
-      sum += S.det[SS][i];
-      p1 += S.det[SS][i] * S.p[i];
-      p2 += S.det[SS][i] * S.q[i];
-    }
-  });
-  double s = 1. / sum;
-  p1 *= s;
-  p2 *= s;
-}
-DEM_HD void j_points(const Simplex& S, unsigned bits, d3& p1, d3& p2) {
-  bool done = false;
-  sfor_down<15, -1>([&](auto B) {
-    constexpr unsigned b = (unsigned)decltype(B)::value;
-    if (!done && bits == b) {
-      j_points_t<b>(S, p1, p2);
-      done = true;
-    }
-  });
-}
-// proper (Convex.cpp:331-338)
-template <unsigned SS>
-DEM_HD bool j_proper(const Simplex& S) {
-  bool ok = true;
-  sfor<0, 4>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    if constexpr ((SS & (1u << i)) != 0u)
-      if (S.det[SS][i] <= kEps3) ok = false;
-  });
-  return ok;
-}
-// closest (Convex.cpp:342-414): the smallest valid subset containing LAST,
-// else the backup procedure over every proper subset
-template <int LAST>
-DEM_HD bool j_closest(Simplex& S, unsigned& bits, unsigned all_bits, d3& v) {
-  constexpr unsigned last_bit = 1u << LAST;
-  j_det<LAST>(S, bits, all_bits);
-  bool found = false;
-  sfor_down<15, 0>([&](auto SI) {
-    constexpr unsigned s = (unsigned)decltype(SI)::value;
-    if constexpr ((s & last_bit) == 0u) {
-      if (!found && (s & bits) == s && j_valid<s | last_bit>(S, all_bits)) {
-        bits = s | last_bit;
-        v = j_vector<s | last_bit>(S);
-        found = true;
+
+// closest (Convex.cpp:342-414) for the point w just added in slot f, the
+// first free one: the smallest valid subset containing it, else the backup
+// procedure.  The kept points of the last step, up to three, are called A, B
+// and C in slot order, the new point L; every determinant of a subset
+// containing L is the slot-indexed one's arithmetic with these names (pairs
+// and triples do not depend on where L stands; the sums over four points and
+// of the result run in slot order, in which L stands after f of A, B, C).
+// One copy of this code serves every slot; of a copy for each slot a wave runs
+// all that its lanes need, one after the other (623 us per launch against 289,
+// 200,000-body hopper).
+DEM_HD bool j_closest(const GjkWork& W, unsigned& bits, unsigned all_bits, int f, const d3& w, d3& v) {
+  const bool hA = bits != 0u;
+  const unsigned r1 = bits & (bits - 1u), r2 = r1 & (r1 - 1u);
+  const bool hB = r1 != 0u, hC = r2 != 0u;
+  const int sA = hA ? __builtin_ctz(bits) : 0, sB = hB ? __builtin_ctz(r1) : 0, sC = hC ? __builtin_ctz(r2) : 0;
+  auto pos = [](double d) { return !(d <= kEps3); };
+  auto neg = [](double d) { return !(d > 0.); };
+  // the subset found: which of A, B, C (1, 2, 4) it holds beside L
+  unsigned sel = 8u;
+  auto take = [&](bool ok, unsigned m) { sel = sel == 8u && ok ? m : sel; };
+  double pA = 0., lA = 0., pB = 0., lB = 0., pC = 0., lC = 0., abA = 0., abB = 0., abL = 0., acA = 0., acC = 0.,
+         acL = 0., bcB = 0., bcC = 0., bcL = 0., qA = 0., qB = 0., qC = 0., qL = 0.;
+  const d3 zero{0., 0., 0.};
+  d3 yA = zero, yB = zero, yC = zero;
+  const double LL = dot(w, w);
+  if (hA) {
+    yA = work_y(W, sA);
+    const double AA = dot(yA, yA), LA = dot(yA, w);
+    pA = LL - LA;  // det of {A, L}: A's, L's
+    lA = AA - LA;
+    bool onlyA = pos(pA) && pos(lA), onlyL = neg(pA);
+    if (hB) {
+      yB = work_y(W, sB);
+      const double BB = dot(yB, yB), LB = dot(yB, w), AB = dot(yA, yB);
+      pB = LL - LB;
+      lB = BB - LB;
+      abA = pB * (BB - AB) + lB * (LB - LA);
+      abB = pA * (AA - AB) + lA * (LA - LB);
+      abL = (BB - AB) * (AA - LA) + (AA - AB) * (AB - LB);
+      bool onlyB = pos(pB) && pos(lB) && neg(abA), onAB = pos(abA) && pos(abB) && pos(abL);
+      onlyA = onlyA && neg(abB);
+      onlyL = onlyL && neg(pB);
+      if (hC) {
+        yC = work_y(W, sC);
+        const double CC = dot(yC, yC), LC = dot(yC, w), AC = dot(yA, yC), BC = dot(yB, yC);
+        pC = LL - LC;
+        lC = CC - LC;
+        acA = pC * (CC - AC) + lC * (LC - LA);
+        acC = pA * (AA - AC) + lA * (LA - LC);
+        acL = (CC - AC) * (AA - LA) + (AA - AC) * (AC - LC);
+        bcB = pC * (CC - BC) + lC * (LC - LB);
+        bcC = pB * (BB - BC) + lB * (LB - LC);
+        bcL = (CC - BC) * (BB - LB) + (BB - BC) * (BC - LC);
+        // four points: sums over the other three in slot order, with the
+        // first of them as the reference point
+        // (l + a and a + l are the same sum, so only "before b" matters)
+        auto sum3 = [](bool l_before_b, double l, double a, double b) {
+          return (a + (l_before_b ? l : b)) + (l_before_b ? b : l);
+        };
+        qL = (work_w(W, sA) * (AA - LA) + work_w(W, sB) * (AB - LB)) + work_w(W, sC) * (AC - LC);
+        const bool l0 = f == 0, l1 = f <= 1, l2 = f <= 2;
+        // others of A: B, C and L (first when f <= 1)
+        qA = sum3(l2, bcL * ((l1 ? LL : LB) - LA), bcB * ((l1 ? LB : BB) - AB), bcC * ((l1 ? LC : BC) - AC));
+        // others of B: A, C and L (first when f == 0)
+        qB = sum3(l2, acL * ((l0 ? LL : LA) - LB), acA * ((l0 ? LA : AA) - AB), acC * ((l0 ? LC : AC) - BC));
+        // others of C: A, B and L (first when f == 0)
+        qC = sum3(l1, abL * ((l0 ? LL : LA) - LC), abA * ((l0 ? LA : AA) - AC), abB * ((l0 ? LB : AB) - BC));
+        take(pos(qA) && pos(qB) && pos(qC) && pos(qL), 7u);
+        take(pos(bcB) && pos(bcC) && pos(bcL) && neg(qA), 6u);
+        take(pos(acA) && pos(acC) && pos(acL) && neg(qB), 5u);
+        take(pos(pC) && pos(lC) && neg(acA) && neg(bcB), 4u);
+        onAB = onAB && neg(qC);
+        onlyB = onlyB && neg(bcC);
+        onlyA = onlyA && neg(acC);
+        onlyL = onlyL && neg(pC);
       }
+      take(onAB, 3u);
+      take(onlyB, 2u);
     }
-  });
-  if (found) return true;
-  if (j_valid<last_bit>(S, all_bits)) {
-    bits = last_bit;
-    v = S.y[LAST];
-    return true;
+    take(onlyA, 1u);
+    take(onlyL, 0u);
+  } else {
+    sel = 0u;
   }
-  double min_dist2 = INFINITY;
-  sfor_down<15, 0>([&](auto SI) {
-    constexpr unsigned s = (unsigned)decltype(SI)::value;
-    if ((s & all_bits) == s && j_proper<s>(S)) {
-      d3 u = j_vector<s>(S);
-      double d2 = dot(u, u);
-      if (d2 < min_dist2) {
-        min_dist2 = d2;
-        bits = s;
-        v = u;
-      }
-    }
-  });
-  return false;
+  if (sel == 8u) {
+    j_backup(W, bits, all_bits, f, v);
+    return false;
+  }
+  const bool cA = (sel & 1u) != 0u, cB = (sel & 2u) != 0u, cC = (sel & 4u) != 0u;
+  const double kL = cC ? (cB ? (cA ? qL : bcL) : (cA ? acL : lC)) : (cB ? (cA ? abL : lB) : (cA ? lA : 1.));
+  const double kA = !cA ? 0. : (cC ? (cB ? qA : acA) : (cB ? abA : pA));
+  const double kB = !cB ? 0. : (cC ? (cA ? qB : bcB) : (cA ? abB : pB));
+  const double kC = !cC ? 0. : (cB ? (cA ? qC : bcC) : (cA ? acC : pC));
+  // computeVector (Convex.cpp:294-306): sums in slot order
+  const bool l1 = f <= 1, l2 = f == 2, l3 = f <= 2;
+  auto ordered = [&](double a, double b, double c, double l) {
+    return (((0. + a) + (l1 ? l : b)) + (l1 ? b : (l2 ? l : c))) + (l3 ? c : l);
+  };
+  if (sel == 0u) {
+    v = w;
+  } else {
+    v.x = ordered(kA * yA.x, kB * yB.x, kC * yC.x, kL * w.x);
+    v.y = ordered(kA * yA.y, kB * yB.y, kC * yC.y, kL * w.y);
+    v.z = ordered(kA * yA.z, kB * yB.z, kC * yC.z, kL * w.z);
+    v *= 1. / ordered(kA, kB, kC, kL);
+  }
+  bits = 1u << f;
+  work_w(W, f) = kL;
+  if (sel & 1u) {
+    bits |= 1u << sA;
+    work_w(W, sA) = kA;
+  }
+  if (sel & 2u) {
+    bits |= 1u << sB;
+    work_w(W, sB) = kB;
+  }
+  if (sel & 4u) {
+    bits |= 1u << sC;
+    work_w(W, sC) = kC;
+  }
+  return true;
 }
+
 // degenerate (Convex.cpp:418-435)
-DEM_HD bool j_degenerate(const Simplex& S, unsigned all_bits, d3 w) {
+DEM_HD bool j_degenerate(const GjkWork& W, unsigned all_bits, const d3& w) {
   bool deg = false;
-  sfor<0, 4>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    if ((all_bits & (1u << i)) && S.y[i].x == w.x && S.y[i].y == w.y && S.y[i].z == w.z) deg = true;
-  });
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (all_bits & (1u << i)) {
+      const d3 y = work_y(W, i);
+      if (y.x == w.x && y.y == w.y && y.z == w.z) deg = true;
+    }
   return deg;
 }
 
-// One iteration of closest_points with the new point in slot LAST: 1 to go
-// on, 0 when the loop ends.
-// sep >= 0: 2 as soon as the support point w proves the distance larger
-// than sep (the lower bound v.w / |v| of the distance exceeds it, with a
-// margin above the rounding of v.w), so that a pair that cannot be in
-// contact stops at once; the distance itself is then not computed.
+// computePoints (Convex.cpp:310-327) for the kept subset and its weights
+DEM_HD void j_points(const GjkWork& W, unsigned bits, d3& p1, d3& p2) {
+  double sum = 0.;
+  p1 = d3{0., 0., 0.};
+  p2 = d3{0., 0., 0.};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (bits & (1u << i)) {
+      const double l = work_w(W, i);
+      sum += l;
+      p1 += l * work_get(W, 12 + 3 * i);
+      p2 += l * work_get(W, 24 + 3 * i);
+    }
+  const double s = 1. / sum;
+  p1 *= s;
+  p2 *= s;
+}
+
 // Nesterov direction of closest_points (Convex.cpp:575-585; GJK_SV.cpp:479-489)
 DEM_HD d3 nesterov_dir(int it, d3 d, d3 v, d3 w) {
   const double momentum = it / (it + 2.), omm = 1. - momentum;
@@ -314,8 +381,11 @@ DEM_HD d3 nesterov_dir(int it, d3 d, d3 v, d3 w) {
 
 // The search direction, support points and optimality-gap test of one
 // iteration, with the tolerance and acceleration of o: 1 to go on with the
-// support points P, Q (local frames) and w, 0 when the loop ends, 2 when w
-// proves the distance larger than sep (sep >= 0, acceleration off).
+// support points P, Q (local frames) and w, 0 when the loop ends, 2 (sep >= 0,
+// acceleration off) as soon as the support point w proves the distance larger
+// than sep (the lower bound v.w / |v| of the distance exceeds it, with a
+// margin above the rounding of v.w), so that a pair that cannot be in
+// contact stops at once; the distance itself is then not computed.
 DEM_HD int gjk_search(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w, const GjkOpts& o,
                       int it, d3 v, double dist, double sep, d3& d, d3& w, bool& accel, d3& P, d3& Q) {
   const double relError = o.tol, absError = 1.e-4 * relError;
@@ -334,21 +404,6 @@ DEM_HD int gjk_search(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, con
     Q = support(B, tf_vec_basis(v, b2w));
     w = tf_apply(a2w, P) - tf_apply(b2w, Q);
   }
-  return 1;
-}
-
-template <int LAST>
-DEM_HD int gjk_iter(Simplex& S, const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w,
-                    unsigned& bits, unsigned& all_bits, d3& v, double& dist, double sep, int it, d3& d, d3& w,
-                    bool& accel) {
-  constexpr unsigned last_bit = 1u << LAST;
-  const int go = gjk_search(A, a2w, B, b2w, A.opt, it, v, dist, sep, d, w, accel, S.p[LAST], S.q[LAST]);
-  if (go != 1) return go;
-  if (j_degenerate(S, all_bits, w)) return 0;
-  S.y[LAST] = w;
-  all_bits = bits | last_bit;
-  if (!j_closest<LAST>(S, bits, all_bits, v)) return 0;
-  dist = norm(v);
   return 1;
 }
 
@@ -372,7 +427,7 @@ DEM_HD double& lw(L4& l) {
 }
 
 struct SvSimplex {
-  d3 y[4], p[4], q[4];
+  d3 y[4];
   L4 lam;
 };
 
@@ -576,30 +631,14 @@ DEM_HD void sv_sub(const d3 (&y)[4], unsigned& bits, L4& lam) {
 // in slot LAST (a compile-time index, as in gjk_iter): 1 when the point
 // joins the simplex (y[LAST] set, bits updated), 0 when the loop ends, 2
 // when the pair is proven farther apart than sep.
-template <int LAST>
-DEM_HD int sv_iter(SvSimplex& S, const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w,
-                   unsigned& bits, const d3& v, double dist, double sep, int it, d3& d, d3& w, bool& accel) {
-  const int go = gjk_search(A, a2w, B, b2w, A.opt, it, v, dist, sep, d, w, accel, S.p[LAST], S.q[LAST]);
-  if (go != 1) return go;
-  bool degen = false;
-  sfor<0, 4>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    if ((bits & (1u << i)) && S.y[i].x == w.x && S.y[i].y == w.y && S.y[i].z == w.z) degen = true;
-  });
-  if (degen) return 0;
-  S.y[LAST] = w;
-  bits |= 1u << LAST;
-  return 1;
-}
-
 // closest_points_GJK_SV (GJK_SV.cpp:428-525), tolerance and acceleration of
 // A.opt; witness points in the local frames; returns the distance
-DEM_HD double gjk_sv_closest(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w, d3& pa, d3& pb,
-                             int& iters, double sep, bool* separated) {
+DEM_HD double gjk_sv_closest(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w, const GjkWork& W,
+                             d3& pa, d3& pb, int& iters, double sep, bool* separated) {
   SvSimplex S;
   sfor<0, 4>([&](auto I) {
     constexpr int i = decltype(I)::value;
-    S.y[i] = S.p[i] = S.q[i] = d3{0., 0., 0.};
+    S.y[i] = d3{0., 0., 0.};
   });
   S.lam = L4{0., 0., 0., 0.};
   unsigned bits = 0;
@@ -614,17 +653,29 @@ DEM_HD double gjk_sv_closest(const ConvexGeo& A, const Tf& a2w, const ConvexGeo&
     const bool plain = !accel;
     const unsigned bits0 = bits;
     const d3 v0 = v;
-    int go;
-    if (!(bits & 1u)) go = sv_iter<0>(S, A, a2w, B, b2w, bits, v, dist, sep, it, d, w, accel);
-    else if (!(bits & 2u)) go = sv_iter<1>(S, A, a2w, B, b2w, bits, v, dist, sep, it, d, w, accel);
-    else if (!(bits & 4u)) go = sv_iter<2>(S, A, a2w, B, b2w, bits, v, dist, sep, it, d, w, accel);
-    else go = sv_iter<3>(S, A, a2w, B, b2w, bits, v, dist, sep, it, d, w, accel);
+    // the first free slot
+    const int f = __builtin_ctz(~bits);
+    d3 P, Q;
+    const int go = gjk_search(A, a2w, B, b2w, A.opt, it, v, dist, sep, d, w, accel, P, Q);
     if (go == 2) {
       if (separated) *separated = true;
       iters = it;
       return dist;
     }
     if (!go) break;
+    bool degen = false;
+    sfor<0, 4>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if ((bits & (1u << i)) && S.y[i].x == w.x && S.y[i].y == w.y && S.y[i].z == w.z) degen = true;
+    });
+    if (degen) break;
+    sfor<0, 4>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      S.y[i] = pick(f == i, w, S.y[i]);
+    });
+    work_put(W, 12 + 3 * f, P);
+    work_put(W, 24 + 3 * f, Q);
+    bits |= 1u << f;
     // one copy of the sub-distance for every slot the point went to
     sv_sub(S.y, bits, S.lam);
     v = sv_point(S.y, bits, S.lam);
@@ -644,8 +695,8 @@ DEM_HD double gjk_sv_closest(const ConvexGeo& A, const Tf& a2w, const ConvexGeo&
   sfor<0, 4>([&](auto I) {
     constexpr int i = decltype(I)::value;
     if (bits & (1u << i)) {
-      pa += lw<i>(S.lam) * S.p[i];
-      pb += lw<i>(S.lam) * S.q[i];
+      pa += lw<i>(S.lam) * work_get(W, 12 + 3 * i);
+      pb += lw<i>(S.lam) * work_get(W, 24 + 3 * i);
     }
   });
   iters = it;
@@ -829,41 +880,63 @@ DEM_HD bool bv_overlap(const ConvexGeo& A, const ConvexGeo& B) {
   return A.opt.bv == 1 ? obb_overlap(A, B) : obc_overlap(A, B);
 }
 
+// A search under way: Johnson's GJK (Convex.cpp:536-627), one iteration per
+// call, so that a wave can hand a lane whose search has ended the next pair.
+struct GjkState {
+  d3 v, w, d;  // current nearest point; last support point and direction (Nesterov)
+  double dist;
+  unsigned bits, all_bits;
+  int it;
+  bool accel;
+};
+DEM_HD void gjk_begin(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w, GjkState& g) {
+  const d3 zero{0., 0., 0.};
+  g.v = tf_apply(a2w, support(A, zero)) - tf_apply(b2w, support(B, zero));
+  g.w = g.d = g.v;
+  g.accel = A.opt.accel != 0;
+  g.dist = norm(g.v);
+  g.bits = g.all_bits = 0u;
+  g.it = 0;
+}
+// 1: go on; 0: the search has ended (g.dist, kept points in W); 2: the
+// distance is proven larger than sep (>= 0)
+DEM_HD int gjk_step(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w, const GjkWork& W, double sep,
+                    GjkState& g) {
+  if (!(g.bits < 15u && g.dist > kEps2 && g.it < 1000)) return 0;
+  ++g.it;
+  // the first free slot
+  const int f = __builtin_ctz(~g.bits);
+  d3 P, Q;
+  const int go = gjk_search(A, a2w, B, b2w, A.opt, g.it, g.v, g.dist, sep, g.d, g.w, g.accel, P, Q);
+  if (go != 1) return go;
+  if (j_degenerate(W, g.all_bits, g.w)) return 0;
+  work_put(W, 3 * f, g.w);
+  work_put(W, 12 + 3 * f, P);
+  work_put(W, 24 + 3 * f, Q);
+  g.all_bits = g.bits | (1u << f);
+  if (!j_closest(W, g.bits, g.all_bits, f, g.w, g.v)) return 0;
+  g.dist = norm(g.v);
+  return 1;
+}
+
 // closest_points with Johnson's sub-distance (Convex.cpp:536-627), the
 // tolerance and acceleration of A.opt; witness points in the local frames;
 // returns the distance (sep >= 0: *separated set when the distance is
 // proven larger than sep; the witness points are then not computed)
-DEM_HD double gjk_johnson_closest(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w, d3& pa,
-                                  d3& pb, int& iters, double sep, bool* separated) {
-  Simplex S;
-  for (int i = 0; i < 16; ++i)
-    for (int j = 0; j < 4; ++j) S.det[i][j] = 0.;
-  for (int i = 0; i < 10; ++i) S.dp[i] = 0.;
-  unsigned bits = 0, all_bits = 0;
-  d3 zero{0., 0., 0.};
-  d3 v = tf_apply(a2w, support(A, zero)) - tf_apply(b2w, support(B, zero));
-  d3 w = v, d = v;
-  bool accel = A.opt.accel != 0;
-  double dist = norm(v);
-  int it = 0;
-  while (bits < 15 && dist > kEps2 && it < 1000) {
-    ++it;
-    // the first free slot
-    int go;
-    if (!(bits & 1u)) go = gjk_iter<0>(S, A, a2w, B, b2w, bits, all_bits, v, dist, sep, it, d, w, accel);
-    else if (!(bits & 2u)) go = gjk_iter<1>(S, A, a2w, B, b2w, bits, all_bits, v, dist, sep, it, d, w, accel);
-    else if (!(bits & 4u)) go = gjk_iter<2>(S, A, a2w, B, b2w, bits, all_bits, v, dist, sep, it, d, w, accel);
-    else go = gjk_iter<3>(S, A, a2w, B, b2w, bits, all_bits, v, dist, sep, it, d, w, accel);
-    if (go == 2) {
-      if (separated) *separated = true;
-      iters = it;
-      return dist;
-    }
-    if (!go) break;
+DEM_HD double gjk_johnson_closest(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w,
+                                  const GjkWork& W, d3& pa, d3& pb, int& iters, double sep, bool* separated) {
+  GjkState g;
+  gjk_begin(A, a2w, B, b2w, g);
+  int go;
+  while ((go = gjk_step(A, a2w, B, b2w, W, sep, g)) == 1) {
   }
-  j_points(S, bits, pa, pb);
-  iters = it;
-  return dist;
+  iters = g.it;
+  if (go == 2) {
+    if (separated) *separated = true;
+    return g.dist;
+  }
+  j_points(W, g.bits, pa, pb);
+  return g.dist;
 }
 
 // The GJK distance the system's options choose: the signed-volume
@@ -871,8 +944,14 @@ DEM_HD double gjk_johnson_closest(const ConvexGeo& A, const Tf& a2w, const Conve
 // options (the ContactError recovery, RigidBodyWithCrust.cpp:545).
 DEM_HD double gjk_closest(const ConvexGeo& A, const Tf& a2w, const ConvexGeo& B, const Tf& b2w, d3& pa, d3& pb,
                           int& iters, double sep = -1., bool* separated = nullptr, bool johnson = false) {
-  if (A.opt.sv && !johnson) return gjk_sv_closest(A, a2w, B, b2w, pa, pb, iters, sep, separated);
-  return gjk_johnson_closest(A, a2w, B, b2w, pa, pb, iters, sep, separated);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const GjkWork W = A.work;
+#else
+  double area[kGjkWork];
+  const GjkWork W{area, 1};
+#endif
+  if (A.opt.sv && !johnson) return gjk_sv_closest(A, a2w, B, b2w, W, pa, pb, iters, sep, separated);
+  return gjk_johnson_closest(A, a2w, B, b2w, W, pa, pb, iters, sep, separated);
 }
 
 // General ClosestPoint path.  Returns 1 with the contact features (the
@@ -930,24 +1009,16 @@ DEM_HD bool recover_gjk(const ConvexGeo& A, const ConvexGeo& B, d3& P, d3& ov, d
   return true;
 }
 
-// One attempt of the general ClosestPoint path: attempt 0 with the
-// crust-shrunk transforms (closest_gjk), attempt 1 with the bodies shrunk by
-// ten crusts (recover_gjk, the ContactError recovery).  Returns 1 with the
-// contact features (d may be >= 0), 2 with the recovered features, 0 when
-// the circumscribed spheres do not meet (attempt 0), -1 when the shrunk
-// bodies intersect (attempt 0: go on with attempt 1; attempt 1:
-// ContactError).  A caller that evaluates every pair through one call of
-// this function holds a single copy of the GJK state in registers.
-// early: attempt 0 stops as soon as the pair is proven farther apart than
-// the crusts (no contact; the iteration count is then not the full run's,
-// so a caller collecting statistics passes false).
-DEM_HD int gjk_attempt(const ConvexGeo& A, const ConvexGeo& B, int attempt, d3& P, d3& ov, double& d,
-                       int& iters, bool early = false) {
+// The transforms of one attempt of the general ClosestPoint path: attempt 0
+// crust-shrunk (closest_gjk), attempt 1 with the bodies shrunk by ten crusts
+// (recover_gjk, the ContactError recovery).  False when the circumscribed
+// spheres (or the bounding volumes) do not meet.
+DEM_HD bool gjk_frames(const ConvexGeo& A, const ConvexGeo& B, int attempt, Tf& a2w, Tf& b2w) {
   d3 sa = A.scaling, sb = B.scaling;
   if (attempt == 0) {
     d3 gcagcb = A.o - B.o;
-    if (!(norm(gcagcb) < A.circR + B.circR)) return 0;
-    if (A.opt.bv && !bv_overlap(A, B)) return 0;
+    if (!(norm(gcagcb) < A.circR + B.circR)) return false;
+    if (A.opt.bv && !bv_overlap(A, B)) return false;
   } else {
     double* as[3] = {&sa.x, &sa.y, &sa.z};
     double* bs[3] = {&sb.x, &sb.y, &sb.z};
@@ -959,19 +1030,22 @@ DEM_HD int gjk_attempt(const ConvexGeo& A, const ConvexGeo& B, int attempt, d3& 
       *bs[a] = y > 0.5 ? y : 0.5;
     }
   }
-  const double crusts = A.crust + B.crust;
-  Tf a2w = tf_scaled(A, sa), b2w = tf_scaled(B, sb);
-  d3 pa, pb;
-  bool separated = false;
-  double distance =
-      gjk_closest(A, a2w, B, b2w, pa, pb, iters, early && attempt == 0 ? crusts : -1., &separated, attempt != 0);
-  if (separated) return 0;
+  a2w = tf_scaled(A, sa);
+  b2w = tf_scaled(B, sb);
+  return true;
+}
+
+// The contact features of an attempt from its search's distance and witness
+// points (local frames): 1 with the features (d may be >= 0), 2 with the
+// recovered features, -1 when the shrunk bodies intersect.
+DEM_HD int gjk_features(const Tf& a2w, const Tf& b2w, int attempt, double crusts, double distance, d3 pa, d3 pb, d3& P,
+                        d3& ov, double& d) {
   if (distance < kEps) return -1;
   pa = tf_apply(a2w, pa);
   pb = tf_apply(b2w, pb);
   d3 ba = pa - pb;
+  P = pa / 2.0 + pb / 2.0;
   if (attempt == 0) {
-    P = pa / 2.0 + pb / 2.0;
     d3 o = ba / distance;
     round_small(o);
     o *= crusts - distance;
@@ -980,11 +1054,29 @@ DEM_HD int gjk_attempt(const ConvexGeo& A, const ConvexGeo& B, int attempt, d3& 
     return 1;
   }
   ba /= norm(ba);
-  P = pa / 2.0 + pb / 2.0;
   double imposed = 1. * crusts;
   ov = imposed * ba;
   d = -imposed;
   return 2;
+}
+
+// One attempt of the general ClosestPoint path (gjk_frames, the search,
+// gjk_features); 0 when the pair is no contact (attempt 0); -1 on attempt 0:
+// go on with attempt 1; on attempt 1: ContactError.
+// early: attempt 0 stops as soon as the pair is proven farther apart than
+// the crusts (no contact; the iteration count is then not the full run's,
+// so a caller collecting statistics passes false).
+DEM_HD int gjk_attempt(const ConvexGeo& A, const ConvexGeo& B, int attempt, d3& P, d3& ov, double& d,
+                       int& iters, bool early = false) {
+  Tf a2w, b2w;
+  if (!gjk_frames(A, B, attempt, a2w, b2w)) return 0;
+  const double crusts = A.crust + B.crust;
+  d3 pa, pb;
+  bool separated = false;
+  double distance =
+      gjk_closest(A, a2w, B, b2w, pa, pb, iters, early && attempt == 0 ? crusts : -1., &separated, attempt != 0);
+  if (separated) return 0;
+  return gjk_features(a2w, b2w, attempt, crusts, distance, pa, pb, P, ov, d);
 }
 
 // --- kinematics of non-spherical bodies --------------------------------------

@@ -734,8 +734,14 @@ __device__ __forceinline__ void record_pair(const StepParams& sp, DevStatus* st,
   }
 }
 
+// Shape classes and vertex table: P's, or copies of them in LDS.
+struct ShapeTables {
+  const ShapeDesc* shapes;
+  const double* verts;
+};
+
 // Body of particle s (storage index) at position x, basis buffer cx.
-__device__ __forceinline__ ConvexGeo convex_of(const Particles& P, int s, d3 x, int cx) {
+__device__ __forceinline__ ConvexGeo convex_of(const Particles& P, int s, d3 x, int cx, const ShapeTables& tab) {
   ConvexGeo g;
   const int sh = P.shape[s];
   for (int j = 0; j < 9; ++j) g.B[j] = P.B[cx][j][s];
@@ -754,10 +760,10 @@ __device__ __forceinline__ ConvexGeo convex_of(const Particles& P, int s, d3 x, 
     g.circR = r;
     g.obb = d3{r, r, r};
   } else {
-    const ShapeDesc& d = P.shapes[sh];
+    const ShapeDesc& d = tab.shapes[sh];
     g.type = d.type;
     g.nv = d.nv;
-    g.verts = P.verts + 3 * (size_t)d.vert_off;
+    g.verts = tab.verts + 3 * d.vert_off;
     g.r = d.radius;
     g.e = d3{d.extent[0], d.extent[1], d.extent[2]};
     g.scaling = d3{d.scaling[0], d.scaling[1], d.scaling[2]};
@@ -794,6 +800,17 @@ __device__ __forceinline__ ConvexGeo convex_of_obstacle(const BoxObstacle& B) {
 // axis a for image code -1, 0, +1.
 __device__ __forceinline__ double image_shift(const Grid& G, int a, int c) {
   return c < 0 ? -G.L[a] : (c > 0 ? G.L[a] : 0.);
+}
+
+// Particle s at the periodic image of image code c (see nbr_entry), seen
+// there by its neighbour: x + vec, added only on the wrapped axes.
+__device__ __forceinline__ d3 image_of(const Particles& P, const Grid& G, int s, int cx, int c) {
+  const int ix = c % 3 - 1, iy = (c / 3) % 3 - 1, iz = c / 9 - 1;
+  d3 x{P.x[cx][0][s], P.x[cx][1][s], P.x[cx][2][s]};
+  if (ix) x.x = x.x + image_shift(G, 0, ix);
+  if (iy) x.y = x.y + image_shift(G, 1, iy);
+  if (iz) x.z = x.z + image_shift(G, 2, iz);
+  return x;
 }
 
 // Enumerates the neighbour candidates of a particle at x as runs of sorted
@@ -895,7 +912,7 @@ __device__ __forceinline__ void narrow_visit(const Particles& P, const Grid& G, 
   int nit = 1;
   if (SHAPES && (mg->type != kShapeSphere ||
                  (P.shape[s2i] >= 0 && P.shapes[P.shape[s2i]].type != kShapeSphere))) {
-    ConvexGeo og = convex_of(P, s2i, xo, cx);
+    ConvexGeo og = convex_of(P, s2i, xo, cx, ShapeTables{P.shapes, P.verts});
     int res = closest_convex(*mg, og, Pc, ov, d, &nit);
     if (res == 0) return;
     if (res < 0) {
@@ -1058,6 +1075,15 @@ __device__ __forceinline__ unsigned nbr_entry(int k2, int ix, int iy, int iz) {
   return (unsigned)k2 | ((unsigned)((ix + 1) + 3 * (iy + 1) + 9 * (iz + 1)) << kNbrSlotBits);
 }
 constexpr int kNbrNoShift = 13;  // the image code of a neighbour without periodic shift
+
+__device__ __forceinline__ int body_type(const Particles& P, int s) {
+  return P.shape[s] < 0 ? kShapeSphere : P.shapes[P.shape[s]].type;
+}
+// A pair without periodic shift whose evaluation is exactly symmetric under
+// the exchange of the bodies (every path but the sphere-sphere closed form,
+// which places the point from body A's centre) is evaluated once, by its
+// lower id.
+__device__ __forceinline__ bool one_sided(int code, bool both_spheres) { return code == kNbrNoShift && !both_spheres; }
 
 // The same contacts as for_each_contact, from the candidate list written by
 // k_detect for this step (same candidates, same order).  A particle whose

@@ -7,7 +7,7 @@
 //   k_scatter            storage index to (cell, arrival slot)
 //   k_canon              per cell: order by particle id, gather (x,y,z,r) into
 //                        the sorted tile array, reset the counts
-//   k_detect             one thread per sorted particle: 27-cell sweep with
+//   k_detect             a few lanes per sorted particle: 27-cell sweep with
 //                        minimum-image shifts, neighbour candidates -> list
 //   k_forces<MODE>       one thread per particle (storage order; sorted order
 //                        with non-spherical bodies): the listed (or, with no
@@ -216,41 +216,120 @@ __global__ __launch_bounds__(256) void k_canon(Particles P, Sorted S, int ncells
 // Broad phase of one step (LinkedCell::ComputeForces, LinkedCell.cpp:1019-1103):
 // every neighbour candidate of each sorted particle that passes the
 // conservative distance reject of the narrow phase, in the order the force
-// sweep visits them, written to the candidate list.  Holding only the
-// particle's position and the nine row ranges, the kernel keeps few
-// registers live, so many waves per SIMD overlap its dependent loads; the
-// force sweep then reads a short list instead of 27 cells.
-// mark (systems with non-spherical bodies): each listed slot's contact
-// record starts as kNoFeat, so that the narrow phase writes only contacts.
+// sweep visits them, written to the candidate list; the force sweep then reads
+// a short list instead of 27 cells.  kDetectLanes lanes share a particle and
+// test that many consecutive candidates at once (the accepted ones numbered by
+// a ballot): one lane alone waits for its candidates' loads one after the
+// other (46.8 us per launch for 343 polyhedra, whose 27 cells hold about 96
+// bodies each; 21.6 us with eight, work list included, and 101 us instead of
+// 123 for 200,000 -- a launch of its own wrote the work list in 59 us).
+// ITEMS (systems with non-spherical bodies): each listed slot's contact
+// record starts as kNoFeat, so that the narrow phase writes only contacts, and
+// the evaluations the narrow phase has to make are appended to its work list:
+// one for each candidate unless the partner's side makes it (a pair without
+// periodic shift is evaluated once, by its lower id, see mirrored_pair) and
+// one for each obstacle whose bounding box the particle meets.
 // After an error raised on the device (which ends the run) the contact
 // searches return at once, so that the rest of a batch of steps costs
 // little whatever the state has become.
-__global__ __launch_bounds__(256) void k_detect(Sorted S, Grid G, int n, NbrList L, int* __restrict__ mark,
-                                                const DevStatus* st) {
-  const int k = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (k >= n || st->code) return;
-  const double* pr = S.posr + 4 * (size_t)k;
-  const d3 x{pr[0], pr[1], pr[2]};
-  const double r = pr[3];
-  int c = 0;
-  // one candidate at a time: at this register count eight waves per SIMD
-  // overlap the loads better than wider batches of loads per thread do
-  for_each_candidate(S, G, 0, 0, n, x, [&](int k2, int ix, int iy, int iz) {
-    if (k2 == k) return;
-    const double* q2 = S.posr + 4 * (size_t)k2;
-    d3 xo{ix ? q2[0] + image_shift(G, 0, ix) : q2[0], iy ? q2[1] + image_shift(G, 1, iy) : q2[1],
-          iz ? q2[2] + image_shift(G, 2, iz) : q2[2]};
-    d3 AB = xo - x;
-    double s2 = AB.x * AB.x + AB.y * AB.y + AB.z * AB.z;
-    double R = r + q2[3];
-    if (s2 > R * R * 1.000000000001) return;
-    if (c < L.cap) {
-      L.ent[(size_t)c * n + k] = nbr_entry(k2, ix, iy, iz);
-      if (mark) mark[(size_t)c * n + k] = kNoFeat;
+constexpr int kDetectLanes = 8;
+constexpr int kItemBuf = 1024;  // items a workgroup collects before it appends them
+
+template <bool ITEMS>
+__global__ __launch_bounds__(kDetectLanes * kDetectBodies) void k_detect(Particles P, Sorted S, Grid G,
+                                                                         const BoxObstacle* __restrict__ obs,
+                                                                         StepParams sp, NbrList L,
+                                                                         const DevStatus* st) {
+  __shared__ NarrowItem buf[ITEMS ? kItemBuf : 1];
+  __shared__ int nbuf, base;
+  if (st->code) return;
+  const int n = sp.n;
+  const int lane = threadIdx.x & (kDetectLanes - 1);
+  const int gshift = threadIdx.x & 63 & ~(kDetectLanes - 1);
+  const int k = xcd_tile(blockIdx.x, gridDim.x) * kDetectBodies + threadIdx.x / kDetectLanes;
+  if (ITEMS) {
+    if (threadIdx.x == 0) nbuf = 0;
+    __syncthreads();
+  }
+  const int list = blockIdx.x & (kItemLists - 1);
+  NarrowItem* const items = ITEMS ? sp.cf.items + (size_t)list * sp.cf.item_stride : nullptr;
+  int* const nitems = ITEMS ? sp.cf.nitems + list * kItemPad : nullptr;
+  if (k < n) {
+    const double* pr = S.posr + 4 * (size_t)k;
+    const d3 x{pr[0], pr[1], pr[2]};
+    const double r = pr[3];
+    const int s = ITEMS ? S.order[k] : 0;
+    const bool body = !ITEMS || (unsigned)s < (unsigned)n;
+    const int id = ITEMS && body ? P.id[s] : 0;
+    const bool sphere = ITEMS && P.spheres && body && body_type(P, s) == kShapeSphere;
+    auto append = [&](unsigned jc, int partner) {
+      const NarrowItem it{k, jc, s, partner};
+      const int i = atomicAdd(&nbuf, 1);
+      if (i < kItemBuf) buf[i] = it;
+      else items[atomicAdd(nitems, 1)] = it;
+    };
+    int c = 0;
+    for_each_run(S, G, 0, 0, n, x, [&](int b, int e, int ix, int iy, int iz) {
+      for (int k0 = b; k0 < e; k0 += kDetectLanes) {
+        const int k2 = k0 + lane;
+        bool hit = k2 < e && k2 != k;
+        if (hit) {
+          const double* q2 = S.posr + 4 * (size_t)k2;
+          const d3 xo{ix ? q2[0] + image_shift(G, 0, ix) : q2[0], iy ? q2[1] + image_shift(G, 1, iy) : q2[1],
+                      iz ? q2[2] + image_shift(G, 2, iz) : q2[2]};
+          const d3 AB = xo - x;
+          const double s2 = AB.x * AB.x + AB.y * AB.y + AB.z * AB.z;
+          const double R = r + q2[3];
+          hit = !(s2 > R * R * 1.000000000001);
+        }
+        const unsigned hits = (unsigned)(__ballot(hit) >> gshift) & ((1u << kDetectLanes) - 1u);
+        const int j = c + __popc(hits & ((1u << lane) - 1u));
+        if (hit && j < L.cap) {
+          const unsigned e2 = nbr_entry(k2, ix, iy, iz);
+          L.ent[(size_t)j * n + k] = e2;
+          if (ITEMS) {
+            sp.cf.ent[(size_t)j * n + k] = kNoFeat;
+            const int o = S.order[k2];
+            if (body && (unsigned)o < (unsigned)n) {
+              const bool both = sphere && body_type(P, o) == kShapeSphere;
+              const int code = (int)(e2 >> kNbrSlotBits);
+              if (!(one_sided(code, both) && id > S.sid[k2])) append((unsigned)j | (e2 & ~kNbrSlotMask), o);
+            }
+          }
+        }
+        c += __popc(hits);
+      }
+    });
+    if (lane == 0) L.count[k] = c;
+    if (ITEMS) {
+      int last = -1;
+      if (body && c <= L.cap)
+        for (int o0 = 0; o0 < sp.nobs; o0 += kDetectLanes) {
+          const int o = o0 + lane;
+          bool met = false;
+          if (o < sp.nobs) {
+            const BoxObstacle& B = obs[o];
+            met = fabs(B.aabb_c[0] - x.x) <= B.aabb_e[0] + r && fabs(B.aabb_c[1] - x.y) <= B.aabb_e[1] + r &&
+                  fabs(B.aabb_c[2] - x.z) <= B.aabb_e[2] + r;
+          }
+          const unsigned hits = (unsigned)(__ballot(met) >> gshift) & ((1u << kDetectLanes) - 1u);
+          if (met && c + o < sp.cf.cap) append((unsigned)(c + o) | ((unsigned)kNbrNoShift << kNbrSlotBits), -1 - o);
+          if (hits) last = o0 + 31 - __builtin_clz(hits);
+        }
+      // every obstacle slot the force sweep will read, met or not, starts empty
+      for (int o = lane; o <= last; o += kDetectLanes)
+        if (c + o < sp.cf.cap) sp.cf.ent[(size_t)(c + o) * n + k] = kNoFeat;
+      // a body without a usable list: -1, k_narrow_full searches its cells
+      if (lane == 0) sp.cf.count[k] = !body ? 0 : (c > L.cap ? -1 : c + last + 1);
     }
-    ++c;
-  });
-  L.count[k] = c;
+  }
+  if (ITEMS) {
+    __syncthreads();
+    const int m = min(nbuf, kItemBuf);
+    if (threadIdx.x == 0) base = m ? atomicAdd(nitems, m) : 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < m; i += kDetectLanes * kDetectBodies) items[base + i] = buf[i];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -473,10 +552,12 @@ hipError_t launch_vfilter(const Particles& P, const Sorted& S, const Grid& G, co
   return hipGetLastError();
 }
 
-hipError_t launch_detect(const Sorted& S, const Grid& G, int n, const NbrList& L, const DevStatus* st,
-                         hipStream_t stream, int* mark) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_detect, dim3(nblk(n, 256)), dim3(256), 0, stream, S, G, n, L, mark, st);
+hipError_t launch_detect(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
+                         const StepParams& sp, const NbrList& L, const DevStatus* st, hipStream_t stream) {
+  if (sp.n == 0) return hipSuccess;
+  const dim3 grid(nblk(sp.n, kDetectBodies)), block(kDetectLanes * kDetectBodies);
+  if (P.shape) hipLaunchKernelGGL(k_detect<true>, grid, block, 0, stream, P, S, G, obs, sp, L, st);
+  else hipLaunchKernelGGL(k_detect<false>, grid, block, 0, stream, P, S, G, obs, sp, L, st);
   return hipGetLastError();
 }
 

@@ -8,16 +8,17 @@
 // records, so that the GJK state and the integrator never share a kernel's
 // registers.  Contact statistics of the evaluation are collected here.
 //
-//   k_items        one thread per sorted particle: the work list of the
-//                  step -- one item per listed candidate the particle
-//                  evaluates and per obstacle whose bounding box it meets
-//                  -- appended with one atomic per wave; the obstacle
-//                  record slots it may fill are marked kNoFeat
-//   k_narrow_items a grid of one-wave workgroups over the work list, one
-//                  evaluation per lane, so that the GJK work of a dense bed
-//                  occupies as many lanes as it has pairs instead of one
-//                  lane per body; a contact's record goes to the item's
-//                  slot (candidate j: slot j; obstacle o: slot nc + o)
+// The work list of the step -- one item per listed candidate a particle
+// evaluates and per obstacle whose bounding box it meets -- is written by the
+// contact search (k_detect).
+//
+//   k_narrow_lanes the work list with the default options: a grid of one-wave
+//                  workgroups, each lane stepping one distance search and
+//                  taking another item when it ends; a contact's record goes
+//                  to the item's slot (candidate j: slot j; obstacle o: slot
+//                  nc + o)
+//   k_narrow_items the work list with other options, and the closed forms
+//                  (spheres), one evaluation per lane
 //   k_narrow       with contact statistics: one thread per particle over
 //                  all its candidates and obstacles, records packed;
 //                  through ONE evaluation site (one copy of the GJK state
@@ -29,17 +30,28 @@
 // both layouts give the same contacts in the same order.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dem_device.hpp"
 #include "dem_forces.hpp"
 #include "dem_launch.hpp"
 
 namespace dem {
 
-// Records each contact (overlap < 0) of one particle.
+// Records each contact (overlap < 0) of one particle.  mirror (k_narrow_full
+// beside the work list): the partners with a usable list and a higher id
+// make no evaluation of their own of a one-sided pair.
 struct FeatureVisitor {
   const ContactFeat& cf;
   int k;
   int c = 0;
+  bool mirror = false;
+  const Particles* P = nullptr;
+  const Sorted* S = nullptr;
+  const NbrList* L = nullptr;
+  const Self* me = nullptr;
+  int s = 0;
+  DevStatus* st = nullptr;
   __device__ __forceinline__ void put(int o, int pid, d3 xo, d3 Pc, d3 ov) {
     put_at(c, o, pid, xo, Pc, ov);
     ++c;
@@ -60,9 +72,11 @@ struct FeatureVisitor {
       cf.f[8][e] = ov.z;
     }
   }
-  __device__ __forceinline__ void pair(int, int s2i, int pid2, d3 xo, double, d3 Pc, d3 ov, double) {
+  __device__ __forceinline__ void pair(int k2, int s2i, int pid2, d3 xo, double, d3 Pc, d3 ov, double d) {
     put(s2i, pid2, xo, Pc, ov);
+    if (mirror && pid2 > me->id && L->count[k2] <= L->cap) mirror_full(k2, s2i, pid2, xo, Pc, ov, d);
   }
+  __device__ __forceinline__ void mirror_full(int k2, int s2i, int pid2, d3 xo, d3 Pc, d3 ov, double d);
   __device__ __forceinline__ void wall(int o, d3 Pc, d3 ov, double) { put(-1 - o, 0, d3{0., 0., 0.}, Pc, ov); }
 };
 
@@ -81,15 +95,62 @@ __device__ __forceinline__ bool load_self(const Particles& P, const Sorted& S, c
   return true;
 }
 
-// A pair without periodic shift whose evaluation is exactly symmetric under
-// the exchange of the bodies (every path but the sphere-sphere closed form,
-// which places the point from body A's centre) is evaluated once, by its
-// lower id, which also writes the partner's record -- the mirror image:
-// same point, opposite overlap vector -- unless the partner has no usable
-// list (k_narrow_full then covers it).  The partner's record slot holds
-// kNoFeat from k_detect until then.
+// A one-sided pair (see one_sided) is evaluated by its lower id, which also
+// writes the partner's record -- the mirror image: same point, opposite
+// overlap vector -- unless the partner has no usable list (k_narrow_full then
+// covers it).  The partner's record slot holds kNoFeat from k_detect until
+// then.
 __device__ __forceinline__ bool mirrored_pair(const NbrList& L, int code, bool both_spheres, int k2) {
-  return code == kNbrNoShift && !both_spheres && L.count[k2] <= L.cap;
+  return one_sided(code, both_spheres) && L.count[k2] <= L.cap;
+}
+
+// The slot of body k in its neighbour k2's list (both seen without periodic
+// shift; the lists are symmetric: the candidate test is exact under the
+// exchange), -1 if it is missing.
+__device__ __forceinline__ int slot_in_list(const NbrList& L, int k2, int k) {
+  const int nc2 = L.count[k2];
+  const unsigned want = nbr_entry(k, 0, 0, 0);
+  for (int i0 = 0; i0 < nc2; i0 += 16) {
+    unsigned hit = 0u;
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (i0 + u < nc2 && L.ent[(size_t)(i0 + u) * L.n + k2] == want) hit |= 1u << u;
+    if (hit) return i0 + __builtin_ctz(hit);
+  }
+  return -1;
+}
+
+// The record of item j of sorted slot k, and, for a mirrored pair, the
+// partner's.
+__device__ __forceinline__ void put_item(const StepParams& sp, DevStatus* st, const NbrList& L, int k, int j, int s,
+                                         const Self& me, int partner, int pid2, int k2, bool mirror, d3 xo, d3 Pc,
+                                         d3 ov) {
+  FeatureVisitor vis{sp.cf, k};
+  vis.put_at(j, partner, pid2, xo, Pc, ov);
+  if (!mirror) return;
+  const int jm = slot_in_list(L, k2, k);
+  if (jm < 0) {
+    raise_error(st, kContactOverflow, me.id, pid2);
+  } else {
+    FeatureVisitor pv{sp.cf, k2};
+    pv.put_at(jm, s, me.id, me.x, Pc, -ov);
+  }
+}
+
+__device__ __forceinline__ void FeatureVisitor::mirror_full(int k2, int s2i, int pid2, d3 xo, d3 Pc, d3 ov, double d) {
+  const double* q2 = S->posr + 4 * (size_t)k2;
+  const bool shifted = xo.x != q2[0] || xo.y != q2[1] || xo.z != q2[2];
+  const bool both = body_type(*P, s) == kShapeSphere && body_type(*P, s2i) == kShapeSphere;
+  if (shifted || both) return;
+  const int jm = slot_in_list(*L, k2, k);
+  if (jm < 0) {
+    raise_error(st, kContactOverflow, me->id, pid2);
+    return;
+  }
+  // a recovered contact (overlap exactly the crusts) counts on both sides
+  if (d == -(me->c + P->crust[s2i])) atomicAdd(&st->n_recovered, 1);
+  FeatureVisitor pv{cf, k2};
+  pv.put_at(jm, s, me->id, me->x, Pc, -ov);
 }
 
 // ITEM: the one evaluation `item` of sorted slot k (a listed candidate if
@@ -101,10 +162,13 @@ __device__ __forceinline__ bool mirrored_pair(const NbrList& L, int code, bool b
 // crust-shrunk bodies intersect comes round once more for the recovery
 // (attempt 1).  A particle without a usable list is marked (count -1) for
 // k_narrow_full.
+// work: the lane's column of the distance search's work area; tab: the shape
+// tables.
 template <bool ITEM>
 __device__ __forceinline__ void narrow_one(const Particles& P, const Sorted& S, const Grid& G,
                                            const BoxObstacle* __restrict__ obs, const StepParams& sp, DevStatus* st,
-                                           const NbrList& L, int k, int item, StatAcc* acc) {
+                                           const NbrList& L, int k, int item, StatAcc* acc, const GjkWork& work,
+                                           const ShapeTables& tab) {
   const int cx = sp.cur & 1;
   Self me;
   int s;
@@ -154,7 +218,6 @@ __device__ __forceinline__ void narrow_one(const Particles& P, const Sorted& S, 
       mult = me.id < pid2 ? image_evaluations(G, me.x, d3{q2[0], q2[1], q2[2]}, sh) : 0;
       const bool osph = P.shape[s2i] < 0 || P.shapes[P.shape[s2i]].type == kShapeSphere;
       if (ITEM && mirrored_pair(L, code, self_type == kShapeSphere && osph, k2)) {
-        if (me.id > pid2) continue;  // the partner's item (k_items lists none here)
         mirror = true;
       }
       if (self_type == kShapeSphere && osph) {
@@ -162,7 +225,7 @@ __device__ __forceinline__ void narrow_one(const Particles& P, const Sorted& S, 
         res = sphere_sphere(me.x, me.r, me.c, AB, sqrt(s2), ro, co, Pc, ov, d);
         if (res < 0) res = recover_ss(me.x, me.r, me.c, xo, ro, co, Pc, ov, d) ? 2 : -1;
       } else {
-        og = convex_of(P, s2i, xo, cx);
+        og = convex_of(P, s2i, xo, cx, tab);
         convex = true;
       }
     } else {
@@ -185,7 +248,8 @@ __device__ __forceinline__ void narrow_one(const Particles& P, const Sorted& S, 
       }
     }
     if (convex) {
-      const ConvexGeo mg = convex_of(P, s, me.x, cx);
+      ConvexGeo mg = convex_of(P, s, me.x, cx, tab);
+      mg.work = work;
       // closest_convex: sphere-box closed forms (a closed form that finds
       // the crusts overlapping recovers through GJK), otherwise GJK
       const bool sb = mg.type == kShapeSphere && og.type == kShapeBox;
@@ -213,27 +277,7 @@ __device__ __forceinline__ void narrow_one(const Particles& P, const Sorted& S, 
     if (acc && mult) acc->add(d, nit, mult);
     if (!(d < 0.)) continue;
     if (ITEM) {
-      vis.put_at(j, partner, pid2, xo, Pc, ov);
-      if (mirror) {
-        // this particle's slot in the partner's list (the lists are
-        // symmetric: the candidate test is exact under the exchange)
-        const int nc2 = L.count[k2];
-        const unsigned want = nbr_entry(k, 0, 0, 0);
-        int jm = -1;
-        for (int i0 = 0; i0 < nc2 && jm < 0; i0 += 16) {
-          unsigned hit = 0u;
-#pragma unroll
-          for (int u = 0; u < 16; ++u)
-            if (i0 + u < nc2 && L.ent[(size_t)(i0 + u) * L.n + k2] == want) hit |= 1u << u;
-          if (hit) jm = i0 + __builtin_ctz(hit);
-        }
-        if (jm < 0) {
-          raise_error(st, kContactOverflow, me.id, pid2);
-        } else {
-          FeatureVisitor pv{sp.cf, k2};
-          pv.put_at(jm, s, me.id, me.x, Pc, -ov);
-        }
-      }
+      put_item(sp, st, L, k, j, s, me, partner, pid2, k2, mirror, xo, Pc, ov);
     } else {
       vis.put(partner, pid2, xo, Pc, ov);
     }
@@ -243,132 +287,212 @@ __device__ __forceinline__ void narrow_one(const Particles& P, const Sorted& S, 
   if (vis.c > sp.cf.cap) raise_error(st, kContactOverflow, me.id, vis.c);
 }
 
-// The work list of sorted slot k (see k_items); returns its number of items
-// and, with out != nullptr, writes them from out[0].  With keep != nullptr
-// (out == nullptr) it also returns which candidates (keep[0], bit j) and
-// obstacles (keep[1], bit o) give items and the last obstacle met (keep[2];
-// -2: no body in the slot), for write_items.
-__device__ __forceinline__ int body_items(const Particles& P, const Sorted& S, const BoxObstacle* __restrict__ obs,
-                                          const StepParams& sp, const NbrList& L, int k,
-                                          unsigned long long* __restrict__ out, long long* keep = nullptr) {
-  const int s = S.order[k];
-  if ((unsigned)s >= (unsigned)sp.n) {
-    if (out) sp.cf.count[k] = 0;
-    if (keep) keep[2] = -2;
-    return 0;
-  }
-  const int nc = L.count[k];
-  if (nc > L.cap) return 0;  // k_narrow_full
-  const double* pr = S.posr + 4 * (size_t)k;
-  const double x[3] = {pr[0], pr[1], pr[2]}, r = pr[3];
-  const int id = P.id[s];
-  const bool ssph = P.shape[s] < 0 || P.shapes[P.shape[s]].type == kShapeSphere;
-  const unsigned long long key = (unsigned long long)(unsigned)k << 32;
-  int c = 0;
-  for (int j = 0; j < nc; ++j) {
-    const unsigned e = L.ent[(size_t)j * L.n + k];
-    const int k2 = (int)(e & kNbrSlotMask), code = (int)(e >> kNbrSlotBits);
-    if (code == kNbrNoShift) {
-      const int s2i = S.order[k2];
-      if ((unsigned)s2i < (unsigned)sp.n) {
-        const bool osph = P.shape[s2i] < 0 || P.shapes[P.shape[s2i]].type == kShapeSphere;
-        if (mirrored_pair(L, code, ssph && osph, k2) && id > S.sid[k2]) continue;
-      }
-    }
-    if (out) out[c] = key | (unsigned)j;
-    if (keep && j < 64) keep[0] |= 1ll << j;
-    ++c;
-  }
-  int last = -1;
-  for (int o = 0; o < sp.nobs; ++o) {
-    const BoxObstacle& B = obs[o];
-    if (fabs(B.aabb_c[0] - x[0]) <= B.aabb_e[0] + r && fabs(B.aabb_c[1] - x[1]) <= B.aabb_e[1] + r &&
-        fabs(B.aabb_c[2] - x[2]) <= B.aabb_e[2] + r) {
-      if (out) out[c] = key | (unsigned)(nc + o);
-      if (keep && o < 64) keep[1] |= 1ll << o;
-      ++c;
-      last = o;
-    }
-  }
-  if (keep) keep[2] = last;
-  if (out) {
-    // every obstacle slot the force sweep will read, met or not, starts empty
-    for (int o = 0; o <= last; ++o) sp.cf.ent[(size_t)(nc + o) * sp.cf.n + k] = kNoFeat;
-    sp.cf.count[k] = nc + last + 1;
-  }
-  return c;
+// Shape classes and polyhedron vertices that a workgroup copies to LDS, so
+// that a body's class costs no dependent global load and a support none at
+// all; a system with more reads them from memory.
+constexpr int kStageShapes = 8;
+constexpr int kStageVerts = 64;
+struct Staged {
+  double verts[3 * kStageVerts];
+  ShapeDesc shapes[kStageShapes];
+};
+struct StagedNone {};
+template <bool STAGED>
+__device__ __forceinline__ ShapeTables stage_tables(const Particles& P, void* lds) {
+  if (!STAGED) return ShapeTables{P.shapes, P.verts};
+  Staged* t = (Staged*)lds;
+  for (int i = threadIdx.x; i < 3 * P.nverts; i += 64) t->verts[i] = P.verts[i];
+  const int words = P.nshapes * (int)(sizeof(ShapeDesc) / 4);
+  for (int i = threadIdx.x; i < words; i += 64) ((int*)t->shapes)[i] = ((const int*)P.shapes)[i];
+  __syncthreads();
+  return ShapeTables{t->shapes, t->verts};
 }
 
-// The items body_items found for slot k, written from the masks it kept
-// (no second pass over the candidate list), in the same order.
-__device__ __forceinline__ void write_items(const StepParams& sp, int k, int nc, const long long* keep,
-                                            unsigned long long* __restrict__ out) {
-  if (keep[2] == -2) {
-    sp.cf.count[k] = 0;
+// RigidBodyWithCrust::ClosestPoint's closed forms: a sphere with a sphere or
+// a box
+__device__ __forceinline__ bool closed_pair(int a, int b) {
+  return (a == kShapeSphere && b != kShapePoly) || (a == kShapeBox && b == kShapeSphere);
+}
+__device__ __forceinline__ bool closed_item(const Particles& P, const NarrowItem& it) {
+  return closed_pair(body_type(P, it.s), it.partner < 0 ? (int)kShapeBox : body_type(P, it.partner));
+}
+
+// The work list one item per lane at a time (one-wave workgroups that stride
+// over a part of it each): every item with the signed-volume sub-distance,
+// acceleration or a bounding-volume pre-test; with the default options the
+// pairs of closed form only (closed), k_narrow_lanes taking the others.
+template <bool STAGED>
+__global__ __launch_bounds__(64) void k_narrow_items(Particles P, Sorted S, Grid G, const BoxObstacle* __restrict__ obs,
+                                                     StepParams sp, DevStatus* st, NbrList L, bool closed) {
+  __shared__ double area[kGjkWork * 64];
+  __shared__ std::conditional_t<STAGED, Staged, StagedNone> lds;
+  const ShapeTables tab = stage_tables<STAGED>(P, &lds);
+  const GjkWork W{area + threadIdx.x, 64};
+  const int list = blockIdx.x & (kItemLists - 1);
+  const NarrowItem* items = sp.cf.items + (size_t)list * sp.cf.item_stride;
+  const int total = sp.cf.nitems[list * kItemPad];
+  const int stride = (gridDim.x / kItemLists) * 64;
+  for (int i = (blockIdx.x / kItemLists) * 64 + threadIdx.x; i < total; i += stride) {
+    const NarrowItem it = items[i];
+    if (closed && !closed_item(P, it)) continue;
+    narrow_one<true>(P, S, G, obs, sp, st, L, it.k, (int)(it.jc & kNbrSlotMask), nullptr, W, tab);
+  }
+}
+
+// What an evaluation that found a contact (or intersecting bodies) needs
+// beside the search, read again from memory so that none of it stays in
+// registers during the search.
+struct PairItem {
+  Self me;
+  int pid2, k2;
+  bool mirror;
+  d3 xo;
+};
+__device__ __forceinline__ void load_pair(const Particles& P, const Sorted& S, const Grid& G,
+                                          const BoxObstacle* __restrict__ obs, const StepParams& sp, const NbrList& L,
+                                          const NarrowItem& it, PairItem& q) {
+  int s;
+  load_self(P, S, sp, it.k, q.me, s);
+  q.k2 = -1;
+  q.mirror = false;
+  q.xo = d3{0., 0., 0.};
+  if (it.partner < 0) {
+    q.pid2 = obs[-1 - it.partner].id;
     return;
   }
-  const unsigned long long key = (unsigned long long)(unsigned)k << 32;
-  int c = 0;
-  for (unsigned long long m = (unsigned long long)keep[0]; m; m &= m - 1)
-    out[c++] = key | (unsigned)__builtin_ctzll(m);
-  for (unsigned long long m = (unsigned long long)keep[1]; m; m &= m - 1)
-    out[c++] = key | (unsigned)(nc + __builtin_ctzll(m));
-  const int last = (int)keep[2];
-  for (int o = 0; o <= last; ++o) sp.cf.ent[(size_t)(nc + o) * sp.cf.n + k] = kNoFeat;
-  sp.cf.count[k] = nc + last + 1;
+  const int j = (int)(it.jc & kNbrSlotMask), code = (int)(it.jc >> kNbrSlotBits);
+  q.k2 = (int)(L.ent[(size_t)j * L.n + it.k] & kNbrSlotMask);
+  q.xo = image_of(P, G, it.partner, sp.cur & 1, code);
+  q.pid2 = S.sid[q.k2];
+  // a pair searched here holds no two spheres
+  q.mirror = mirrored_pair(L, code, false, q.k2);
 }
 
-// One thread per sorted slot: counts its items, one atomic per wave reserves
-// the wave's run of the list, then each lane writes its items (from the
-// masks of the count pass when the candidates and obstacles fit 64 bits).
-// Particles without a usable list get count -1 (k_narrow_full).
-__global__ __launch_bounds__(256) void k_items(Particles P, Sorted S, const BoxObstacle* __restrict__ obs,
-                                               StepParams sp, NbrList L, const DevStatus* st) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool mine = k < sp.n && !st->code;  // after an error: an empty list
-  if (mine && L.count[k] > L.cap) sp.cf.count[k] = -1;
-  long long keep[3] = {0, 0, -1};
-  const int c = mine ? body_items(P, S, obs, sp, L, k, nullptr, keep) : 0;
-  // inclusive scan of the counts over the wave
-  const int lane = threadIdx.x & 63;
-  int incl = c;
-  for (int off = 1; off < 64; off <<= 1) {
-    const int v = __shfl_up(incl, off);
-    if (lane >= off) incl += v;
+// What follows an evaluation: errors, the recovery count, the records.
+__device__ __forceinline__ void item_result(const StepParams& sp, DevStatus* st, const NbrList& L,
+                                            const NarrowItem& it, const PairItem& q, int res, double d,
+                                            d3 Pc, d3 ov) {
+  if (res == 0) return;
+  if (res < 0) {
+    raise_error(st, kContactError, q.me.id, q.pid2);
+    return;
   }
-  const int total = __shfl(incl, 63);
-  int base = 0;
-  if (lane == 63 && total > 0) base = atomicAdd(sp.cf.nitems, total);
-  base = __shfl(base, 63);
-  if (mine && L.count[k] <= L.cap) {
-    unsigned long long* out = sp.cf.items + base + (incl - c);
-    if (L.cap <= 64 && sp.nobs <= 64) write_items(sp, k, L.count[k], keep, out);
-    else body_items(P, S, obs, sp, L, k, out);
-  }
+  if (res == 2) atomicAdd(&st->n_recovered, q.mirror ? 2 : 1);  // counted on each body's side
+  if (d < 0.)
+    put_item(sp, st, L, it.k, (int)(it.jc & kNbrSlotMask), it.s, q.me, it.partner, q.pid2, q.k2, q.mirror, q.xo, Pc, ov);
 }
 
-// The work list, one item per lane at a time (a grid of one-wave
-// workgroups that strides over it).
-__global__ __launch_bounds__(64) void k_narrow_items(Particles P, Sorted S, Grid G, const BoxObstacle* __restrict__ obs,
+// The work list with the default options.  Searches differ in length (most
+// pairs are proven apart within a few iterations, the others take up to a
+// dozen), so a wave holds up to 64 searches and steps them together; lanes
+// whose search has ended take the next items of the wave's run of the list
+// as soon as kRefill of them are free (starting a pair costs about as much
+// as two iterations, so not at once).  The next items are loaded ahead, so
+// that a start waits for one round of loads only.
+// Measured on the 200,000-body hopper (343 bodies in a box), per launch: 623
+// (68) us with a copy of the search per slot and vertices in memory, 289 (34)
+// with one copy over LDS, 232 (35) with the lanes refilled, 171 (30) with the
+// items naming what a start loads and the tables in LDS; refilling at 16 as at
+// 24 free lanes, 190 us at 40; held to two waves per SIMD the registers spill
+// (211 us).  Bound by the latency of one wave per SIMD (296 registers).
+constexpr int kRefill = 24;
+
+template <bool STAGED>
+__global__ __launch_bounds__(64) void k_narrow_lanes(Particles P, Sorted S, Grid G, const BoxObstacle* __restrict__ obs,
                                                      StepParams sp, DevStatus* st, NbrList L) {
-  const int total = *sp.cf.nitems;
-  for (int i = blockIdx.x * 64 + threadIdx.x; i < total; i += gridDim.x * 64) {
-    const unsigned long long it = sp.cf.items[i];
-    narrow_one<true>(P, S, G, obs, sp, st, L, (int)(it >> 32), (int)(unsigned)it, nullptr);
+  __shared__ double area[kGjkWork * 64];
+  __shared__ std::conditional_t<STAGED, Staged, StagedNone> lds;
+  const ShapeTables tab = stage_tables<STAGED>(P, &lds);
+  const GjkWork W{area + threadIdx.x, 64};
+  const int cx = sp.cur & 1;
+  const int lane = threadIdx.x;
+  const int list = blockIdx.x & (kItemLists - 1), waves = gridDim.x / kItemLists;
+  const NarrowItem* items = sp.cf.items + (size_t)list * sp.cf.item_stride;
+  const int total = sp.cf.nitems[list * kItemPad];
+  const int per = (total + waves - 1) / waves;
+  int next = (int)(blockIdx.x / kItemLists) * per;
+  const int end = min(next + per, total);
+  auto ahead = [&]() { return next + lane < end ? items[next + lane] : NarrowItem{0, 0u, 0, 0}; };
+  NarrowItem pre = ahead();
+  bool active = false;
+  NarrowItem it{0, 0u, 0, 0};
+  int att = 0;
+  ConvexGeo A{}, B{};
+  Tf a2w{}, b2w{};
+  GjkState g{};
+  double crusts = 0.;
+  auto start = [&]() {
+    const double* pr = S.posr + 4 * (size_t)it.k;
+    A = convex_of(P, it.s, d3{pr[0], pr[1], pr[2]}, cx, tab);
+    A.opt.sv = A.opt.accel = A.opt.bv = 0;
+    if (it.partner >= 0) B = convex_of(P, it.partner, image_of(P, G, it.partner, cx, (int)(it.jc >> kNbrSlotBits)), cx, tab);
+    else B = convex_of_obstacle(obs[-1 - it.partner]);
+    crusts = A.crust + B.crust;
+    // closed forms are k_narrow_items'; one with intersecting bodies as well
+    active = !closed_pair(A.type, B.type) && gjk_frames(A, B, att, a2w, b2w);
+    if (active) gjk_begin(A, a2w, B, b2w, g);
+  };
+  for (;;) {
+    const unsigned long long idle = __ballot(!active);
+    const int nidle = __popcll(idle);
+    if (next < end && nidle >= kRefill) {
+      // the r-th free lane takes the r-th of the items loaded ahead
+      const int r = __popcll(idle & ((1ull << lane) - 1ull));
+      const NarrowItem mine{__shfl(pre.k, r), (unsigned)__shfl((int)pre.jc, r), __shfl(pre.s, r), __shfl(pre.partner, r)};
+      const bool got = !active && next + r < end;
+      next += nidle;
+      pre = ahead();
+      if (got) {
+        it = mine;
+        att = 0;
+        // (a body whose candidates overflowed its list is k_narrow_full's)
+        if (L.count[it.k] <= L.cap) start();
+      }
+      continue;
+    }
+    if (nidle == 64) break;
+    if (active) {
+      const int go = gjk_step(A, a2w, B, b2w, W, att == 0 ? crusts : -1., g);
+      if (go == 2) active = false;
+      if (go == 0) {
+        d3 pa, pb, Pc, ov;
+        double d = 0.;
+        j_points(W, g.bits, pa, pb);
+        const int res = gjk_features(a2w, b2w, att, crusts, g.dist, pa, pb, Pc, ov, d);
+        active = false;
+        if (res < 0 && att == 0) {
+          att = 1;
+          start();
+        } else if (res != 1 || d < 0.) {
+          PairItem q;
+          load_pair(P, S, G, obs, sp, L, it, q);
+          item_result(sp, st, L, it, q, res, d, Pc, ov);
+        }
+      }
+    }
   }
 }
 
 // The generic 27-cell sweep for the particles k_narrow marked.
 __device__ __forceinline__ void narrow_full_one(const Particles& P, const Sorted& S, const Grid& G,
                                                 const BoxObstacle* __restrict__ obs, const StepParams& sp,
-                                                DevStatus* st, int k, StatAcc* acc) {
+                                                DevStatus* st, const NbrList& L, int k, StatAcc* acc,
+                                                const GjkWork& work, bool mirror) {
   const int cx = sp.cur & 1;
   Self me;
   int s;
   if (!load_self(P, S, sp, k, me, s)) return;
   me.acc = acc;
-  const ConvexGeo mg = convex_of(P, s, me.x, cx);
+  ConvexGeo mg = convex_of(P, s, me.x, cx, ShapeTables{P.shapes, P.verts});
+  mg.work = work;
   FeatureVisitor vis{sp.cf, k};
+  vis.mirror = mirror;
+  vis.P = &P;
+  vis.S = &S;
+  vis.L = &L;
+  vis.me = &me;
+  vis.s = s;
+  vis.st = st;
   for_each_contact<FeatureVisitor, true>(P, S, G, obs, sp.nobs, st, 0, 0, sp.n, k, me, vis, &mg, cx);
   sp.cf.count[k] = vis.c;
   if (vis.c > sp.cf.cap) raise_error(st, kContactOverflow, me.id, vis.c);
@@ -377,48 +501,69 @@ __device__ __forceinline__ void narrow_full_one(const Particles& P, const Sorted
 // One thread per sorted slot, records packed: with statistics (256-thread
 // workgroups whose partial sums k_stats_fold adds up), and for lists too
 // long for the slot layout.
-__global__ __launch_bounds__(256) void k_narrow(Particles P, Sorted S, Grid G, const BoxObstacle* __restrict__ obs,
-                                                StepParams sp, DevStatus* st, NbrList L) {
-  const int k = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+// (BS threads: 256 with statistics)
+template <int BS>
+__global__ __launch_bounds__(BS) void k_narrow(Particles P, Sorted S, Grid G, const BoxObstacle* __restrict__ obs,
+                                               StepParams sp, DevStatus* st, NbrList L) {
+  __shared__ double area[kGjkWork * BS];
+  const GjkWork W{area + threadIdx.x, BS};
+  const int k = xcd_tile(blockIdx.x, gridDim.x) * BS + threadIdx.x;
   const bool mine = k < sp.n && !st->code;  // an error ended the run
-  if (!sp.stats) {
-    if (mine) narrow_one<false>(P, S, G, obs, sp, st, L, k, 0, nullptr);
+  if (BS == 64) {
+    if (mine) narrow_one<false>(P, S, G, obs, sp, st, L, k, 0, nullptr, W, ShapeTables{P.shapes, P.verts});
     return;
   }
   StatAcc acc;
-  if (mine) narrow_one<false>(P, S, G, obs, sp, st, L, k, 0, &acc);
+  if (mine) narrow_one<false>(P, S, G, obs, sp, st, L, k, 0, &acc, W, ShapeTables{P.shapes, P.verts});
   block_stats(acc, sp.stats + 5 * (size_t)blockIdx.x);
 }
 
-__global__ __launch_bounds__(256) void k_narrow_full(Particles P, Sorted S, Grid G,
-                                                     const BoxObstacle* __restrict__ obs, StepParams sp,
-                                                     DevStatus* st) {
-  const int k = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+template <int BS>
+__global__ __launch_bounds__(BS) void k_narrow_full(Particles P, Sorted S, Grid G,
+                                                    const BoxObstacle* __restrict__ obs, StepParams sp,
+                                                    DevStatus* st, NbrList L, bool mirror) {
+  // the work list is empty again for the next step
+  if (blockIdx.x == 0 && threadIdx.x < kItemLists) sp.cf.nitems[threadIdx.x * kItemPad] = 0;
+  __shared__ double area[kGjkWork * BS];
+  const GjkWork W{area + threadIdx.x, BS};
+  const int k = xcd_tile(blockIdx.x, gridDim.x) * BS + threadIdx.x;
   const bool mine = k < sp.n && sp.cf.count[k] < 0 && !st->code;
-  if (!sp.stats) {
-    if (mine) narrow_full_one(P, S, G, obs, sp, st, k, nullptr);
+  if (BS == 64) {
+    if (mine) narrow_full_one(P, S, G, obs, sp, st, L, k, nullptr, W, mirror);
     return;
   }
   StatAcc acc;
-  if (mine) narrow_full_one(P, S, G, obs, sp, st, k, &acc);
+  if (mine) narrow_full_one(P, S, G, obs, sp, st, L, k, &acc, W, false);
   block_stats<true>(acc, sp.stats + 5 * (size_t)blockIdx.x);
 }
 
 hipError_t launch_narrow(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
                          const StepParams& sp, DevStatus* st, const NbrList& L, hipStream_t stream) {
   if (sp.n == 0) return hipSuccess;
+  const dim3 grid64((sp.n + 63) / 64), grid256((sp.n + 255) / 256);
   // packed records where slots would not fit the obstacles' records
-  if (sp.stats || !L.count || L.cap + sp.nobs > sp.cf.cap) {
-    const dim3 grid((sp.n + 255) / 256);
-    hipLaunchKernelGGL(k_narrow, grid, dim3(256), 0, stream, P, S, G, obs, sp, st, L);
-    hipLaunchKernelGGL(k_narrow_full, grid, dim3(256), 0, stream, P, S, G, obs, sp, st);
+  if (sp.stats) {
+    hipLaunchKernelGGL(k_narrow<256>, grid256, dim3(256), 0, stream, P, S, G, obs, sp, st, L);
+    hipLaunchKernelGGL(k_narrow_full<256>, grid256, dim3(256), 0, stream, P, S, G, obs, sp, st, L, false);
     return hipGetLastError();
   }
-  hipError_t e = launch_clear(sp.cf.nitems, 1, stream);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_items, dim3((sp.n + 255) / 256), dim3(256), 0, stream, P, S, obs, sp, L, st);
-  hipLaunchKernelGGL(k_narrow_items, dim3(sp.cf.item_blocks), dim3(64), 0, stream, P, S, G, obs, sp, st, L);
-  hipLaunchKernelGGL(k_narrow_full, dim3((sp.n + 63) / 64), dim3(64), 0, stream, P, S, G, obs, sp, st);
+  if (!L.count || L.cap + sp.nobs > sp.cf.cap) {
+    hipLaunchKernelGGL(k_narrow<64>, grid64, dim3(64), 0, stream, P, S, G, obs, sp, st, L);
+    hipLaunchKernelGGL(k_narrow_full<64>, grid64, dim3(64), 0, stream, P, S, G, obs, sp, st, L, false);
+    return hipGetLastError();
+  }
+  const dim3 grid(sp.cf.item_blocks), block(64);
+  const bool plain = !P.gjk.sv && !P.gjk.accel && !P.gjk.bv;
+  const bool staged = P.nverts <= kStageVerts && P.nshapes <= kStageShapes;
+  if (plain) {
+    if (staged) hipLaunchKernelGGL(k_narrow_lanes<true>, grid, block, 0, stream, P, S, G, obs, sp, st, L);
+    else hipLaunchKernelGGL(k_narrow_lanes<false>, grid, block, 0, stream, P, S, G, obs, sp, st, L);
+  }
+  if (!plain || P.spheres) {
+    if (staged) hipLaunchKernelGGL(k_narrow_items<true>, grid, block, 0, stream, P, S, G, obs, sp, st, L, plain);
+    else hipLaunchKernelGGL(k_narrow_items<false>, grid, block, 0, stream, P, S, G, obs, sp, st, L, plain);
+  }
+  hipLaunchKernelGGL(k_narrow_full<64>, grid64, block, 0, stream, P, S, G, obs, sp, st, L, true);
   return hipGetLastError();
 }
 

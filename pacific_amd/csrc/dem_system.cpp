@@ -122,6 +122,11 @@ int grains_gpu_system::allocate() {
     HIPCHECK(this, track(this, &d_verts, shape_verts.size()));
     P.shapes = d_shapes;
     P.verts = d_verts;
+    P.nshapes = (int)shapes.size();
+    P.nverts = (int)(shape_verts.size() / 3);
+    P.spheres = 0;
+    for (int sh : h_shape)
+      if (sh < 0 || shapes[sh].type == kShapeSphere) P.spheres = 1;
     P.gjk = gjk_opts;
   }
   HIPCHECK(this, track(this, &d_obs, obstacles.size()));
@@ -157,11 +162,15 @@ int grains_gpu_system::allocate() {
     HIPCHECK(this, hipMemsetAsync(cf.count, 0, sizeof(int) * n, stream));
     cf.cap = (int)fcap;
     cf.n = (int)n;
-    HIPCHECK(this, track(this, &cf.items, fcap * n));
-    HIPCHECK(this, track(this, &cf.nitems, 1));
+    const size_t blocks = (n + kDetectBodies - 1) / kDetectBodies;
+    cf.item_stride = (int)((blocks + kItemLists - 1) / kItemLists * kDetectBodies * fcap);
+    HIPCHECK(this, track(this, &cf.items, (size_t)kItemLists * cf.item_stride));
+    HIPCHECK(this, track(this, &cf.nitems, (size_t)kItemLists * kItemPad));
+    HIPCHECK(this, hipMemsetAsync(cf.nitems, 0, sizeof(int) * kItemLists * kItemPad, stream));
     int ncu = 0;
     HIPCHECK(this, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
-    cf.item_blocks = 8 * std::max(ncu, 1);  // one-wave workgroups, two per SIMD
+    // one-wave workgroups, one per SIMD, equally many for each part of the list
+    cf.item_blocks = (4 * std::max(ncu, 1) + kItemLists - 1) / kItemLists * kItemLists;
   }
   HIPCHECK(this, track(this, &d_stat_part, 5 * ((n + 255) / 256) + 5));
   HIPCHECK(this, track(this, &d_stat_tot, 8));
@@ -395,7 +404,7 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
   const dem::NbrList L = nbr_list();
   if (L.count && !verlet) {
     if (prof && (e = mark(prof->detect_ev, prof->ndetect))) return e;
-    HIPCHECK(this, launch_detect(S, grid, nparticles, L, d_status, stream, P.shape ? cf.ent : nullptr));
+    HIPCHECK(this, launch_detect(P, S, grid, d_obs, sp, L, d_status, stream));
     if (prof && (e = mark(prof->detect_ev, prof->ndetect))) return e;
   }
   if (P.shape) {
@@ -806,6 +815,9 @@ int grains_gpu_add_shape(grains_gpu_system* s, int type, double radius, const do
     return fail(s, GRAINS_CONFIG_ERROR, err);
   b.desc.vert_off = (int)(s->shape_verts.size() / 3);
   s->shape_verts.insert(s->shape_verts.end(), b.verts.begin(), b.verts.end());
+  // whole groups of vertices (support)
+  for (int i = nv; type == kShapePoly && i % kVertGroup; ++i)
+    s->shape_verts.insert(s->shape_verts.end(), b.verts.end() - 3, b.verts.end());
   std::vector<int> faces;
   if (type == kShapePoly) {
     int off = 0;

@@ -117,6 +117,8 @@ struct Particles {
   double* I3[3];
   const ShapeDesc* shapes;
   const double* verts;
+  int nshapes, nverts;  // entries of the two tables
+  int spheres;  // whether any body of a system with non-spherical ones is a sphere
   GjkOpts gjk;  // narrow phase options of the system's general pairs
 };
 
@@ -193,17 +195,32 @@ enum ErrCode {
 // A slot whose candidate is not in contact holds ent = kNoFeat (neither a
 // storage index nor an obstacle).
 constexpr int kNoFeat = -2147483647 - 1;
+// One evaluation: body A's sorted slot k and storage index s, its record slot
+// j with the periodic image code above kNbrSlotBitsHost, and the partner (as
+// in ContactFeat::ent).  Everything that the search needs to load is named
+// here, so that its loads do not wait for one another.
+struct alignas(16) NarrowItem {
+  int k;
+  unsigned jc;
+  int s, partner;
+};
+// The list is appended to in parts with a counter each, on lines of their
+// own: atomics on one address are served one at a time.
+constexpr int kItemLists = 8;
+constexpr int kItemPad = 32;
 struct ContactFeat {
   int* count;    // [n] record slots of each sorted slot (may exceed cap: error)
   int* ent;      // [cap * n]
   int* pid;      // [cap * n]
   double* f[9];  // [cap * n] each
   int cap, n;
-  // the narrow phase's work list: (sorted slot << 32 | record slot) of
-  // every evaluation of the step, and its length
-  unsigned long long* items;  // [cap * n]
+  // the narrow phase's work list: every evaluation of the step, in kItemLists
+  // parts of item_stride entries each, and their lengths (kItemPad ints
+  // apart; zero between steps)
+  NarrowItem* items;
   int* nitems;
-  int item_blocks;  // workgroups of the work-list kernel
+  int item_stride;
+  int item_blocks;  // workgroups of the work-list kernels
 };
 enum Scheme { kLeapFrog = 0, kFirstOrderExplicit = 1, kSecondOrderExplicit = 2, kAdamsBashforth2 = 3 };
 
