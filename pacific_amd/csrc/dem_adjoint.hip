@@ -377,18 +377,16 @@ int grains_gpu_adjoint_backward(grains_gpu_system* s, int matA, int matB, const 
     ACHECK(s, hipMalloc((void**)&A.gth, 3 * n * sizeof(double)));
     ad->allocs.push_back(A.gth);
   }
-  // storage <-> id order
-  std::vector<int> ids(n);
-  ACHECK(s, hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost));
-  std::vector<double> buf(n);
-  auto up = [&](double* dst, const double* src, int c) -> hipError_t {
-    for (int i = 0; i < N; ++i) buf[i] = src ? src[3 * (size_t)(ids[i] - 1) + c] : 0.;
-    return hipMemcpy(dst, buf.data(), n * sizeof(double), hipMemcpyHostToDevice);
-  };
+  // cotangents of the final state, rows by id
+  RowIO in(N);
+  in.add(dJ_dx, A.xb, 3);
+  in.add(dJ_dv, A.vb, 3);
+  in.add(dJ_dw, A.wb, 3);
+  ACHECK(s, s->rows.up(in, s->P.id, N, s->device, s->stream));
   for (int c = 0; c < 3; ++c) {
-    ACHECK(s, up(A.xb[c], dJ_dx, c));
-    ACHECK(s, up(A.vb[c], dJ_dv, c));
-    ACHECK(s, up(A.wb[c], dJ_dw, c));
+    if (!dJ_dx) ACHECK(s, hipMemsetAsync(A.xb[c], 0, n * sizeof(double), s->stream));
+    if (!dJ_dv) ACHECK(s, hipMemsetAsync(A.vb[c], 0, n * sizeof(double), s->stream));
+    if (!dJ_dw) ACHECK(s, hipMemsetAsync(A.wb[c], 0, n * sizeof(double), s->stream));
   }
   const double h = 0.5 * s->cfg.dt, dt = s->cfg.dt;
   hipLaunchKernelGGL(k_adj_init, dim3(nblk(N, 256)), dim3(256), 0, s->stream, s->P, A, N, h);
@@ -437,19 +435,12 @@ int grains_gpu_adjoint_backward(grains_gpu_system* s, int matA, int matB, const 
   hipLaunchKernelGGL(k_adj_sweep, dim3(nblk(N, 64)), dim3(64), 0, s->stream, s->P, s->S, s->grid, s->d_obs,
                      (int)s->obstacles.size(), s->d_models, A, N, 0, matA, matB, h, dt, 1., 1, s->d_status);
   ACHECK(s, hipGetLastError());
-  ACHECK(s, hipStreamSynchronize(s->stream));
   // results
-  auto down = [&](double* dst, double* src, int c) -> hipError_t {
-    if (!dst) return hipSuccess;
-    hipError_t er = hipMemcpy(buf.data(), src, n * sizeof(double), hipMemcpyDeviceToHost);
-    for (int i = 0; i < N; ++i) dst[3 * (size_t)(ids[i] - 1) + c] = buf[i];
-    return er;
-  };
-  for (int c = 0; c < 3; ++c) {
-    ACHECK(s, down(grad_x0, A.xb[c], c));
-    ACHECK(s, down(grad_v0, A.vb[c], c));
-    ACHECK(s, down(grad_w0, A.wb[c], c));
-  }
+  RowIO out(N);
+  out.add(grad_x0, A.xb, 3);
+  out.add(grad_v0, A.vb, 3);
+  out.add(grad_w0, A.wb, 3);
+  ACHECK(s, s->rows.down(out, s->P.id, N, s->device, s->stream));
   if (grad_params) {
     std::vector<double> gth(3 * n);
     ACHECK(s, hipMemcpy(gth.data(), A.gth, 3 * n * sizeof(double), hipMemcpyDeviceToHost));

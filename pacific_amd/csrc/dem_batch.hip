@@ -386,9 +386,14 @@ struct grains_gpu_batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::vector<void*> allocations;
+  RowBuffers rows;                // buffers of the state transfers
+  DevStatus* h_status = nullptr;  // pinned
   ~grains_gpu_batch();
   int launch(int mode, int nsteps);
   int launch_flat(int mode, int nsteps);
+  // as grains_gpu_system::fetch_status, read_status, check_status
+  int fetch();
+  int read();
   int check();
 };
 
@@ -426,6 +431,8 @@ grains_gpu_batch::~grains_gpu_batch() {
   if (exec) (void)hipGraphExecDestroy(exec);
   if (graph) (void)hipGraphDestroy(graph);
   for (void* p : allocations) (void)hipFree(p);
+  rows.release();
+  if (h_status) (void)hipHostFree(h_status);
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
   if (stream) (void)hipStreamDestroy(stream);
@@ -488,10 +495,20 @@ int grains_gpu_batch::launch(int mode, int nsteps) {
   return GRAINS_OK;
 }
 
+int grains_gpu_batch::fetch() {
+  BCHECK(this, hipMemcpyAsync(h_status, d_status, sizeof(DevStatus), hipMemcpyDeviceToHost, stream));
+  return GRAINS_OK;
+}
+
 int grains_gpu_batch::check() {
-  DevStatus st;
-  BCHECK(this, hipMemcpyAsync(&st, d_status, sizeof(st), hipMemcpyDeviceToHost, stream));
+  int e = fetch();
+  if (e) return e;
   BCHECK(this, hipStreamSynchronize(stream));
+  return read();
+}
+
+int grains_gpu_batch::read() {
+  const DevStatus st = *h_status;
   last_status = st;
   if (st.code) {
     static const char* names[] = {"", "ContactError", "MotionError", "SimulationError"};
@@ -667,6 +684,7 @@ int grains_gpu_batch_create(grains_gpu_system* const* systems, int nsys, int pre
   BCHECK(b, balloc(b, &b->d_models, hmod.size()));
   BCHECK(b, up(b->d_models, hmod));
   BCHECK(b, balloc(b, &b->d_status, 1));
+  BCHECK(b, hipHostMalloc((void**)&b->h_status, sizeof(DevStatus), hipHostMallocDefault));
   BCHECK(b, hipMemset(b->d_status, 0, sizeof(DevStatus)));
   b->time = systems[0]->cfg.t_start;
   int e = b->launch(0, 0);  // bin + initial forces
@@ -805,26 +823,23 @@ int grains_gpu_batch_get_state(grains_gpu_batch* b, int isys, double* x, double*
                                double* T) {
   if (!b || isys < 0 || isys >= b->nsys) return GRAINS_ARGUMENT_ERROR;
   BCHECK(b, hipSetDevice(b->device));
-  BCHECK(b, hipStreamSynchronize(b->stream));
   const int n = b->np[isys], p0 = b->p0[isys];
-  std::vector<int> ids((size_t)n);
-  BCHECK(b, hipMemcpy(ids.data(), b->P.id + p0, sizeof(int) * n, hipMemcpyDeviceToHost));
-  std::vector<double> buf((size_t)n);
-  auto down = [&](double* dst, double* src, int stride, int comp) -> hipError_t {
-    if (!dst) return hipSuccess;
-    hipError_t e = hipMemcpy(buf.data(), src + p0, sizeof(double) * n, hipMemcpyDeviceToHost);
-    for (int i = 0; i < n; ++i) dst[(size_t)stride * (ids[i] - 1) + comp] = buf[i];
-    return e;
+  auto at = [&](double* const* a, int k, double** o) {
+    for (int c = 0; c < k; ++c) o[c] = a[c] + p0;
+    return o;
   };
-  for (int a = 0; a < 3; ++a) {
-    BCHECK(b, down(x, b->P.x[0][a], 3, a));
-    BCHECK(b, down(v, b->P.v[0][a], 3, a));
-    BCHECK(b, down(w, b->P.w[0][a], 3, a));
-    BCHECK(b, down(F, b->P.F[a], 3, a));
-    BCHECK(b, down(T, b->P.T[a], 3, a));
-  }
-  for (int a = 0; a < 4; ++a) BCHECK(b, down(q, b->P.q[a], 4, a));
-  return b->check();
+  double* o[4];
+  RowIO io(n);
+  io.add(x, at(b->P.x[0], 3, o), 3);
+  io.add(v, at(b->P.v[0], 3, o), 3);
+  io.add(w, at(b->P.w[0], 3, o), 3);
+  io.add(q, at(b->P.q, 4, o), 4);
+  io.add(F, at(b->P.F, 3, o), 3);
+  io.add(T, at(b->P.T, 3, o), 3);
+  int e = b->fetch();
+  if (e) return e;
+  BCHECK(b, b->rows.down(io, b->P.id + p0, n, b->device, b->stream));
+  return b->read();
 }
 
 const char* grains_gpu_batch_last_error(const grains_gpu_batch* b) { return b ? b->last_error.c_str() : "null batch"; }

@@ -50,6 +50,9 @@ void grains_gpu_system::free_device() {
   drop_graphs();
   for (void* p : allocations) (void)hipFree(p);
   allocations.clear();
+  rows.release();
+  if (h_status) (void)hipHostFree(h_status);
+  h_status = nullptr;
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
   if (stream) (void)hipStreamDestroy(stream);
@@ -132,6 +135,7 @@ int grains_gpu_system::allocate() {
   HIPCHECK(this, track(this, &d_obs, obstacles.size()));
   HIPCHECK(this, track(this, &d_models, (size_t)kMaxMaterials * kMaxMaterials));
   HIPCHECK(this, track(this, &d_status, 1));
+  HIPCHECK(this, hipHostMalloc((void**)&h_status, sizeof(DevStatus), hipHostMallocDefault));
   if (verlet)
     for (int a = 0; a < 3; ++a) HIPCHECK(this, track(this, &V.xb[a], n));
   mem = dem::ContactMemory{};
@@ -566,10 +570,20 @@ int grains_gpu_system::graph_chunk(bool& done) {
   return GRAINS_OK;
 }
 
+int grains_gpu_system::fetch_status() {
+  HIPCHECK(this, hipMemcpyAsync(h_status, d_status, sizeof(DevStatus), hipMemcpyDeviceToHost, stream));
+  return GRAINS_OK;
+}
+
 int grains_gpu_system::check_status() {
-  DevStatus st;
-  HIPCHECK(this, hipMemcpyAsync(&st, d_status, sizeof(DevStatus), hipMemcpyDeviceToHost, stream));
+  int e = fetch_status();
+  if (e) return e;
   HIPCHECK(this, hipStreamSynchronize(stream));
+  return read_status();
+}
+
+int grains_gpu_system::read_status() {
+  const DevStatus st = *h_status;
   last_status = st;
   if (st.code) {
     static const char* names[] = {"", "ContactError", "MotionError", "SimulationError"};
@@ -1131,13 +1145,12 @@ int grains_gpu_set_hydro_ft(grains_gpu_system* s, const double* ft, size_t m) {
   if (n == 0) return GRAINS_OK;
   const bool fresh = !s->d_hyd;
   if (fresh) HIPCHECK(s, track(s, &s->d_hyd, 6 * (size_t)n));
-  std::vector<int> ids((size_t)n);
-  HIPCHECK(s, hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost));
-  std::vector<double> buf(6 * (size_t)n);
-  for (int i = 0; i < n; ++i)
-    for (int c = 0; c < 6; ++c) buf[(size_t)c * n + i] = ft[6 * (size_t)(ids[i] - 1) + c];
+  double* comps[6];
+  for (int c = 0; c < 6; ++c) comps[c] = s->d_hyd + (size_t)c * n;
+  RowIO io(n);
+  io.add(ft, comps, 6);
+  HIPCHECK(s, s->rows.up(io, s->P.id, n, s->device, s->stream));
   HIPCHECK(s, hipStreamSynchronize(s->stream));
-  HIPCHECK(s, hipMemcpy(s->d_hyd, buf.data(), sizeof(double) * buf.size(), hipMemcpyHostToDevice));
   // step graphs captured before hold StepParams without the fluid forces
   if (fresh) s->drop_graphs();
   return GRAINS_OK;
@@ -1166,45 +1179,31 @@ int grains_gpu_get_state(grains_gpu_system* s, double* x, double* v, double* w, 
                          double* T) {
   if (!s || !s->initialized) return GRAINS_ARGUMENT_ERROR;
   HIPCHECK(s, hipSetDevice(s->device));
-  HIPCHECK(s, hipStreamSynchronize(s->stream));
   const int n = s->nparticles;
-  std::vector<int> ids((size_t)n);
-  HIPCHECK(s, hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost));
-  std::vector<double> buf((size_t)n);
   const int cx = s->cur & 1, cv = (s->cur >> 1) & 1;
-  auto down = [&](double* dst, double* src, int stride, int comp) -> hipError_t {
-    if (!dst) return hipSuccess;
-    hipError_t e = hipMemcpy(buf.data(), src, sizeof(double) * n, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return e;
-    for (int i = 0; i < n; ++i) dst[(size_t)stride * (ids[i] - 1) + comp] = buf[i];
-    return hipSuccess;
-  };
-  for (int a = 0; a < 3; ++a) {
-    HIPCHECK(s, down(x, s->P.x[cx][a], 3, a));
-    HIPCHECK(s, down(v, s->P.v[cv][a], 3, a));
-    HIPCHECK(s, down(w, s->P.w[cv][a], 3, a));
-    HIPCHECK(s, down(wb, s->P.wb[a], 3, a));
-    HIPCHECK(s, down(F, s->P.F[a], 3, a));
-    HIPCHECK(s, down(T, s->P.T[a], 3, a));
-  }
-  for (int a = 0; a < 4; ++a) HIPCHECK(s, down(q, s->P.q[a], 4, a));
-  return s->check_status();
+  RowIO io(n);
+  io.add(x, s->P.x[cx], 3);
+  io.add(v, s->P.v[cv], 3);
+  io.add(w, s->P.w[cv], 3);
+  io.add(wb, s->P.wb, 3);
+  io.add(q, s->P.q, 4);
+  io.add(F, s->P.F, 3);
+  io.add(T, s->P.T, 3);
+  // the status comes back with the rows
+  int e = s->fetch_status();
+  if (e) return e;
+  HIPCHECK(s, s->rows.down(io, s->P.id, n, s->device, s->stream));
+  return s->read_status();
 }
 
 int grains_gpu_get_basis(grains_gpu_system* s, double* B) {
   if (!s || !s->initialized || !B) return GRAINS_ARGUMENT_ERROR;
   if (!s->has_shapes()) return fail(s, GRAINS_ARGUMENT_ERROR, "the system has no non-spherical particles");
   HIPCHECK(s, hipSetDevice(s->device));
-  HIPCHECK(s, hipStreamSynchronize(s->stream));
   const int n = s->nparticles;
-  std::vector<int> ids((size_t)n);
-  HIPCHECK(s, hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost));
-  std::vector<double> buf((size_t)n);
-  const int cx = s->cur & 1;
-  for (int j = 0; j < 9; ++j) {
-    HIPCHECK(s, hipMemcpy(buf.data(), s->P.B[cx][j], sizeof(double) * n, hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; ++i) B[9 * (size_t)(ids[i] - 1) + j] = buf[i];
-  }
+  RowIO io(n);
+  io.add(B, s->P.B[s->cur & 1], 9);
+  HIPCHECK(s, s->rows.down(io, s->P.id, n, s->device, s->stream));
   return s->check_status();
 }
 
@@ -1212,16 +1211,11 @@ int grains_gpu_set_basis(grains_gpu_system* s, const double* B) {
   if (!s || !s->initialized || !B) return GRAINS_ARGUMENT_ERROR;
   if (!s->has_shapes()) return fail(s, GRAINS_ARGUMENT_ERROR, "the system has no non-spherical particles");
   HIPCHECK(s, hipSetDevice(s->device));
-  HIPCHECK(s, hipStreamSynchronize(s->stream));
   const int n = s->nparticles;
-  std::vector<int> ids((size_t)n);
-  HIPCHECK(s, hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost));
-  std::vector<double> buf((size_t)n);
-  const int cx = s->cur & 1;
-  for (int j = 0; j < 9; ++j) {
-    for (int i = 0; i < n; ++i) buf[i] = B[9 * (size_t)(ids[i] - 1) + j];
-    HIPCHECK(s, hipMemcpy(s->P.B[cx][j], buf.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-  }
+  RowIO io(n);
+  io.add(B, s->P.B[s->cur & 1], 9);
+  HIPCHECK(s, s->rows.up(io, s->P.id, n, s->device, s->stream));
+  HIPCHECK(s, hipStreamSynchronize(s->stream));
   return GRAINS_OK;
 }
 
@@ -1229,49 +1223,16 @@ int grains_gpu_set_state(grains_gpu_system* s, const double* x, const double* v,
                          int recompute_forces) {
   if (!s || !s->initialized) return GRAINS_ARGUMENT_ERROR;
   HIPCHECK(s, hipSetDevice(s->device));
-  HIPCHECK(s, hipStreamSynchronize(s->stream));
   const int n = s->nparticles;
-  std::vector<int> ids((size_t)n);
-  HIPCHECK(s, hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost));
   const int cx = s->cur & 1, cv = (s->cur >> 1) & 1;
-  std::vector<double> buf((size_t)n);
-  auto get = [&](double* src, std::vector<double>& dst, int stride, int comp) -> hipError_t {
-    hipError_t e = hipMemcpy(buf.data(), src, sizeof(double) * n, hipMemcpyDeviceToHost);
-    for (int i = 0; i < n; ++i) dst[(size_t)stride * (ids[i] - 1) + comp] = buf[i];
-    return e;
-  };
-  auto put = [&](double* dst, const std::vector<double>& src, int stride, int comp) -> hipError_t {
-    for (int i = 0; i < n; ++i) buf[i] = src[(size_t)stride * (ids[i] - 1) + comp];
-    return hipMemcpy(dst, buf.data(), sizeof(double) * n, hipMemcpyHostToDevice);
-  };
-  // current q and w (needed to rebuild the body-fixed angular velocity)
-  std::vector<double> qq((size_t)4 * n), ww((size_t)3 * n);
-  for (int a = 0; a < 4; ++a) HIPCHECK(s, get(s->P.q[a], qq, 4, a));
-  for (int a = 0; a < 3; ++a) HIPCHECK(s, get(s->P.w[cv][a], ww, 3, a));
-  if (q) std::copy(q, q + 4 * (size_t)n, qq.begin());
-  if (w) std::copy(w, w + 3 * (size_t)n, ww.begin());
-  std::vector<double> wbv((size_t)3 * n);
-  for (int i = 0; i < n; ++i) {
-    quat qi{d3{qq[4 * i], qq[4 * i + 1], qq[4 * i + 2]}, qq[4 * i + 3]};
-    d3 wb = to_body(qi, d3{ww[3 * i], ww[3 * i + 1], ww[3 * i + 2]});
-    wbv[3 * i] = wb.x;
-    wbv[3 * i + 1] = wb.y;
-    wbv[3 * i + 2] = wb.z;
-  }
-  std::vector<double> tmp;
-  for (int a = 0; a < 3; ++a) {
-    if (x) {
-      tmp.assign(x, x + 3 * (size_t)n);
-      HIPCHECK(s, put(s->P.x[cx][a], tmp, 3, a));
-    }
-    if (v) {
-      tmp.assign(v, v + 3 * (size_t)n);
-      HIPCHECK(s, put(s->P.v[cv][a], tmp, 3, a));
-    }
-    HIPCHECK(s, put(s->P.w[cv][a], ww, 3, a));
-    HIPCHECK(s, put(s->P.wb[a], wbv, 3, a));
-  }
-  for (int a = 0; a < 4; ++a) HIPCHECK(s, put(s->P.q[a], qq, 4, a));
+  RowIO io(n);
+  io.add(x, s->P.x[cx], 3);
+  io.add(v, s->P.v[cv], 3);
+  io.add(w, s->P.w[cv], 3);
+  io.add(q, s->P.q, 4);
+  HIPCHECK(s, s->rows.up(io, s->P.id, n, s->device, s->stream));
+  // the body-fixed angular velocity follows w and q, given or kept
+  HIPCHECK(s, launch_body_spin(s->P, n, cv, s->stream));
   int e = s->bin_current();
   if (e) return e;
   if (recompute_forces) {

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/grains_gpu.h"
+#include "dem_io.hpp"
 #include "dem_types.hpp"
 
 namespace dem {
@@ -141,6 +142,8 @@ struct grains_gpu_system {
     v.stamp = verlet ? st : 0;
     return v;
   }
+  dem::RowBuffers rows;               // buffers of the state transfers
+  dem::DevStatus* h_status = nullptr;  // pinned: the status block comes back without a staging copy
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::vector<void*> allocations;
@@ -186,6 +189,10 @@ struct grains_gpu_system {
   int graph_chunk(bool& done);
   void drop_graphs();
   int recover();
+  // fetch_status enqueues the copy of the status block, read_status looks at
+  // it once the stream has drained; check_status does both
+  int fetch_status();
+  int read_status();
   int check_status();
   // particles of the XML input waiting for insertion over time
   // (<Mode Type="OverTime">), tried once per step by the time loop
