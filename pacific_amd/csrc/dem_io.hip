@@ -62,6 +62,42 @@ hipError_t launch_body_spin(const Particles& P, int n, int cv, hipStream_t strea
   return hipGetLastError();
 }
 
+template <class T>
+struct ArrayGroup {
+  T* a[kPermuteGroup];
+};
+// blockIdx.y selects the array; gather into tmp, then back
+template <class T>
+__global__ __launch_bounds__(256) void k_permute(ArrayGroup<T> g, const int* __restrict__ order, int n,
+                                                 T* __restrict__ tmp, bool back) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  T* const t = tmp + (size_t)blockIdx.y * n;
+  if (back) {
+    g.a[blockIdx.y][i] = t[i];
+  } else {
+    const int o = order[i];
+    t[i] = g.a[blockIdx.y][(unsigned)o < (unsigned)n ? o : i];
+  }
+}
+template <class T>
+static hipError_t permute_arrays(const std::vector<T*>& a, const int* order, int n, T* tmp, hipStream_t stream) {
+  for (size_t k = 0; k < a.size(); k += kPermuteGroup) {
+    ArrayGroup<T> g{};
+    const int m = (int)std::min<size_t>(kPermuteGroup, a.size() - k);
+    for (int j = 0; j < m; ++j) g.a[j] = a[k + j];
+    for (int back = 0; back < 2; ++back)
+      hipLaunchKernelGGL(k_permute<T>, dim3((n + 255) / 256, m), dim3(256), 0, stream, g, order, n, tmp, back != 0);
+  }
+  return hipGetLastError();
+}
+hipError_t launch_permute(const std::vector<double*>& a8, const std::vector<int*>& a4, const int* order, int n,
+                          double* tmp, hipStream_t stream) {
+  if (n == 0) return hipSuccess;
+  hipError_t e = permute_arrays(a8, order, n, tmp, stream);
+  return e == hipSuccess ? permute_arrays(a4, order, n, (int*)tmp, stream) : e;
+}
+
 void RowIO::add(double* host, double* const* comps, int width) {
   if (!host || n_ == 0) return;
   for (int c = 0; c < width; ++c) {

@@ -25,6 +25,12 @@ hipError_t launch_rows_in(const RowMap& m, const int* id, int n, const double* i
 // body-fixed angular velocity from w and q (ParticleKinematics::setAngularVelocity)
 hipError_t launch_body_spin(const Particles& P, int n, int cv, hipStream_t stream);
 
+// a[k][i] <- a[k][order[i]] for every array (8- and 4-byte elements); tmp
+// holds kPermuteGroup * n doubles
+constexpr int kPermuteGroup = 4;
+hipError_t launch_permute(const std::vector<double*>& a8, const std::vector<int*>& a4, const int* order, int n,
+                          double* tmp, hipStream_t stream);
+
 // The rows of one call (rows of `width` doubles per particle in the caller's
 // array; a null array is left out) and the buffers they pass through: a device
 // buffer in row layout and pinned host slices, both kept for the next call

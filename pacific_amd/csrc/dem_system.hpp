@@ -156,6 +156,10 @@ struct grains_gpu_system {
   void free_device();
   dem::StepParams params() const;
   int bin_current();
+  // particles given in an order without relation to their places are stored
+  // in cell order (see there)
+  bool scattered() const;
+  int sort_storage();
   int reset_pair_counter();
   // commit: the evaluation belongs to the time loop (contact memory advances)
   int forces(int mode, int first_step, bool commit = true);

@@ -1,0 +1,61 @@
+"""Particles given in an order without relation to their places are stored in
+cell order: everything by id stays what it is.  Against the oracle, which keeps
+the given order: contact records equal, forces within 1e-12 of weight plus
+contact force (the order of a particle's sum is the list's, by cells and ids,
+as without), states in id order after some steps."""
+import numpy as np
+import pytest
+
+from pacific_amd import workloads
+from tests.helpers import contact_scale, make_gpu, make_oracle, pair_set, rel_force_error
+
+pytestmark = pytest.mark.gpu
+
+
+def shuffled(kind):
+    rng = np.random.default_rng(4)
+    if kind == "polyhedra":
+        wl = workloads.polyhedra_box((17, 17, 15), seed=3, spheres=True, sigma=0.3)
+        # touching from the start: the lattice pulled together
+        wl["groups"] = [(g[0], 2.2e-3 + (g[1] - 1.9e-3) * (2.9 / 3.8)) + g[2:] for g in wl["groups"]]
+        order = rng.permutation(len(wl["groups"]))
+        wl["groups"] = [wl["groups"][i] for i in order]
+        return wl
+    wl = workloads.dense_pack(side=17, periodic=kind == "periodic",
+                              gravity=(0.0, 0.0, 0.0) if kind == "periodic" else (0.0, 0.0, -9.81))
+    order = rng.permutation(len(wl["x"]))
+    for k in ("radius", "density", "crust", "material", "x", "v", "w"):
+        wl[k] = np.asarray(wl[k])[order]
+    # unequal particles, so that a mixed-up array shows
+    wl["density"] = wl["density"] * rng.uniform(0.8, 1.2, len(order))
+    wl["radius"] = wl["radius"] * rng.uniform(0.9995, 1.0, len(order))
+    if kind == "memory":
+        wl["models"] = [("memory", 0, 0, 1e4, 0.8, 0.4, 2e3, -1.0, 0.02, 0.1, 1e-10)]
+    return wl
+
+
+@pytest.mark.parametrize("kind,skin", [("walls", None), ("walls", 0.0), ("periodic", None), ("memory", None),
+                                       ("polyhedra", None)])
+def test_random_order_against_oracle(gpu, kind, skin):
+    wl = shuffled(kind)
+    o = make_oracle(wl)
+    g = make_gpu(wl, skin=skin)
+    po = pair_set(o.pairs())
+    assert pair_set(g.pairs()) == po and len(po) > 20
+    scale = contact_scale(o.state(), o.masses()[2])
+    assert rel_force_error(g.state()["F"], o.state()["F"], scale) <= (1e-9 if kind == "memory" else 1e-12)
+    assert np.array_equal(g.masses()[0], o.masses()[0])
+    ft = np.random.default_rng(1).normal(size=(g.n, 6)) * 1e-9
+    o.step(12)
+    g.step(12)
+    so, sg = o.state(), g.state()
+    for k in ("x", "v", "w", "q"):
+        rms = np.sqrt(np.mean(so[k] ** 2))
+        # twelve steps of rounding, amplified by contacts that open and close
+        assert np.max(np.abs(sg[k] - so[k])) <= 1e-9 * max(rms, 1e-12), k
+    # rows of the fluid's forces reach their particles
+    g.compute_forces()
+    f0 = g.state()["F"]
+    g.set_hydro_ft(ft)
+    g.compute_forces()
+    assert np.max(np.abs(g.state()["F"] - f0 - ft[:, :3])) <= 1e-15 * np.max(np.abs(f0))
