@@ -617,7 +617,7 @@ __device__ __forceinline__ Kin load_kin(const Particles& P, int s, int cx, int c
 // ParticleKinematics::setAngularVelocity (ParticleKinematics.cpp:197-203).
 // Then the cell key is computed and the arrival slot reserved.
 __device__ __forceinline__ void wrap_and_bin(Kin& k, const Grid& G, const Sorted& S, DevStatus* st, int s, int pid,
-                                             int cell_base = 0, const VerletState* V = nullptr) {
+                                             int cell_base = 0, const VerletState* V = nullptr, int nx = 0, int stale = 0) {
   bool wrapped = false;
   double* xs[3] = {&k.x.x, &k.x.y, &k.x.z};
   int c[3];
@@ -645,7 +645,8 @@ __device__ __forceinline__ void wrap_and_bin(Kin& k, const Grid& G, const Sorted
   if (wrapped) k.wb = to_body(k.q, k.w);
   if (V && V->stamp) {
     // a Verlet list is in use: no binning here (stamp < 0: the list is
-    // rebuilt next, nothing to check); the list goes stale once the
+    // rebuilt next, nothing to check); the list goes stale (stale: what
+    // DevStatus::rebuild[nx] is then set to) once the
     // particle is more than half the skin from where it was built (nearest
     // periodic image, so that a role swap is no displacement)
     if (V->stamp < 0) return;
@@ -659,7 +660,7 @@ __device__ __forceinline__ void wrap_and_bin(Kin& k, const Grid& G, const Sorted
       }
       d2 += d * d;
     }
-    if (d2 > V->half2) st->rebuild = V->stamp;
+    if (d2 > V->half2) st->rebuild[nx] = stale;
     return;
   }
   int key = cell_base + (c[1] * G.n[2] + c[2]) * G.n[0] + c[0];  // LinkedCell::getCellNumber order
@@ -894,6 +895,43 @@ __device__ __forceinline__ void for_each_candidate(const Sorted& S, const Grid& 
   });
 }
 
+// Two spheres whose centres pass the conservative distance reject (AB = xo -
+// x_self, nab = Norm(AB)): true with the contact features (d may be >= 0);
+// false when there is none, or after a ContactError.
+__device__ __forceinline__ bool sphere_features(const Particles& P, DevStatus* st, const Self& me, int s2i, int pid2,
+                                                d3 xo, double ro, d3 AB, double nab, d3& Pc, d3& ov, double& d) {
+  const double co = P.crust[s2i];
+  const int res = sphere_sphere(me.x, me.r, me.c, AB, nab, ro, co, Pc, ov, d);
+  if (res < 0) {
+    if (!recover_ss(me.x, me.r, me.c, xo, ro, co, Pc, ov, d)) {
+      raise_error(st, kContactError, me.id, pid2);
+      return false;
+    }
+    atomicAdd(&st->n_recovered, 1);
+  }
+  return res != 0;
+}
+
+// The bounding-box test of a particle against an obstacle
+// (SimpleObstacle::InterAction, SimpleObstacle.cpp:222-271), and a sphere's
+// contact features with it, as sphere_features.
+__device__ __forceinline__ bool near_obstacle(const BoxObstacle& B, const d3& x, double r) {
+  return fabs(B.aabb_c[0] - x.x) <= B.aabb_e[0] + r && fabs(B.aabb_c[1] - x.y) <= B.aabb_e[1] + r &&
+         fabs(B.aabb_c[2] - x.z) <= B.aabb_e[2] + r;
+}
+__device__ __forceinline__ bool wall_features(const BoxObstacle& B, DevStatus* st, const Self& me, d3& Pc, d3& ov,
+                                              double& d) {
+  const int res = sphere_box(B, me.x, me.r, me.c, Pc, ov, d);
+  if (res < 0) {
+    if (!recover_sb(B, me.x, me.r, me.c, Pc, ov, d)) {
+      raise_error(st, kContactError, me.id, B.id);
+      return false;
+    }
+    atomicAdd(&st->n_recovered, 1);
+  }
+  return res != 0;
+}
+
 // Narrow phase of a neighbour candidate that passed the conservative
 // distance reject: particle s2i (storage index; sorted slot k2 when known,
 // id pid2, radius ro) seen at xo, AB = xo - x_self, nab = Norm(AB); for a
@@ -906,7 +944,6 @@ template <class V, bool SHAPES>
 __device__ __forceinline__ void narrow_visit(const Particles& P, const Grid& G, DevStatus* st, const Self& me,
                                              V& vis, const ConvexGeo* mg, int cx, int k2, int s2i, int pid2, d3 xo,
                                              double ro, d3 AB, double nab, const d3& xb, const int sh[3]) {
-  const double co = P.crust[s2i];
   d3 Pc, ov;
   double d;
   int nit = 1;
@@ -923,15 +960,7 @@ __device__ __forceinline__ void narrow_visit(const Particles& P, const Grid& G, 
       atomicAdd(&st->n_recovered, 1);
     }
   } else {
-    int res = sphere_sphere(me.x, me.r, me.c, AB, nab, ro, co, Pc, ov, d);
-    if (res == 0) return;
-    if (res < 0) {
-      if (!recover_ss(me.x, me.r, me.c, xo, ro, co, Pc, ov, d)) {
-        raise_error(st, kContactError, me.id, pid2);
-        return;
-      }
-      atomicAdd(&st->n_recovered, 1);
-    }
+    if (!sphere_features(P, st, me, s2i, pid2, xo, ro, AB, nab, Pc, ov, d)) return;
   }
   if (me.acc && me.id < pid2) me.acc->add(d, nit, image_evaluations(G, me.x, xb, sh));
   if (!(d < 0.)) return;
@@ -1006,10 +1035,7 @@ __device__ __forceinline__ void visit_obstacles(const BoxObstacle* __restrict__ 
                                                 const Self& me, V& vis, const ConvexGeo* mg) {
   for (int o = 0; o < nobs; ++o) {
     const BoxObstacle& B = obs[o];
-    bool probable = fabs(B.aabb_c[0] - me.x.x) <= B.aabb_e[0] + me.r &&
-                    fabs(B.aabb_c[1] - me.x.y) <= B.aabb_e[1] + me.r &&
-                    fabs(B.aabb_c[2] - me.x.z) <= B.aabb_e[2] + me.r;
-    if (!probable) continue;
+    if (!near_obstacle(B, me.x, me.r)) continue;
     d3 Pc, ov;
     double d;
     int nit = 1;
@@ -1025,15 +1051,7 @@ __device__ __forceinline__ void visit_obstacles(const BoxObstacle* __restrict__ 
         atomicAdd(&st->n_recovered, 1);
       }
     } else {
-      int res = sphere_box(B, me.x, me.r, me.c, Pc, ov, d);
-      if (res == 0) continue;
-      if (res < 0) {
-        if (!recover_sb(B, me.x, me.r, me.c, Pc, ov, d)) {
-          raise_error(st, kContactError, me.id, B.id);
-          continue;
-        }
-        atomicAdd(&st->n_recovered, 1);
-      }
+      if (!wall_features(B, st, me, Pc, ov, d)) continue;
     }
     if (me.acc) me.acc->add(d, nit, 1);
     if (!(d < 0.)) continue;
@@ -1303,6 +1321,33 @@ __device__ __forceinline__ void sweep_particle(const Particles& P, const Sorted&
     sp.mem.n[sp.mem.cur ^ 1][s] = min(vis.nmem, sp.mem.cap);
     if (vis.nmem > sp.mem.cap) raise_error(st, kMemoryOverflow, me.id, vis.nmem);
   }
+}
+
+// The particle in arrival place j of the sorted order: its rank by id among
+// the particles of its cell gives its sorted slot (deterministic, and
+// independent of the atomic arrival order); writes order / sid / inv / posr
+// there.  One thread per particle: a thread per cell, which sorted the cell's
+// particles one after the other, waited for their loads in turn.
+__device__ __forceinline__ void rank_particle(const Particles& P, const Sorted& S, int j, int cx, int n) {
+  // indices are out of range only after an interrupted binning
+  int s = S.tmp_order[j];
+  if ((unsigned)s >= (unsigned)n) s = 0;
+  const int key = S.key[s], id = P.id[s];
+  const int b = min(max(S.start[key], 0), n), e = min(S.start[key + 1], n);
+  int rank = 0;
+  for (int i = b; i < e; ++i) {
+    const int o = S.tmp_order[i];
+    rank += (unsigned)o < (unsigned)n && P.id[o] < id;
+  }
+  const int k = min(b + rank, n - 1);
+  S.order[k] = s;
+  S.sid[k] = id;
+  if (S.inv) S.inv[s] = k;
+  double* pr = S.posr + 4 * (size_t)k;
+  pr[0] = P.x[cx][0][s];
+  pr[1] = P.x[cx][1][s];
+  pr[2] = P.x[cx][2][s];
+  pr[3] = P.rad[s];
 }
 
 // Orders the particles of one cell (sorted slots [b, e)) by id, writes

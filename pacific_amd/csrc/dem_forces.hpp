@@ -11,6 +11,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dem_device.hpp"
 
 namespace dem {
@@ -54,7 +56,7 @@ __device__ __forceinline__ void sphere_tail(const Particles& P, const Sorted& S,
     }
   }
   if (depl > crust) raise_error(st, kMotionError, id, 0);
-  wrap_and_bin(kin, G, S, st, s, id, 0, &VS);
+  wrap_and_bin(kin, G, S, st, s, id, 0, &VS, cx ^ 1, VS.stamp > 0 ? st->seq[cx] + 2 : 0);
   st3(P.x[cx ^ 1], s, kin.x);
   st3(P.v[nv], s, kin.v);
   st3(P.w[nv], s, kin.w);
@@ -202,6 +204,15 @@ __device__ __forceinline__ void force_one(const Particles& P, const Sorted& S, c
   sphere_tail<MODE>(P, S, G, sp, st, VS, s, cx, cv, kin, me.m, me.c, me.id, cf, I, F, T);
 }
 
+// The number of the positions a fused sweep writes (DevStatus::seq), and the
+// counters of a rebuild for them.
+__device__ __forceinline__ void number_next(const StepParams& sp, DevStatus* st, const VerletState& VS) {
+  if (blockIdx.x != 0) return;
+  const int nx = (sp.cur & 1) ^ 1;
+  if (threadIdx.x == 0) st->seq[nx] = st->seq[nx ^ 1] + 1;
+  if (VS.sync && threadIdx.x < sizeof(RebuildSync) / sizeof(int)) ((int*)(VS.sync + nx))[threadIdx.x] = 0;
+}
+
 // Per-block sums of the contact statistics (sum and max of the overlaps,
 // their count, GJK iterations and evaluations), in a fixed order.
 // (ADD: combined with the sums already in out, written by an earlier launch
@@ -245,6 +256,7 @@ __global__ __launch_bounds__(256) void k_forces(Particles P, Sorted S, Grid G, c
                                                 const HookeModel* __restrict__ models, StepParams sp, DevStatus* st,
                                                 int* pairs, NbrList L, VerletState VS, NbrList CL) {
   const int t = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  if (MODE == kFused && VS.stamp > 0) number_next(sp, st, VS);
   if (!EXTRAS) {
     if (t < sp.n) force_one<MODE, MIXED, SHAPES, false>(P, S, G, obs, models, sp, st, pairs, L, VS, CL, t, nullptr);
     return;
@@ -268,6 +280,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     Particles P, Sorted S, Grid G, const BoxObstacle* __restrict__ obs, const HookeModel* __restrict__ models,
     StepParams sp, DevStatus* st, int* pairs, NbrList L, VerletState VS, NbrList CL) {
   const int t = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  if (MODE == kFused && VS.stamp > 0) number_next(sp, st, VS);
   if (t < sp.n) force_one<MODE, false, false, false>(P, S, G, obs, models, sp, st, pairs, L, VS, CL, t, nullptr);
 }
 

@@ -9,20 +9,21 @@ namespace dem {
 enum ForceMode { kModeForcesOnly = 0, kModeForcesKick = 1, kModeFused = 2 };
 
 // first half kick + drift (or a full Move of the explicit schemes) in place,
-// then cell key and arrival slot
+// then cell key and arrival slot; number: the number of the positions written
+// (DevStatus::seq)
 hipError_t launch_move(const Particles& P, const Sorted& S, const Grid& G, const StepParams& sp, DevStatus* st,
-                       double dtv, double dtx, const VerletState& V, hipStream_t stream);
+                       double dtv, double dtx, const VerletState& V, int number, hipStream_t stream);
 // cell key and arrival slot of the current positions (no motion)
 hipError_t launch_key(const Particles& P, const Sorted& S, const Grid& G, const StepParams& sp, DevStatus* st,
                       const VerletState& V, hipStream_t stream);
 // counts -> start, scatter, per-cell ordering; cx = position buffer to gather;
-// with gate, only when *gate == stamp
+// with gate, only when *gate == *seq + 1
 hipError_t launch_bin(const Particles& P, const Sorted& S, const Grid& G, int n, int cx, hipStream_t stream,
-                      const int* gate = nullptr, int stamp = 0);
-// Verlet list build (keys on its grid, binning, candidates); stamp > 0: only
-// if the list was found stale (DevStatus::rebuild == stamp)
+                      const int* gate = nullptr, const int* seq = nullptr);
+// Verlet list build (keys on its grid, binning, candidates) from position
+// buffer cx; gated: only if the drift that wrote it found the list stale
 hipError_t launch_verlet_build(const Particles& P, const Sorted& S, const VerletState& V, int n, int cx,
-                               DevStatus* st, const NbrList& L, int stamp, hipStream_t stream);
+                               DevStatus* st, const NbrList& L, bool gated, hipStream_t stream);
 int scan_blocks(int ncells);
 // zero n ints with a kernel (safe inside captured graphs, unlike hipMemsetAsync)
 hipError_t launch_clear(int* p, int n, hipStream_t stream);
@@ -43,6 +44,11 @@ constexpr int kDetectBodies = 32;
 // into sp.cf, and the contact statistics when sp.stats is set
 hipError_t launch_narrow(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
                          const StepParams& sp, DevStatus* st, const NbrList& L, hipStream_t stream);
+// force sweep of a small system of spheres with a Verlet list, which it
+// rebuilds itself when it is stale (k_forces_solo)
+hipError_t launch_forces_solo(int mode, bool mixed, const Particles& P, const Sorted& S, const Grid& G,
+                              const BoxObstacle* obs, const HookeModel* models, const StepParams& sp, DevStatus* st,
+                              int* pairs, const NbrList& L, const VerletState& V, hipStream_t stream);
 // force sweep over the candidates of L (L.count == nullptr: 27-cell sweep)
 hipError_t launch_forces(int mode, bool mixed, const Particles& P, const Sorted& S, const Grid& G,
                          const BoxObstacle* obs, const HookeModel* models, const StepParams& sp, DevStatus* st,

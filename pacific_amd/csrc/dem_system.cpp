@@ -138,6 +138,12 @@ int grains_gpu_system::allocate() {
   HIPCHECK(this, hipHostMalloc((void**)&h_status, sizeof(DevStatus), hipHostMallocDefault));
   if (verlet)
     for (int a = 0; a < 3; ++a) HIPCHECK(this, track(this, &V.xb[a], n));
+  V.sync = nullptr;
+  solo = verlet && n > 0 && n <= (size_t)kSoloMax && nbr_cap <= 64 && obstacles.size() <= 64;
+  if (solo) {
+    HIPCHECK(this, track(this, &V.sync, 2));
+    HIPCHECK(this, hipMemsetAsync(V.sync, 0, 2 * sizeof(RebuildSync), stream));
+  }
   mem = dem::ContactMemory{};
   if (has_memory() && n > 0) {
     const size_t m = (size_t)kMemoryCap * n;
@@ -190,7 +196,7 @@ int grains_gpu_system::allocate() {
   } else {
     d_nbr_count = nullptr;
     d_nbr = nullptr;
-    verlet = false;
+    verlet = solo = false;
   }
   pair_cap = (int)std::min<size_t>(16 * n + 4096, (size_t)1 << 28);
   HIPCHECK(this, track(this, &d_pairs, 2 * (size_t)pair_cap));
@@ -358,7 +364,7 @@ int grains_gpu_system::bin_current() {
   if (verlet) {
     // periodic wrap of the current positions, then a Verlet list build
     HIPCHECK(this, launch_key(P, S, grid, sp, d_status, vstate(-1), stream));
-    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), 0, stream));
+    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), false, stream));
     return GRAINS_OK;
   }
   HIPCHECK(this, launch_key(P, S, grid, sp, d_status, vstate(0), stream));
@@ -428,8 +434,10 @@ int grains_gpu_system::mark(std::vector<hipEvent_t>& evs, size_t& n) {
 int grains_gpu_system::bin_launch() {
   int e;
   if (prof && (e = mark(prof->bin_ev, prof->nbin))) return e;
-  if (verlet)
-    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), kStale, stream));
+  if (solo)
+    ;  // the force sweep rebuilds the list itself
+  else if (verlet)
+    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), true, stream));
   else
     HIPCHECK(this, launch_bin(P, S, grid, nparticles, cur & 1, stream));
   if (prof && (e = mark(prof->bin_ev, prof->nbin))) return e;
@@ -462,6 +470,22 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     HIPCHECK(this, launch_narrow(P, S, grid, d_obs, sp, d_status, L, stream));
     if (prof && (e = mark(prof->narrow_ev, prof->nnarrow))) return e;
   }
+  if (solo && !sp.stats && !sp.fsum) {
+    // one launch: list rebuild if stale, contacts, forces, integration
+    if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
+    HIPCHECK(this, launch_forces_solo(mode, cfg.precision == GRAINS_MIXED, P, S, grid, d_obs, d_models, sp, d_status,
+                                      d_pairs, L, vstate(1), stream));
+    if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
+    if (commit && mem.cap) mem.cur ^= 1;
+    if (mode == kModeForcesKick) cur ^= 2;
+    if (mode == kModeFused) {
+      cur ^= 3;
+      ++step_number;
+    }
+    return GRAINS_OK;
+  }
+  if (solo)  // an evaluation of the general sweep: the list must be current
+    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, L, true, stream));
   const dem::NbrList CL = contact_list();
   if (CL.count) {
     // this step's contacts from the Verlet list
@@ -471,13 +495,16 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
   }
   if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
   HIPCHECK(this, launch_forces(mode, cfg.precision == GRAINS_MIXED, P, S, grid, d_obs, d_models, sp, d_status,
-                               d_pairs, L, vstate(next_stamp()), CL, stream));
+                               d_pairs, L, vstate(1), CL, stream));
   if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
   if (sp.stats) HIPCHECK(this, launch_stats_fold(d_stat_part, nparticles, d_stat_tot, force_time, stream));
   // the evaluation wrote the other memory buffer: it becomes current
   if (commit && mem.cap) mem.cur ^= 1;
   if (mode == kModeForcesKick) cur ^= 2;
-  if (mode == kModeFused) cur ^= 3;
+  if (mode == kModeFused) {
+    cur ^= 3;
+    ++step_number;
+  }
   return GRAINS_OK;
 }
 
@@ -509,7 +536,8 @@ int grains_gpu_system::enqueue_steps_impl(int nsteps) {
     // forces of step j are evaluated at the time the step reaches (the
     // reference adds dt to m_time before them, Grains.cpp:290)
     force_time = time;
-    HIPCHECK(this, launch_move(P, S, grid, sp, d_status, 0.5 * cfg.dt, cfg.dt, vstate(next_stamp()), stream));
+    HIPCHECK(this, launch_move(P, S, grid, sp, d_status, 0.5 * cfg.dt, cfg.dt, vstate(1), ++step_number,
+                               stream));
     if ((e = bin_launch())) return e;
     if (recording && (e = record_state())) return e;
     int i = 1;
@@ -576,12 +604,13 @@ int grains_gpu_system::graph_chunk(bool& done) {
   for (auto& g : graphs)
     if (g.first == key) {
       for (int j = 0; j < kGraphSteps; ++j) force_time += cfg.dt;
+      step_number += kGraphSteps;
       HIPCHECK(this, hipGraphLaunch(g.second, stream));
       ++graph_replays;
       done = true;
       return GRAINS_OK;
     }
-  const int cur0 = cur, mem0 = mem.cur;
+  const int cur0 = cur, mem0 = mem.cur, number0 = step_number;
   const double ft0 = force_time;
   HIPCHECK(this, hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
   int e = GRAINS_OK;
@@ -602,6 +631,7 @@ int grains_gpu_system::graph_chunk(bool& done) {
     // captured launches never ran: back to the state before the capture
     cur = cur0;
     mem.cur = mem0;
+    step_number = number0;
     force_time = ft0;
     graphs_failed = true;
     (void)hipGetLastError();

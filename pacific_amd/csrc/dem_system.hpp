@@ -131,12 +131,15 @@ struct grains_gpu_system {
   double* d_stat_part = nullptr;
   double* d_stat_tot = nullptr;
   double force_time = 0.;
-  // stale flag of the Verlet list: set by the drift that finds the list
-  // stale, read by the rebuild launches, cleared by the next contact filter
-  // (the same kernel arguments every step, so that steps can be replayed
-  // from a captured graph)
-  static constexpr int kStale = 1;
-  int next_stamp() const { return kStale; }
+  // systems whose force sweep also rebuilds the Verlet list and finds the
+  // contacts in it, one launch per step (k_forces_solo: faster up to this many
+  // spheres in beds and gases alike, figures there); its masks hold 64 listed
+  // neighbours and 64 obstacles
+  static constexpr int kSoloMax = 65536;
+  bool solo = false;
+  // the number of the last positions written (DevStatus::seq counts along on
+  // the device, so that captured steps need no new arguments)
+  int step_number = 0;
   dem::VerletState vstate(int st) const {
     dem::VerletState v = V;
     v.stamp = verlet ? st : 0;

@@ -147,6 +147,15 @@ struct NbrList {
   int cap, n;
 };
 
+// Progress of a list rebuild inside a force sweep (k_forces_solo): the next
+// piece of work and how many pieces of each phase are done.  One set per
+// position buffer; the sweep of the other buffer clears it.
+struct RebuildSync {
+  int ticket;
+  int done[6];
+  int pad[9];
+};
+
 // Verlet neighbour list: every pair closer than the contact distance plus
 // a skin at the last build, kept until some particle has moved more than
 // half the skin since then (each contact of the meantime is then a listed
@@ -159,8 +168,9 @@ struct VerletState {
   double* xb[3];  // positions at the last build (storage order)
   double skin;
   double half2;   // (skin / 2)^2
-  int stamp;      // > 0: the staleness check sets DevStatus::rebuild = stamp; 0 = no Verlet list; < 0 wrap only
+  int stamp;      // > 0: the staleness check is on; 0 = no Verlet list; < 0 wrap only
   int pad;
+  RebuildSync* sync;  // [2], of a system whose force sweep rebuilds the list itself
 };
 
 // Device-side error / statistics block (one per system)
@@ -173,7 +183,13 @@ struct DevStatus {
   int n_recovered;   // ContactError recoveries
   int pad;
   double overlap_max;
-  int rebuild;       // Verlet list found stale (the drift's stamp), cleared by the contact filter
+  // The steps of a run are numbered, seq[b] holding the number of the
+  // positions in buffer b.  A drift to buffer b that finds the Verlet list
+  // stale sets rebuild[b] to one more than the number of the positions it
+  // writes, so that later steps, with other numbers, need not have it cleared,
+  // and the launch that reads one of the pair writes the other.
+  int rebuild[2];
+  int seq[2];
   int n_rebuild;     // Verlet list builds
 };
 
