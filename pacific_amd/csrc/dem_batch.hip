@@ -104,6 +104,7 @@ __device__ __forceinline__ StepParams batch_params(const BatchSys& B, int hi) {
   sp.stats = nullptr;
   sp.mem = ContactMemory{};
   sp.cf = ContactFeat{};
+  sp.crust_all = sp.cfac_all = -1.;
   sp.fsum = nullptr;
   sp.hyd = nullptr;
   return sp;
@@ -137,6 +138,7 @@ __global__ __launch_bounds__(512) void k_batch(const BatchSys* __restrict__ sys,
   sp.stats = nullptr;
   sp.mem = ContactMemory{};
   sp.cf = ContactFeat{};
+  sp.crust_all = sp.cfac_all = -1.;
   sp.fsum = nullptr;
   sp.hyd = nullptr;
   const BoxObstacle* bobs = obs + B.o0;
@@ -151,7 +153,7 @@ __global__ __launch_bounds__(512) void k_batch(const BatchSys* __restrict__ sys,
         double depl = lf_move(k, ld3(P.F, s), ld3(P.T, s), P.mass[s], P.cfac[s], P.inertia[s], 0.5 * B.dt, B.dt);
         if (depl > P.crust[s]) raise_error(st, kMotionError, pid, 0);
       }
-      wrap_and_bin(k, B.grid, S, st, s, pid, B.c0);
+      wrap_and_bin(k, B.grid, S, st, s, P.id, B.c0);
       st3(P.x[0], s, k.x);
       st3(P.v[0], s, k.v);
       st3(P.w[0], s, k.w);
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(256) void k_fb_move(const BatchSys* __restrict__ sy
     const double depl = lf_move(k, ld3(P.F, s), ld3(P.T, s), P.mass[s], P.cfac[s], P.inertia[s], 0.5 * B.dt, B.dt);
     if (depl > P.crust[s]) raise_error(st, kMotionError, pid, 0);
   }
-  wrap_and_bin(k, B.grid, S, st, s, pid, B.c0);
+  wrap_and_bin(k, B.grid, S, st, s, P.id, B.c0);
   st3(P.x[0], s, k.x);
   st3(P.v[0], s, k.v);
   st3(P.w[0], s, k.w);
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   if (MODE == 2) {
     const double depl = lf_move(kin, F, T, me.m, cf, I, 0.5 * B.dt, B.dt);
     if (depl > me.c) raise_error(st, kMotionError, me.id, 0);
-    wrap_and_bin(kin, B.grid, S, st, s, me.id, B.c0);
+    wrap_and_bin(kin, B.grid, S, st, s, P.id, B.c0);
     st3(P.x[0], s, kin.x);
     P.q[0][s] = kin.q.v.x;
     P.q[1][s] = kin.q.v.y;

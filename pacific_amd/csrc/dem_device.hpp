@@ -616,7 +616,9 @@ __device__ __forceinline__ Kin load_kin(const Particles& P, int s, int cx, int c
 // the clone's body-fixed angular velocity is rebuilt from w and q by
 // ParticleKinematics::setAngularVelocity (ParticleKinematics.cpp:197-203).
 // Then the cell key is computed and the arrival slot reserved.
-__device__ __forceinline__ void wrap_and_bin(Kin& k, const Grid& G, const Sorted& S, DevStatus* st, int s, int pid,
+// (ids: by storage index, read on an error)
+__device__ __forceinline__ void wrap_and_bin(Kin& k, const Grid& G, const Sorted& S, DevStatus* st, int s,
+                                             const int* __restrict__ ids,
                                              int cell_base = 0, const VerletState* V = nullptr, int nx = 0, int stale = 0) {
   bool wrapped = false;
   double* xs[3] = {&k.x.x, &k.x.y, &k.x.z};
@@ -637,7 +639,7 @@ __device__ __forceinline__ void wrap_and_bin(Kin& k, const Grid& G, const Sorted
     }
     int gi = ri - G.off[a];
     if (gi < 0 || gi >= G.n[a]) {
-      raise_error(st, kSimulationError, pid, 0);
+      raise_error(st, kSimulationError, ids[s], 0);
       gi = gi < 0 ? 0 : G.n[a] - 1;
     }
     c[a] = gi;

@@ -24,7 +24,7 @@ enum { kForcesOnly = 0, kForcesKick = 1, kFused = 2 };
 template <int MODE>
 __device__ __forceinline__ void sphere_tail(const Particles& P, const Sorted& S, const Grid& G, const StepParams& sp,
                                             DevStatus* st, const VerletState& VS, int s, int cx, int cv, Kin& kin,
-                                            double mass, double crust, int id, double cf, double I, const d3& F,
+                                            double mass, double crust, double cf, double I, const d3& F,
                                             const d3& T) {
   const int nv = cv ^ 1;
   if (MODE == kForcesKick) {
@@ -55,8 +55,8 @@ __device__ __forceinline__ void sphere_tail(const Particles& P, const Sorted& S,
       st3(P.dWdt_nm2, s, ab.dWdt_nm2);
     }
   }
-  if (depl > crust) raise_error(st, kMotionError, id, 0);
-  wrap_and_bin(kin, G, S, st, s, id, 0, &VS, cx ^ 1, VS.stamp > 0 ? st->seq[cx] + 2 : 0);
+  if (depl > crust) raise_error(st, kMotionError, P.id[s], 0);
+  wrap_and_bin(kin, G, S, st, s, P.id, 0, &VS, cx ^ 1, VS.stamp > 0 ? st->seq[cx] + 2 : 0);
   st3(P.x[cx ^ 1], s, kin.x);
   st3(P.v[nv], s, kin.v);
   st3(P.w[nv], s, kin.w);
@@ -188,7 +188,7 @@ __device__ __forceinline__ void force_one(const Particles& P, const Sorted& S, c
     if (MODE == kFused) {
       double depl = lf_move_body(kin, gyro, F, T, me.m, cf, I, I3, 0.5 * sp.dt, sp.dt, B);
       if (depl > me.c) raise_error(st, kMotionError, me.id, 0);
-      wrap_and_bin(kin, G, S, st, s, me.id, 0, &VS);
+      wrap_and_bin(kin, G, S, st, s, P.id, 0, &VS);
       st3(P.x[cx ^ 1], s, kin.x);
       for (int j = 0; j < 9; ++j) P.B[cx ^ 1][j][s] = B[j];
       P.q[0][s] = kin.q.v.x;
@@ -201,7 +201,7 @@ __device__ __forceinline__ void force_one(const Particles& P, const Sorted& S, c
     st3(P.wb, s, kin.wb);
     return;
   }
-  sphere_tail<MODE>(P, S, G, sp, st, VS, s, cx, cv, kin, me.m, me.c, me.id, cf, I, F, T);
+  sphere_tail<MODE>(P, S, G, sp, st, VS, s, cx, cv, kin, me.m, me.c, cf, I, F, T);
 }
 
 // The number of the positions a fused sweep writes (DevStatus::seq), and the
@@ -211,6 +211,111 @@ __device__ __forceinline__ void number_next(const StepParams& sp, DevStatus* st,
   const int nx = (sp.cur & 1) ^ 1;
   if (threadIdx.x == 0) st->seq[nx] = st->seq[nx ^ 1] + 1;
   if (VS.sync && threadIdx.x < sizeof(RebuildSync) / sizeof(int)) ((int*)(VS.sync + nx))[threadIdx.x] = 0;
+}
+
+// One sphere of a system with a Verlet list and this step's contacts (no
+// extras): force_one with every load that the integration needs issued first,
+// and what only a contact needs (spin, radius, material, ...) read only for
+// particles that may have one.  A contact-free particle-step moves 276 B
+// instead of 348.
+template <int MODE, bool MIXED>
+__device__ __forceinline__ void force_verlet(const Particles& P, const Sorted& S, const Grid& G,
+                                             const BoxObstacle* __restrict__ obs, const HookeModel* __restrict__ models,
+                                             const StepParams& sp, DevStatus* st, int* pairs, const NbrList& L,
+                                             const VerletState& VS, const NbrList& CL, int s, bool touched) {
+  const int cx = sp.cur & 1, cv = (sp.cur >> 1) & 1;
+  Kin kin;
+  kin.x = ld3(P.x[cx], s);
+  kin.v = ld3(P.v[cv], s);
+  kin.wb = ld3(P.wb, s);
+  kin.q = quat{d3{P.q[0][s], P.q[1][s], P.q[2][s]}, P.q[3][s]};
+  const double mass = P.mass[s], I = P.inertia[s];
+  // InitializeForce: torsor = weight at the centre (Particle.cpp:1408-1415)
+  d3 F{0., 0., 0.}, T{0., 0., 0.};
+  if (sp.g[0] != 0. || sp.g[1] != 0. || sp.g[2] != 0.) {
+    const double wf = P.wfac[s];
+    F = d3{sp.g[0] * wf, sp.g[1] * wf, sp.g[2] * wf};
+  }
+  if (touched) {
+    Self me;
+    me.x = kin.x;
+    me.v = kin.v;
+    me.w = ld3(P.w[cv], s);
+    me.r = P.rad[s];
+    me.m = P.mass[s];
+    me.c = P.crust[s];
+    me.req = P.req[s];
+    me.mat = P.mat[s];
+    me.id = P.id[s];
+    sweep_particle<MIXED, false, false>(P, S, G, obs, sp.nobs, models, sp, st, pairs, 0, 0, sp.n, cv, 0, me, F, T,
+                                        nullptr, cx, &L, &VS, s, &CL);
+  }
+  // forces of the fluid (AppPRSHydroFT::ComputeForces, AppPRSHydroFT.cpp:
+  // 27-44): an application after the contacts, the force at the centre
+  if (sp.hyd) {
+    const size_t n = (size_t)sp.n;
+    F += d3{sp.hyd[s], sp.hyd[n + s], sp.hyd[2 * n + s]};
+    T += d3{sp.hyd[3 * n + s], sp.hyd[4 * n + s], sp.hyd[5 * n + s]};
+  }
+  if (!(MODE == kFused && sp.scheme == kLeapFrog)) {
+    st3(P.F, s, F);
+    st3(P.T, s, T);
+  }
+  sphere_tail<MODE>(P, S, G, sp, st, VS, s, cx, cv, kin, mass, sp.crust_all >= 0. ? sp.crust_all : P.crust[s],
+                    sp.cfac_all >= 0. ? sp.cfac_all : P.cfac[s], I, F, T);
+}
+
+template <int MODE, bool MIXED>
+__device__ __forceinline__ void forces_verlet(const Particles& P, const Sorted& S, const Grid& G,
+                                              const BoxObstacle* __restrict__ obs,
+                                              const HookeModel* __restrict__ models, const StepParams& sp,
+                                              DevStatus* st, int* pairs, const NbrList& L, const VerletState& VS,
+                                              const NbrList& CL) {
+  const int s = xcd_tile(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
+  if (MODE == kFused) number_next(sp, st, VS);
+  if (s < sp.n)
+    force_verlet<MODE, MIXED>(P, S, G, obs, models, sp, st, pairs, L, VS, CL, s, CL.count[s] != 0 || sp.nobs != 0);
+}
+
+// FP64 takes what registers it needs (2 waves per SIMD): with 3 it spills
+// (bed of 200,000: 59 us -> 66; 1M gas 88 -> 118).  FP32 arithmetic fits in
+// three (1M gas: 89 us -> 78).
+template <int MODE>
+__global__ __launch_bounds__(64) void k_verlet64(Particles P, Sorted S, Grid G, const BoxObstacle* __restrict__ obs,
+                                                 const HookeModel* __restrict__ models, StepParams sp, DevStatus* st,
+                                                 int* pairs, NbrList L, VerletState VS, NbrList CL) {
+  forces_verlet<MODE, false>(P, S, G, obs, models, sp, st, pairs, L, VS, CL);
+}
+template <int MODE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_verlet32(
+    Particles P, Sorted S, Grid G, const BoxObstacle* __restrict__ obs, const HookeModel* __restrict__ models,
+    StepParams sp, DevStatus* st, int* pairs, NbrList L, VerletState VS, NbrList CL) {
+  forces_verlet<MODE, true>(P, S, G, obs, models, sp, st, pairs, L, VS, CL);
+}
+
+// The same for a gas (a system that keeps a touch list), where one particle in
+// a hundred has a contact: the first `tblocks` workgroups take those from the
+// list, 64 to a wave, and the others stream through the rest, so that no wave
+// waits for a single contact.  Three waves per SIMD: the sweep spills, but few
+// waves run it, and the streaming part, bound by memory, has the waves that it
+// needs.  1M gas, FP64: 91.7 us -> 78.9 per launch, of which 60 are the
+// streaming, 276 MB (4.6 TB/s).  FP32 arithmetic has three waves as it is.
+template <int MODE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_forces_gas(
+    Particles P, Sorted S, Grid G, const HookeModel* __restrict__ models, StepParams sp, DevStatus* st, int* pairs,
+    NbrList L, VerletState VS, NbrList CL, TouchList TL, int tblocks) {
+  if (MODE == kFused) number_next(sp, st, VS);
+  if ((int)blockIdx.x < tblocks) {
+    const int list = blockIdx.x & (kTouchLists - 1);
+    const int total = TL.count[list * kItemPad];
+    const int* idx = TL.idx + (size_t)list * TL.stride;
+    for (int i = (blockIdx.x / kTouchLists) * 64 + threadIdx.x; i < total; i += (tblocks / kTouchLists) * 64)
+      force_verlet<MODE, false>(P, S, G, nullptr, models, sp, st, pairs, L, VS, CL, idx[i], true);
+    return;
+  }
+  const int s = xcd_tile(blockIdx.x - tblocks, gridDim.x - tblocks) * 64 + threadIdx.x;
+  if (s < sp.n && CL.count[s] == 0)
+    force_verlet<MODE, false>(P, S, G, nullptr, models, sp, st, pairs, L, VS, CL, s, false);
 }
 
 // Per-block sums of the contact statistics (sum and max of the overlaps,
@@ -286,6 +391,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 
 
 constexpr int kSphereBlock = 64;
+constexpr int kTouchWaves = 4096;  // waves for the particles of a touch list, at most
 static inline int nblk_f(int n, int b) { return (n + b - 1) / b; }
 
 // Launchers of the force sweep, one explicit instantiation per translation
@@ -294,7 +400,7 @@ static inline int nblk_f(int n, int b) { return (n + b - 1) / b; }
 template <int MODE, bool MIXED>
 void launch_forces_sph(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
                        const HookeModel* models, const StepParams& sp, DevStatus* st, int* pairs, const NbrList& L,
-                       const VerletState& V, const NbrList& CL, hipStream_t stream);
+                       const VerletState& V, const NbrList& CL, const TouchList& TL, hipStream_t stream);
 template <int MODE, bool MIXED>
 void launch_forces_shp(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
                        const HookeModel* models, const StepParams& sp, DevStatus* st, int* pairs, const NbrList& L,

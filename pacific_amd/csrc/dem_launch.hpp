@@ -23,13 +23,14 @@ hipError_t launch_bin(const Particles& P, const Sorted& S, const Grid& G, int n,
 // Verlet list build (keys on its grid, binning, candidates) from position
 // buffer cx; gated: only if the drift that wrote it found the list stale
 hipError_t launch_verlet_build(const Particles& P, const Sorted& S, const VerletState& V, int n, int cx,
-                               DevStatus* st, const NbrList& L, bool gated, hipStream_t stream);
+                               DevStatus* st, const NbrList& L, int* tcount, bool gated, hipStream_t stream);
 int scan_blocks(int ncells);
 // zero n ints with a kernel (safe inside captured graphs, unlike hipMemsetAsync)
 hipError_t launch_clear(int* p, int n, hipStream_t stream);
-// contacts of this step from the Verlet list L into CL
+// contacts of this step from the Verlet list L into CL, and the particles that
+// have one into TL (if kept)
 hipError_t launch_vfilter(const Particles& P, const Sorted& S, const Grid& G, const VerletState& V, int n, int cx,
-                          const NbrList& L, const NbrList& CL, DevStatus* st, hipStream_t stream);
+                          const NbrList& L, const NbrList& CL, const TouchList& TL, DevStatus* st, hipStream_t stream);
 // folds the per-block contact statistics of the last force launch over n
 // particles into the running totals (6 doubles), at the given time
 hipError_t launch_stats_fold(const double* part, int n, double* tot, double time, hipStream_t stream);
@@ -53,6 +54,6 @@ hipError_t launch_forces_solo(int mode, bool mixed, const Particles& P, const So
 hipError_t launch_forces(int mode, bool mixed, const Particles& P, const Sorted& S, const Grid& G,
                          const BoxObstacle* obs, const HookeModel* models, const StepParams& sp, DevStatus* st,
                          int* pairs, const NbrList& L, const VerletState& V, const NbrList& CL,
-                         hipStream_t stream);
+                         const TouchList& TL, hipStream_t stream);
 
 }  // namespace dem

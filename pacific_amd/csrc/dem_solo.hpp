@@ -393,12 +393,11 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
     F += d3{(double)Fc.x, (double)Fc.y, (double)Fc.z};
     Tq += d3{(double)Tc.x, (double)Tc.y, (double)Tc.z};
   }
-  const int id = P.id[s];
   if (MEM && sp.mem.cap) {
     // this evaluation's contact memory of the particle (every particle, so
     // that entries of contacts that ended are dropped)
     sp.mem.n[sp.mem.cur ^ 1][s] = min(rank0[tid], sp.mem.cap);
-    if (rank0[tid] > sp.mem.cap) raise_error(st, kMemoryOverflow, id, rank0[tid]);
+    if (rank0[tid] > sp.mem.cap) raise_error(st, kMemoryOverflow, P.id[s], rank0[tid]);
   }
   // forces of the fluid (AppPRSHydroFT::ComputeForces, AppPRSHydroFT.cpp:
   // 27-44): an application after the contacts, the force at the centre
@@ -418,7 +417,7 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
   kin.w = d3{self[6][tid], self[7][tid], self[8][tid]};
   kin.wb = ld3(P.wb, s);
   kin.q = quat{d3{P.q[0][s], P.q[1][s], P.q[2][s]}, P.q[3][s]};
-  sphere_tail<MODE>(P, S, G, sp, st, VS, s, cx, cv, kin, self[10][tid], P.crust[s], id, P.cfac[s], P.inertia[s], F, Tq);
+  sphere_tail<MODE>(P, S, G, sp, st, VS, s, cx, cv, kin, self[10][tid], P.crust[s], P.cfac[s], P.inertia[s], F, Tq);
 }
 
 template <bool MIXED>

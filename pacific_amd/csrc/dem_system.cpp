@@ -185,6 +185,21 @@ int grains_gpu_system::allocate() {
   HIPCHECK(this, track(this, &d_stat_part, 5 * ((n + 255) / 256) + 5));
   HIPCHECK(this, track(this, &d_stat_tot, 8));
   HIPCHECK(this, hipMemsetAsync(d_stat_tot, 0, 8 * sizeof(double), stream));
+  // a touch list where nothing holds the particles together, neither weight
+  // nor walls, so that contacts are collisions and few, and where the state no
+  // longer fits the 256 MB cache, so that the sweep waits for memory and the
+  // wave of a contact holds up the others (us per step without and with it:
+  // gas of 110,000 32 and 41, of 400,000 63.5 and 64.8, of 600,000 87 and 81, of
+  // 1M 142 and 132; a settled bed of 200,000 80 and 95)
+  touch = dem::TouchList{};
+  const bool gas = cfg.gravity[0] == 0. && cfg.gravity[1] == 0. && cfg.gravity[2] == 0. && obstacles.empty();
+  if (verlet && gas && n > (size_t)kTouchMin && cfg.precision != GRAINS_MIXED) {
+    const size_t blocks = (n + 255) / 256;
+    touch.stride = (int)((blocks + kTouchLists - 1) / kTouchLists * 256);
+    HIPCHECK(this, track(this, &touch.idx, (size_t)kTouchLists * touch.stride));
+    HIPCHECK(this, track(this, &touch.count, (size_t)kTouchLists * kItemPad));
+    HIPCHECK(this, hipMemsetAsync(touch.count, 0, sizeof(int) * kTouchLists * kItemPad, stream));
+  }
   if (verlet) {
     HIPCHECK(this, track(this, &d_ct_count, n));
     HIPCHECK(this, track(this, &d_ct, (size_t)kContactCap * n));
@@ -197,6 +212,7 @@ int grains_gpu_system::allocate() {
     d_nbr_count = nullptr;
     d_nbr = nullptr;
     verlet = solo = false;
+    touch = dem::TouchList{};
   }
   pair_cap = (int)std::min<size_t>(16 * n + 4096, (size_t)1 << 28);
   HIPCHECK(this, track(this, &d_pairs, 2 * (size_t)pair_cap));
@@ -312,6 +328,13 @@ int grains_gpu_system::upload() {
   HIPCHECK(this, hipMemcpy(P.inertia, h_inertia.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   HIPCHECK(this, hipMemcpy(P.crust, h_crust.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   HIPCHECK(this, hipMemcpy(P.wfac, h_wfac.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  auto uniform = [&](const std::vector<double>& a) {
+    for (int i = 1; i < n; ++i)
+      if (a[i] != a[0]) return -1.;
+    return n && a[0] >= 0. ? a[0] : -1.;
+  };
+  crust_all = uniform(h_crust);
+  cfac_all = uniform(h_cfac);
   HIPCHECK(this, hipMemcpy(P.cfac, h_cfac.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   HIPCHECK(this, hipMemcpy(P.req, h_req.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   std::vector<int> ids((size_t)n);
@@ -354,6 +377,8 @@ StepParams grains_gpu_system::params() const {
   sp.stats = stats_on && !recording ? d_stat_part : nullptr;
   sp.mem = mem;
   sp.cf = cf;
+  sp.crust_all = crust_all;
+  sp.cfac_all = cfac_all;
   sp.fsum = fsum_on ? fsum_buf : nullptr;
   sp.hyd = d_hyd;
   return sp;
@@ -364,7 +389,8 @@ int grains_gpu_system::bin_current() {
   if (verlet) {
     // periodic wrap of the current positions, then a Verlet list build
     HIPCHECK(this, launch_key(P, S, grid, sp, d_status, vstate(-1), stream));
-    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), false, stream));
+    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), touch.count, false,
+                                       stream));
     return GRAINS_OK;
   }
   HIPCHECK(this, launch_key(P, S, grid, sp, d_status, vstate(0), stream));
@@ -437,7 +463,8 @@ int grains_gpu_system::bin_launch() {
   if (solo)
     ;  // the force sweep rebuilds the list itself
   else if (verlet)
-    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), true, stream));
+    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), touch.count, true,
+                                       stream));
   else
     HIPCHECK(this, launch_bin(P, S, grid, nparticles, cur & 1, stream));
   if (prof && (e = mark(prof->bin_ev, prof->nbin))) return e;
@@ -485,17 +512,19 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     return GRAINS_OK;
   }
   if (solo)  // an evaluation of the general sweep: the list must be current
-    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, L, true, stream));
+    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, L, touch.count, true, stream));
   const dem::NbrList CL = contact_list();
+  // (not for evaluations outside the step loop, nor with extras)
+  const dem::TouchList TL = mode == kModeForcesOnly || sp.stats || sp.fsum || sp.mem.cap ? dem::TouchList{} : touch;
   if (CL.count) {
     // this step's contacts from the Verlet list
     if (prof && (e = mark(prof->detect_ev, prof->ndetect))) return e;
-    HIPCHECK(this, launch_vfilter(P, S, grid, V, nparticles, cur & 1, L, CL, d_status, stream));
+    HIPCHECK(this, launch_vfilter(P, S, grid, V, nparticles, cur & 1, L, CL, TL, d_status, stream));
     if (prof && (e = mark(prof->detect_ev, prof->ndetect))) return e;
   }
   if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
   HIPCHECK(this, launch_forces(mode, cfg.precision == GRAINS_MIXED, P, S, grid, d_obs, d_models, sp, d_status,
-                               d_pairs, L, vstate(1), CL, stream));
+                               d_pairs, L, vstate(1), CL, TL, stream));
   if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
   if (sp.stats) HIPCHECK(this, launch_stats_fold(d_stat_part, nparticles, d_stat_tot, force_time, stream));
   // the evaluation wrote the other memory buffer: it becomes current

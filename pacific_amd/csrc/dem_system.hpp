@@ -102,6 +102,8 @@ struct grains_gpu_system {
   dem::VerletState V{};
   // contacts of the current step filtered from the Verlet list
   static constexpr int kContactCap = 16;
+  dem::TouchList touch{};  // the particles of a large gas that have a contact
+  static constexpr int kTouchMin = 500000;
   int* d_ct_count = nullptr;
   unsigned* d_ct = nullptr;
   dem::NbrList contact_list() const {
@@ -157,6 +159,7 @@ struct grains_gpu_system {
   int allocate();
   int upload();
   void free_device();
+  double crust_all = -1., cfac_all = -1.;  // StepParams
   dem::StepParams params() const;
   int bin_current();
   // particles given in an order without relation to their places are stored

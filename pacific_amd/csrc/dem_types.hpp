@@ -147,6 +147,16 @@ struct NbrList {
   int cap, n;
 };
 
+// The particles of a step that have a contact, by storage index, appended by
+// k_vfilter in kTouchLists parts of `stride` entries with a counter each
+// (kItemPad ints apart, cleared by the launches that renew the Verlet list).
+constexpr int kTouchLists = 8;
+struct TouchList {
+  int* idx;    // nullptr: not kept
+  int* count;
+  int stride;
+};
+
 // Progress of a list rebuild inside a force sweep (k_forces_solo): the next
 // piece of work and how many pieces of each phase are done.  One set per
 // position buffer; the sweep of the other buffer clears it.
@@ -254,6 +264,9 @@ struct StepParams {
   double* stats;      // contact statistics: 5 partial sums per force block (nullptr: not collected)
   ContactMemory mem;  // HookeMemory tables (mem.cap == 0: none)
   ContactFeat cf;     // contacts found by the narrow phase (systems with non-spherical bodies)
+  // crust thickness and coupling factor where every particle has the same (the
+  // arrays are then not read; crust_all < 0, cfac_all < 0: read them)
+  double crust_all, cfac_all;
   double* fsum;       // per storage index: sum of the magnitudes of its contact forces (nullptr: not kept)
   const double* hyd;  // fluid force and torque per storage index, component c at hyd[c * n + s] (nullptr: none)
 };
