@@ -68,6 +68,7 @@ struct AdjVisitor {
     in.mu = hm.muc;
     return in;
   }
+  static constexpr bool kEager = false;
   __device__ __forceinline__ void pair(int k2, int s2i, int pid2, d3 xo, double ro, d3 Pc, d3 ov, double d) {
     (void)k2;
     (void)Pc;

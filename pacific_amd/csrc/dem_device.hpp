@@ -737,6 +737,29 @@ __device__ __forceinline__ void record_pair(const StepParams& sp, DevStatus* st,
   }
 }
 
+// A particle's id, read when it is needed (errors, pair records, contact
+// memory, statistics).
+struct IdAt {
+  const int* p;
+  __device__ __forceinline__ operator int() const { return *p; }
+};
+
+// What a contact needs of the partner besides its position and radius.  The
+// FP64 sweeps with a thread per particle read all of it as soon as the partner
+// is known: read where it is used it is a chain of waits for memory (bed of
+// 200,000: 60 us -> 56; batches: 288 -> 280).  With FP32 arithmetic it spills at
+// three waves per SIMD (1M gas: 78 us -> 81), and a lane per contact has
+// nothing to gain (17.5 us for 18, and a wave per SIMD less).
+struct Other {
+  d3 v, w;
+  double m, c, req;
+  int mat;
+};
+
+__device__ __forceinline__ Other other_of(const Particles& P, int cv, int s) {
+  return Other{ld3(P.v[cv], s), ld3(P.w[cv], s), P.mass[s], P.crust[s], P.req[s], P.mat[s]};
+}
+
 // Shape classes and vertex table: P's, or copies of them in LDS.
 struct ShapeTables {
   const ShapeDesc* shapes;
@@ -900,9 +923,8 @@ __device__ __forceinline__ void for_each_candidate(const Sorted& S, const Grid& 
 // Two spheres whose centres pass the conservative distance reject (AB = xo -
 // x_self, nab = Norm(AB)): true with the contact features (d may be >= 0);
 // false when there is none, or after a ContactError.
-__device__ __forceinline__ bool sphere_features(const Particles& P, DevStatus* st, const Self& me, int s2i, int pid2,
-                                                d3 xo, double ro, d3 AB, double nab, d3& Pc, d3& ov, double& d) {
-  const double co = P.crust[s2i];
+__device__ __forceinline__ bool sphere_features(DevStatus* st, const Self& me, double co, IdAt pid2, d3 xo, double ro,
+                                                d3 AB, double nab, d3& Pc, d3& ov, double& d) {
   const int res = sphere_sphere(me.x, me.r, me.c, AB, nab, ro, co, Pc, ov, d);
   if (res < 0) {
     if (!recover_ss(me.x, me.r, me.c, xo, ro, co, Pc, ov, d)) {
@@ -944,7 +966,7 @@ __device__ __forceinline__ bool wall_features(const BoxObstacle& B, DevStatus* s
 // the reference meets it (image_evaluations; sh = the image code of xo).
 template <class V, bool SHAPES>
 __device__ __forceinline__ void narrow_visit(const Particles& P, const Grid& G, DevStatus* st, const Self& me,
-                                             V& vis, const ConvexGeo* mg, int cx, int k2, int s2i, int pid2, d3 xo,
+                                             V& vis, const ConvexGeo* mg, int cx, int k2, int s2i, IdAt pid2, d3 xo,
                                              double ro, d3 AB, double nab, const d3& xb, const int sh[3]) {
   d3 Pc, ov;
   double d;
@@ -962,7 +984,10 @@ __device__ __forceinline__ void narrow_visit(const Particles& P, const Grid& G, 
       atomicAdd(&st->n_recovered, 1);
     }
   } else {
-    if (!sphere_features(P, st, me, s2i, pid2, xo, ro, AB, nab, Pc, ov, d)) return;
+    double co;
+    if constexpr (V::kEager) co = vis.o.c;
+    else co = P.crust[s2i];
+    if (!sphere_features(st, me, co, pid2, xo, ro, AB, nab, Pc, ov, d)) return;
   }
   if (me.acc && me.id < pid2) me.acc->add(d, nit, image_evaluations(G, me.x, xb, sh));
   if (!(d < 0.)) return;
@@ -988,8 +1013,9 @@ __device__ __forceinline__ void visit_candidate(const Particles& P, const Sorted
   double nab = sqrt(s2);
   const int s2i = S.order[k2];
   if (s2i < slot_lo || s2i >= slot_hi) return;
+  if constexpr (V::kEager) vis.o = other_of(P, vis.cv, s2i);
   const int sh[3] = {ix, iy, iz};
-  narrow_visit<V, SHAPES>(P, G, st, me, vis, mg, cx, k2, s2i, S.sid[k2], xo, ro, AB, nab, d3{q2[0], q2[1], q2[2]},
+  narrow_visit<V, SHAPES>(P, G, st, me, vis, mg, cx, k2, s2i, IdAt{S.sid + k2}, xo, ro, AB, nab, d3{q2[0], q2[1], q2[2]},
                           sh);
 }
 
@@ -1013,6 +1039,7 @@ __device__ __forceinline__ d3 nearest_image(const Grid& G, d3 xo, const d3& x) {
 template <class V, bool SHAPES>
 __device__ __forceinline__ void visit_current_at(const Particles& P, const Grid& G, DevStatus* st, const Self& me,
                                                  V& vis, const ConvexGeo* mg, int cx, int s2i, d3 x2, double ro) {
+  if constexpr (V::kEager) vis.o = other_of(P, vis.cv, s2i);
   const d3 xo = nearest_image(G, x2, me.x);
   d3 AB = xo - me.x;
   double s2 = AB.x * AB.x + AB.y * AB.y + AB.z * AB.z;
@@ -1020,7 +1047,8 @@ __device__ __forceinline__ void visit_current_at(const Particles& P, const Grid&
   if (s2 > R * R * 1.000000000001) return;
   const int sh[3] = {xo.x < x2.x ? -1 : (xo.x > x2.x ? 1 : 0), xo.y < x2.y ? -1 : (xo.y > x2.y ? 1 : 0),
                      xo.z < x2.z ? -1 : (xo.z > x2.z ? 1 : 0)};
-  narrow_visit<V, SHAPES>(P, G, st, me, vis, mg, cx, -1, s2i, P.id[s2i], xo, ro, AB, sqrt(s2), x2, sh);
+  narrow_visit<V, SHAPES>(P, G, st, me, vis, mg, cx, -1, s2i, IdAt{P.id + s2i}, xo, ro, AB, sqrt(s2), x2,
+                          sh);
 }
 
 template <class V, bool SHAPES>
@@ -1119,8 +1147,10 @@ __device__ __forceinline__ void for_each_listed(const Particles& P, const Sorted
     for_each_contact<V, SHAPES>(P, S, G, obs, nobs, st, start_base, slot_lo, slot_hi, k, me, vis, mg, cx);
     return;
   }
+  unsigned next = c > 0 ? L.ent[k] : 0u;
   for (int i = 0; i < c; ++i) {
-    const unsigned e = L.ent[(size_t)i * L.n + k];
+    const unsigned e = next;
+    if (i + 1 < c) next = L.ent[(size_t)(i + 1) * L.n + k];
     const int code = (int)(e >> kNbrSlotBits);
     visit_candidate<V, SHAPES>(P, S, G, st, slot_lo, slot_hi, me, vis, mg, cx, (int)(e & kNbrSlotMask),
                                code % 3 - 1, (code / 3) % 3 - 1, code / 9 - 1);
@@ -1141,8 +1171,10 @@ __device__ __forceinline__ void for_each_verlet(const Particles& P, const Sorted
   // this step's contacts, filtered from the list (k_vfilter) in its order
   const int c2 = CL ? CL->count[s] : 0;
   if (CL && c2 <= CL->cap) {
+    unsigned next = c2 > 0 ? CL->ent[s] : 0u;
     for (int i = 0; i < c2; ++i) {
-      const unsigned s2i = CL->ent[(size_t)i * CL->n + s];
+      const unsigned s2i = next;
+      if (i + 1 < c2) next = CL->ent[(size_t)(i + 1) * CL->n + s];
       if (s2i < (unsigned)n) visit_current<V, SHAPES>(P, G, st, me, vis, mg, cx, (int)s2i);
     }
     visit_obstacles<V, SHAPES>(obs, nobs, st, me, vis, mg);
@@ -1169,7 +1201,8 @@ __device__ __forceinline__ void for_each_verlet(const Particles& P, const Sorted
 // the weight.  MIXED evaluates the model in FP32 on lever arms.
 // EXTRAS: contact memory models and statistics may occur (checked at run
 // time); without, the visitor carries none of their code.
-template <bool MIXED, bool EXTRAS = false>
+// EAGER: the partner's data are read before pair().
+template <bool MIXED, bool EXTRAS = false, bool EAGER = !MIXED>
 struct ForceVisitor {
   const Particles& P;
   const Sorted& S;
@@ -1184,6 +1217,8 @@ struct ForceVisitor {
   f3 Fc, Tc;
   int s = -1;     // storage index of self (contact memory)
   int nmem = 0;   // memory entries written by this evaluation
+  Other o{};      // the partner of the contact (EAGER: set before pair())
+  static constexpr bool kEager = EAGER;
   double fs = 0.; // sum of the contact-force magnitudes (EXTRAS with sp.fsum)
 
   // HookeMemory: this pair's entry of the last evaluation (zero when new),
@@ -1231,13 +1266,14 @@ struct ForceVisitor {
     return slip;
   }
 
-  __device__ __forceinline__ void pair(int k2, int s2i, int pid2, d3 xo, double ro, d3 Pc, d3 ov, double d) {
+  __device__ __forceinline__ void pair(int k2, int s2i, IdAt pid2, d3 xo, double ro, d3 Pc, d3 ov, double d) {
     (void)k2;
     (void)ro;
     (void)d;
-    const HookeModel& hm = models[me.mat * kMaxMaterials + P.mat[s2i]];
-    d3 vo = ld3(P.v[cv], s2i), wo = ld3(P.w[cv], s2i);
-    double mo = P.mass[s2i], reqo = P.req[s2i];
+    if constexpr (!EAGER) o = other_of(P, cv, s2i);
+    const HookeModel& hm = models[me.mat * kMaxMaterials + o.mat];
+    const d3 &vo = o.v, &wo = o.w;
+    const double mo = o.m, reqo = o.req;
     bool slip;
     if (EXTRAS && hm.memory) {
       slip = memory_pair(hm, pid2, xo, vo, wo, mo, reqo, Pc, ov);
@@ -1258,7 +1294,7 @@ struct ForceVisitor {
       if (hm.kr != 0.) T += dM * 1.;
       if (EXTRAS && sp.fsum) fs += norm(f);
     }
-    record_pair(sp, st, pairs, me.id, pid2, slip);
+    if (sp.record_pairs) record_pair(sp, st, pairs, me.id, pid2, slip);
   }
 
   __device__ __forceinline__ void wall(int o, d3 Pc, d3 ov, double d) {

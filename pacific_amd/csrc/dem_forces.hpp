@@ -94,7 +94,9 @@ __device__ __forceinline__ void listed_contacts(const Particles& P, const Sorted
       const int o = cf.ent[e];
       const d3 Pc{cf.f[3][e], cf.f[4][e], cf.f[5][e]}, ov{cf.f[6][e], cf.f[7][e], cf.f[8][e]};
       if (o >= 0) {
-        if (o < sp.n) vis.pair(-1, o, cf.pid[e], d3{cf.f[0][e], cf.f[1][e], cf.f[2][e]}, 0., Pc, ov, -1.);
+        if (o >= sp.n) continue;
+        if constexpr (decltype(vis)::kEager) vis.o = other_of(P, cv, o);
+        vis.pair(-1, o, IdAt{cf.pid + e}, d3{cf.f[0][e], cf.f[1][e], cf.f[2][e]}, 0., Pc, ov, -1.);
       } else if (-1 - o < sp.nobs) {
         vis.wall(-1 - o, Pc, ov, -1.);
       }

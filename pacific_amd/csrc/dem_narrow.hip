@@ -72,6 +72,7 @@ struct FeatureVisitor {
       cf.f[8][e] = ov.z;
     }
   }
+  static constexpr bool kEager = false;
   __device__ __forceinline__ void pair(int k2, int s2i, int pid2, d3 xo, double, d3 Pc, d3 ov, double d) {
     put(s2i, pid2, xo, Pc, ov);
     if (mirror && pid2 > me->id && L->count[k2] <= L->cap) mirror_full(k2, s2i, pid2, xo, Pc, ov, d);

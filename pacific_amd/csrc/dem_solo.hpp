@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
     StepParams sp, DevStatus* st, int* pairs, NbrList L, VerletState VS) {
   constexpr int T = kSoloThreads, B = kSoloBodies;
   static_assert(B == 64, "the offsets are scanned by one wave");
-  using FV = ForceVisitor<MIXED, MEM>;
+  using FV = ForceVisitor<MIXED, MEM, false>;
   using Term = TermT<MIXED, MEM>;
   __shared__ double self[11][B];
   __shared__ Term term[6][T];
@@ -250,7 +250,8 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
     const d3 AB = xo - me.x;
     const double s2 = AB.x * AB.x + AB.y * AB.y + AB.z * AB.z, R = me.r + ro;
     if (s2 > R * R * 1.000000000001) return false;
-    return sphere_features(P, st, me, s2i, P.id[s2i], xo, ro, AB, sqrt(s2), Pc, ov, d) && d < 0.;
+    const int id2 = P.id[s2i];
+    return sphere_features(st, me, P.crust[s2i], IdAt{&id2}, xo, ro, AB, sqrt(s2), Pc, ov, d) && d < 0.;
   };
   // exclusive offsets of n items per particle over the block; returns the total
   auto offsets = [&](int n, int which, int& off) {
@@ -343,7 +344,8 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
         return s2i < (unsigned)sp.n && pair_of(me, (int)s2i, xo, ro, Pc, ov, d);
       },
       [&](FV& vis, int s2i, d3 xo, double ro, d3 Pc, d3 ov, double d) {
-        vis.pair(-1, s2i, P.id[s2i], xo, ro, Pc, ov, d);
+        const int id2 = P.id[s2i];
+        vis.pair(-1, s2i, IdAt{&id2}, xo, ro, Pc, ov, d);
       });
   if (sp.nobs) {
     __syncthreads();
@@ -371,7 +373,7 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
     auto one = [&](int s2i) {
       d3 xo, Pc, ov;
       double ro, d = 0.;
-      if (pair_of(me, s2i, xo, ro, Pc, ov, d)) vis.pair(-1, s2i, P.id[s2i], xo, ro, Pc, ov, d);
+      if (pair_of(me, s2i, xo, ro, Pc, ov, d)) vis.pair(-1, s2i, IdAt{P.id + s2i}, xo, ro, Pc, ov, d);
     };
     const d3 xb{VS.xb[0][s], VS.xb[1][s], VS.xb[2][s]};
     for_each_candidate(S, VS.Gv, 0, 0, sp.n, xb, [&](int k2, int, int, int) {
