@@ -26,12 +26,12 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# Algorithmic bytes per particle-step: state read once and written once per
-# step.  FP64: x, v, w, q read+write (13 f64 x 8 B x 2 = 208 B), radius read
-# (8 B), F and T carried between the half kicks (6 f64 read+write = 96 B),
-# cell key write+read (8 B) -> 320 B; mixed: F, T in FP32 -> 272 B; plus 16 B
-# per contact pair (one int32 pair written and read).
-B_ALG = {"fp64": 320.0, "mixed": 272.0}
+# Algorithmic bytes per particle-step of the fused sweep of the gas: x, v, body
+# spin and q read (13 f64, 104 B), x, v, spins and q written (16 f64, 128 B), mass
+# and inertia (16 B), contact count (4 B), build position of the list (24 B)
+# -> 276 B in either precision; plus 16 B per contact pair (one int32 pair
+# written and read).
+B_ALG = {"fp64": 276.0, "mixed": 276.0}
 B_PAIR = 16.0
 
 
@@ -664,7 +664,8 @@ def main():
                    "contacts_per_particle": cbar, "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": f"k_forces{'64' if headline == FP64 else ''}<fused>", "kernel_ms": force_ms,
+                     "kernel": "k_verlet32<fused>" if headline == MIXED else
+                     "k_forces_gas<fused>" if args.n > 500000 else "k_verlet64<fused>", "kernel_ms": force_ms,
                      "bytes_alg_per_launch": b_alg, "contacts_per_particle": cbar, "binning_ms": bin_ms,
                      "contact_filter_ms": detect_ms, "verlet_skin_m": skin, "verlet_builds": builds},
     }
