@@ -181,8 +181,9 @@ __device__ __forceinline__ void solo_rebuild(const Particles& P, const Sorted& S
 }
 
 // ---------------------------------------------------------------------------
-// MEM: contact models with memory; the entries of a particle are numbered by
-// the contacts before (a mask per particle of those that touch).
+// MEM: contact models with memory.  A particle's entries are numbered by its
+// earlier contacts whose material pair has memory (a mask per particle): pairs
+// of a plain Hooke law, which write none, may stand between them.
 template <bool MIXED, bool MEM>
 using TermT = std::conditional_t<MIXED && !MEM, float, double>;
 
@@ -267,8 +268,9 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
     __syncthreads();
     return total_of[which];
   };
-  // the items of one kind: window after window of T, one per lane
-  auto sweep = [&](int n, int which, auto&& entry, auto&& features, auto&& force) {
+  // the items of one kind: window after window of T, one per lane; material: a
+  // partner's
+  auto sweep = [&](int n, int which, auto&& entry, auto&& features, auto&& material, auto&& force) {
     int off = 0;
     const int total = offsets(n, which, off);
     for (int base = 0; base < total; base += T) {
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
              f3{0.f, 0.f, 0.f}};
       if (MEM) {
         // (the window holds items of rising index per particle: bit e)
-        if (live) atomicOr(&touch[p], 1ull << (e & 63));
+        if (live && models[me.mat * kMaxMaterials + material(partner)].memory) atomicOr(&touch[p], 1ull << (e & 63));
         __syncthreads();
         vis.s = t0 + p;
         if (live) vis.nmem = rank0[p] + __popcll(touch[p] & ((1ull << (e & 63)) - 1ull));
@@ -343,6 +345,7 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
         partner = (int)s2i;
         return s2i < (unsigned)sp.n && pair_of(me, (int)s2i, xo, ro, Pc, ov, d);
       },
+      [&](int s2i) { return P.mat[s2i]; },
       [&](FV& vis, int s2i, d3 xo, double ro, d3 Pc, d3 ov, double d) {
         const int id2 = P.id[s2i];
         vis.pair(-1, s2i, IdAt{&id2}, xo, ro, Pc, ov, d);
@@ -361,7 +364,7 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
           partner = e;
           return wall_features(obs[e], st, me, Pc, ov, d) && d < 0.;
         },
-        [&](FV& vis, int o, d3, double, d3 Pc, d3 ov, double d) { vis.wall(o, Pc, ov, d); });
+        [&](int o) { return obs[o].mat; }, [&](FV& vis, int o, d3, double, d3 Pc, d3 ov, double d) { vis.wall(o, Pc, ov, d); });
   }
   if (!mine) return;
   if (over) {

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from pacific_amd import MIXED, workloads
-from tests.helpers import make_gpu
+from tests.helpers import contact_scale, make_gpu, make_oracle, pair_set, rel_force_error
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +83,71 @@ def test_many_obstacles(gpu):
     a, _ = run(wl, 0, 32, False, (50,))
     b, _ = run(wl, 0, 32, True, (50,))
     assert np.array_equal(a["x"], b["x"]) and np.array_equal(a["F"], b["F"])
+
+
+# laws of the material pairs (particles 0 and 1, walls 2); some with memory,
+# the others without: only the former have an entry in a particle's memory
+LAWS = {
+    "walls without": {(0, 0): 1, (0, 1): 1, (1, 1): 1, (0, 2): 0, (1, 2): 0},
+    "walls with": {(0, 0): 0, (0, 1): 0, (1, 1): 0, (0, 2): 1, (1, 2): 1},
+    "mixture": {(0, 0): 1, (0, 1): 0, (1, 1): 1, (0, 2): 1, (1, 2): 0},
+}
+
+
+def with_laws(wl, laws):
+    wl["models"] = [("memory", a, b, 1e4, 0.8, 0.4, 2e3, -1.0, 0.0, 0.1, 1e-10) if m else
+                    (a, b, 1e4, 0.8, 0.4, 0.0, -1.0) for (a, b), m in LAWS[laws].items()]
+    wl["boxes"] = [(L, c, B, crust, 2) for L, c, B, crust, _ in wl["boxes"]]
+    return wl
+
+
+@pytest.mark.parametrize("precision", [0, MIXED])
+@pytest.mark.parametrize("laws", sorted(LAWS))
+def test_memory_beside_plain_laws(gpu, laws, precision):
+    # contacts that open and close: against the general launches, bit for bit,
+    # and in FP64 the oracle (each side of a pair evaluates its own contact
+    # point: rounding, amplified over the steps as in the one-law packings)
+    wl = with_laws(workloads.dense_pack(side=6, sigma=0.2, squeeze=-1e-5), laws)
+    wl["material"] = (np.arange(216) % 2).astype(np.int32)
+    a = make_gpu(wl, precision=precision, record=True)
+    b = make_gpu(wl, precision=precision, record=True, stats=True)
+    o = make_oracle(wl)
+    npairs = set()
+    for k in (1, 60, 139):
+        a.step(k)
+        b.step(k)
+        o.step(k)
+        sa, sb, so = a.state(), b.state(), o.state()
+        for f in ("x", "v", "w", "F", "T"):
+            assert np.array_equal(sa[f], sb[f]), f
+        if precision == 0:
+            assert pair_set(a.pairs()) == pair_set(o.pairs())
+            scale = contact_scale(so, o.masses()[2])
+            # positions that differ by dx change a contact's force by kn dx: six
+            # neighbours, both ends, against a scale as small as the weight
+            dx = np.abs(sa["x"] - so["x"]).max()
+            assert dx <= 1e-13
+            assert rel_force_error(sa["F"], so["F"], scale) <= 1e-9 + 12 * 1e4 * dx / scale.min()
+        npairs.add(len(a.pairs()))
+    assert len(npairs) > 1 and max(npairs) > 100
+
+
+def test_many_plain_contacts_few_with_memory(gpu):
+    # a sphere on the floor (memory) with 40 small ones around it (none): more
+    # contacts than a particle keeps entries, but one entry
+    i = np.arange(40) + 0.5
+    th, ph = np.arccos(1 - 1.6 * i / 40), np.pi * (1 + 5 ** 0.5) * i
+    R, r = 4e-3, 0.4e-3
+    d = np.stack([np.cos(ph) * np.sin(th), np.sin(ph) * np.sin(th), np.cos(th)], 1)
+    c = np.array([0.01, 0.01, R - 1e-6])
+    wl = with_laws(workloads.settling_box(41), "mixture")
+    wl["x"] = np.concatenate([[c], c + d * (R + r - 1e-6)])
+    wl["radius"] = np.concatenate([[R], np.full(40, r)])
+    wl["material"] = np.array([0] + [1] * 40, np.int32)
+    a, b, o = make_gpu(wl, nbr=64), make_gpu(wl, nbr=64, stats=True), make_oracle(wl)
+    assert len(a.pairs()) == 81 and pair_set(a.pairs()) == pair_set(o.pairs())
+    for s in (a, b, o):
+        s.step(30)
+    for f in ("x", "v", "w", "F", "T"):
+        assert np.array_equal(a.state()[f], b.state()[f]), f
+    assert np.abs(a.state()["x"] - o.state()["x"]).max() <= 1e-12
