@@ -24,7 +24,7 @@ __global__ __launch_bounds__(256) void k_rows_out(RowMap m, const int* __restric
   if (s >= n) return;
   const unsigned i = (unsigned)(id[s] - 1);
   if (i >= (unsigned)n) return;
-  for (int c = 0; c < m.nc; ++c) out[(size_t)m.base[c] + (size_t)m.stride[c] * i] = m.comp[c][s];
+  for (int c = 0; c < m.nc; ++c) out[m.base[c] + (size_t)m.stride[c] * i] = m.comp[c][s];
 }
 
 __global__ __launch_bounds__(256) void k_rows_in(RowMap m, const int* __restrict__ id, int n,
@@ -33,7 +33,7 @@ __global__ __launch_bounds__(256) void k_rows_in(RowMap m, const int* __restrict
   if (s >= n) return;
   const unsigned i = (unsigned)(id[s] - 1);
   if (i >= (unsigned)n) return;
-  for (int c = 0; c < m.nc; ++c) m.comp[c][s] = in[(size_t)m.base[c] + (size_t)m.stride[c] * i];
+  for (int c = 0; c < m.nc; ++c) m.comp[c][s] = in[m.base[c] + (size_t)m.stride[c] * i];
 }
 
 __global__ __launch_bounds__(256) void k_body_spin(Particles P, int n, int cv) {
@@ -96,18 +96,6 @@ hipError_t launch_permute(const std::vector<double*>& a8, const std::vector<int*
   if (n == 0) return hipSuccess;
   hipError_t e = permute_arrays(a8, order, n, tmp, stream);
   return e == hipSuccess ? permute_arrays(a4, order, n, (int*)tmp, stream) : e;
-}
-
-void RowIO::add(double* host, double* const* comps, int width) {
-  if (!host || n_ == 0) return;
-  for (int c = 0; c < width; ++c) {
-    map_.comp[map_.nc] = comps[c];
-    map_.base[map_.nc] = (unsigned)(off_ + c);
-    map_.stride[map_.nc] = width;
-    ++map_.nc;
-  }
-  segs_.push_back(Seg{host, off_, (size_t)width * n_});
-  off_ += (size_t)width * n_;
 }
 
 namespace {

@@ -16,7 +16,7 @@ namespace dem {
 struct RowMap {
   static constexpr int kMax = 24;
   double* comp[kMax];
-  unsigned base[kMax];
+  size_t base[kMax];
   int stride[kMax];
   int nc = 0;
 };
@@ -38,7 +38,17 @@ hipError_t launch_permute(const std::vector<double*>& a8, const std::vector<int*
 class RowIO {
  public:
   explicit RowIO(int n) : n_(n) {}
-  void add(double* host, double* const* comps, int width);
+  void add(double* host, double* const* comps, int width) {
+    if (!host || n_ == 0) return;
+    for (int c = 0; c < width; ++c) {
+      map_.comp[map_.nc] = comps[c];
+      map_.base[map_.nc] = off_ + c;
+      map_.stride[map_.nc] = width;
+      ++map_.nc;
+    }
+    segs_.push_back(Seg{host, off_, (size_t)width * n_});
+    off_ += (size_t)width * n_;
+  }
   void add(const double* host, double* const* comps, int width) { add(const_cast<double*>(host), comps, width); }
   const RowMap& map() const { return map_; }
   size_t doubles() const { return off_; }
