@@ -211,7 +211,10 @@ __device__ __forceinline__ void force_one(const Particles& P, const Sorted& S, c
 __device__ __forceinline__ void number_next(const StepParams& sp, DevStatus* st, const VerletState& VS) {
   if (blockIdx.x != 0) return;
   const int nx = (sp.cur & 1) ^ 1;
-  if (threadIdx.x == 0) st->seq[nx] = st->seq[nx ^ 1] + 1;
+  if (threadIdx.x == 0) {
+    st->seq[nx] = st->seq[nx ^ 1] + 1;
+    st->stop[nx] = st->code != 0;
+  }
   if (VS.sync && threadIdx.x < sizeof(RebuildSync) / sizeof(int)) ((int*)(VS.sync + nx))[threadIdx.x] = 0;
 }
 

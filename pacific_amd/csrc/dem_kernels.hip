@@ -40,7 +40,10 @@ __global__ __launch_bounds__(256) void k_move(Particles P, Sorted S, Grid G, Ste
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   // the number of these positions (DevStatus::seq); no list rebuild is under
   // way: both sets of its counters start anew
-  if (V.stamp > 0 && s == 0) st->seq[sp.cur & 1] = number;
+  if (V.stamp > 0 && s == 0) {
+    st->seq[sp.cur & 1] = number;
+    st->stop[sp.cur & 1] = st->code != 0;
+  }
   if (V.sync && s < 2 * (int)(sizeof(RebuildSync) / sizeof(int))) ((int*)V.sync)[s] = 0;
   if (s >= sp.n) return;
   const int cx = sp.cur & 1, cv = (sp.cur >> 1) & 1;

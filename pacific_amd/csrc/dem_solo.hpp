@@ -205,7 +205,10 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
   const int tid = threadIdx.x;
   const int t0 = xcd_tile(blockIdx.x, gridDim.x) * B;
   const int cx = sp.cur & 1, cv = (sp.cur >> 1) & 1;
-  if (st->rebuild[cx] == st->seq[cx] + 1) solo_rebuild(P, S, VS, L, sp.n, cx, st);
+  // after an error (which ends the run) the rest of a batch of steps neither
+  // rebuilds nor searches, so that it costs little whatever the state has become
+  const bool stop = st->stop[cx] != 0;
+  if (!stop && st->rebuild[cx] == st->seq[cx] + 1) solo_rebuild(P, S, VS, L, sp.n, cx, st);
   if (MODE == kFused) number_next(sp, st, VS);
   const bool mine = tid < B && t0 + tid < sp.n;
   const int s = t0 + tid;
@@ -222,10 +225,11 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
     for (int k = 0; k < 11; ++k) self[k][tid] = a[k];
     // InitializeForce: torsor = weight at the centre (Particle.cpp:1408-1415)
     F = d3{sp.g[0] * wf, sp.g[1] * wf, sp.g[2] * wf};
-    c = L.count[s];
+    c = stop ? 0 : L.count[s];
     over = c > L.cap;
     if (over) c = 0;
-    for (int o = 0; o < sp.nobs; ++o)
+    const int nobs = stop ? 0 : sp.nobs;
+    for (int o = 0; o < nobs; ++o)
       if (near_obstacle(obs[o], x, r)) walls |= 1ull << o;
     cw = over ? 0 : __popcll(walls);
   }
@@ -268,9 +272,9 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
     __syncthreads();
     return total_of[which];
   };
-  // the items of one kind: window after window of T, one per lane; material: a
-  // partner's
-  auto sweep = [&](int n, int which, auto&& entry, auto&& features, auto&& material, auto&& force) {
+  // the items of one kind: window after window of T, one per lane; features
+  // also says whether the pair's law has memory
+  auto sweep = [&](int n, int which, auto&& entry, auto&& features, auto&& force) {
     int off = 0;
     const int total = offsets(n, which, off);
     for (int base = 0; base < total; base += T) {
@@ -286,16 +290,16 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
       d3 Pc, ov, xo{0., 0., 0.};
       double d = 0., ro = 0.;
       int partner = 0;
-      bool live = false;
+      bool live = false, memory = false;
       if (item) {
         me = body(p);
-        live = features(me, p, e, partner, xo, ro, Pc, ov, d);
+        live = features(me, p, e, partner, memory, xo, ro, Pc, ov, d);
       }
       FV vis{P, S, obs, models, sp, st, pairs, cv, me, d3{0., 0., 0.}, d3{0., 0., 0.}, f3{0.f, 0.f, 0.f},
              f3{0.f, 0.f, 0.f}};
       if (MEM) {
         // (the window holds items of rising index per particle: bit e)
-        if (live && models[me.mat * kMaxMaterials + material(partner)].memory) atomicOr(&touch[p], 1ull << (e & 63));
+        if (live && memory) atomicOr(&touch[p], 1ull << (e & 63));
         __syncthreads();
         vis.s = t0 + p;
         if (live) vis.nmem = rank0[p] + __popcll(touch[p] & ((1ull << (e & 63)) - 1ull));
@@ -340,12 +344,13 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
   };
   sweep(
       c, 0, [](int i) { return i; },
-      [&](const Self& me, int p, int e, int& partner, d3& xo, double& ro, d3& Pc, d3& ov, double& d) {
+      [&](const Self& me, int p, int e, int& partner, bool& memory, d3& xo, double& ro, d3& Pc, d3& ov, double& d) {
         const unsigned s2i = L.ent[(size_t)e * L.n + t0 + p];
         partner = (int)s2i;
-        return s2i < (unsigned)sp.n && pair_of(me, (int)s2i, xo, ro, Pc, ov, d);
+        if (s2i >= (unsigned)sp.n) return false;
+        if (MEM) memory = models[me.mat * kMaxMaterials + P.mat[s2i]].memory != 0;
+        return pair_of(me, (int)s2i, xo, ro, Pc, ov, d);
       },
-      [&](int s2i) { return P.mat[s2i]; },
       [&](FV& vis, int s2i, d3 xo, double ro, d3 Pc, d3 ov, double d) {
         const int id2 = P.id[s2i];
         vis.pair(-1, s2i, IdAt{&id2}, xo, ro, Pc, ov, d);
@@ -360,11 +365,12 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
           left &= left - 1ull;
           return o;
         },
-        [&](const Self& me, int, int e, int& partner, d3&, double&, d3& Pc, d3& ov, double& d) {
+        [&](const Self& me, int, int e, int& partner, bool& memory, d3&, double&, d3& Pc, d3& ov, double& d) {
           partner = e;
+          if (MEM) memory = models[me.mat * kMaxMaterials + obs[e].mat].memory != 0;
           return wall_features(obs[e], st, me, Pc, ov, d) && d < 0.;
         },
-        [&](int o) { return obs[o].mat; }, [&](FV& vis, int o, d3, double, d3 Pc, d3 ov, double d) { vis.wall(o, Pc, ov, d); });
+        [&](FV& vis, int o, d3, double, d3 Pc, d3 ov, double d) { vis.wall(o, Pc, ov, d); });
   }
   if (!mine) return;
   if (over) {

@@ -200,6 +200,10 @@ struct DevStatus {
   // and the launch that reads one of the pair writes the other.
   int rebuild[2];
   int seq[2];
+  // whether an error was raised before the positions in buffer b were written,
+  // as the launch that wrote them found it: the same for the whole of a launch
+  // that reads it, in which errors may be raised while workgroups start
+  int stop[2];
   int n_rebuild;     // Verlet list builds
 };
 

@@ -6,10 +6,12 @@ enough to rebuild the list many times, packings whose workgroups hold more
 contacts than lanes, lists too short for their neighbours (searched in their
 cells), contact memory, and the size above which the general launches run
 anyway."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from pacific_amd import MIXED, workloads
+from pacific_amd import GrainsError, MIXED, workloads
 from tests.helpers import contact_scale, make_gpu, make_oracle, pair_set, rel_force_error
 
 pytestmark = pytest.mark.gpu
@@ -151,3 +153,26 @@ def test_many_plain_contacts_few_with_memory(gpu):
     for f in ("x", "v", "w", "F", "T"):
         assert np.array_equal(a.state()[f], b.state()[f]), f
     assert np.abs(a.state()["x"] - o.state()["x"]).max() <= 1e-12
+
+
+@pytest.mark.parametrize("laws", [None, "mixture"])
+@pytest.mark.parametrize("precision", [0, MIXED])
+def test_nothing_searched_after_an_error(gpu, precision, laws):
+    # one sphere too fast (more than the crust's thickness in a step): the
+    # batch goes on without contacts, at a force that is the weight alone, over
+    # graph replays and single steps, and reports the first error
+    wl = workloads.dense_pack(side=6)
+    if laws:
+        with_laws(wl, laws)
+    wl["v"][17] = (6.0, 0.0, 0.0)
+    g = make_gpu(wl, precision=precision, record=False)
+    assert np.abs(g.state()["F"] - g.masses()[2]).max() > 1e-3
+    L = g._check.__globals__["lib"]()
+    for k in (200, 1, 2):
+        with pytest.raises(GrainsError, match="MotionError") as e:
+            g.step(k)
+        assert e.value.ids[0] == 18
+        F = np.empty((216, 3))
+        p = F.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+        L.grains_gpu_get_state(g.h, None, None, None, None, None, p, None)
+        assert np.array_equal(F, g.masses()[2])
