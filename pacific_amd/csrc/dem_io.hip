@@ -125,41 +125,56 @@ void RowBuffers::release() {
   lanes_.clear();
 }
 
-hipError_t RowBuffers::reserve(size_t doubles) {
-  if (doubles <= dev_cap_) return hipSuccess;
-  if (dev_) (void)hipFree(dev_);
-  dev_ = nullptr;
-  dev_cap_ = 0;
-  hipError_t e = hipMalloc((void**)&dev_, doubles * sizeof(double));
-  if (e == hipSuccess) dev_cap_ = doubles;
-  return e;
+// How many threads copy a part, and the pinned bytes it needs.
+static int copy_threads(size_t total) {
+  if (total <= kSingle) return 0;
+  return (int)std::min<size_t>({(size_t)kThreads, total / kChunk,
+                                (size_t)std::max(1u, std::thread::hardware_concurrency() / 2)});
 }
 
-hipError_t RowBuffers::copy(const RowIO& io, bool to_host, int device, hipStream_t stream) {
-  const size_t total = io.doubles() * sizeof(double);
-  const bool single = total <= kSingle;
-  const int nthreads =
-      single ? 0
-             : (int)std::min<size_t>({(size_t)kThreads, total / kChunk,
-                                      (size_t)std::max(1u, std::thread::hardware_concurrency() / 2)});
-  const size_t want = single ? std::max<size_t>(total, 4096) : (size_t)nthreads * 2 * kChunk;
-  if (want > pin_cap_) {
+hipError_t RowBuffers::reserve(const RowIO& io, size_t first, size_t last, hipStream_t stream) {
+  size_t total = 0;
+  for (size_t k = first; k < last; ++k) total += io.segs()[k].count * sizeof(double);
+  const int nthreads = copy_threads(total);
+  const size_t pinned = nthreads ? (size_t)nthreads * 2 * kChunk : std::max<size_t>(total, 4096);
+  if (total <= dev_cap_ && pinned <= pin_cap_) return hipSuccess;
+  // what was enqueued before may still use the buffers
+  hipError_t e = hipStreamSynchronize(stream);
+  if (e != hipSuccess) return e;
+  if (total > dev_cap_) {
+    if (dev_) (void)hipFree(dev_);
+    dev_ = nullptr;
+    dev_cap_ = 0;
+    if ((e = hipMalloc((void**)&dev_, total)) != hipSuccess) return e;
+    dev_cap_ = total;
+  }
+  if (pinned > pin_cap_) {
     if (pin_) (void)hipHostFree(pin_);
     pin_ = nullptr;
     pin_cap_ = 0;
-    hipError_t e = hipHostMalloc((void**)&pin_, want, hipHostMallocDefault);
-    if (e != hipSuccess) return e;
-    pin_cap_ = want;
+    if ((e = hipHostMalloc((void**)&pin_, pinned, hipHostMallocDefault)) != hipSuccess) return e;
+    pin_cap_ = pinned;
   }
-  if (single) {
+  return e;
+}
+
+hipError_t RowBuffers::copy(const RowIO& io, size_t first, size_t last, bool to_host, int device, hipStream_t stream) {
+  size_t total = 0;
+  for (size_t k = first; k < last; ++k) total += io.segs()[k].count * sizeof(double);
+  const int nthreads = copy_threads(total);
+  if (!nthreads) {
     if (to_host) {
       hipError_t e = hipMemcpyAsync(pin_, dev_, total, hipMemcpyDeviceToHost, stream);
       if (e == hipSuccess) e = hipStreamSynchronize(stream);
       if (e != hipSuccess) return e;
-      for (auto& s : io.segs()) std::memcpy(s.host, (double*)pin_ + s.off, s.count * sizeof(double));
+      const char* from = pin_;
+      for (size_t k = first; k < last; from += io.segs()[k++].count * sizeof(double))
+        std::memcpy(io.segs()[k].host, from, io.segs()[k].count * sizeof(double));
       return hipSuccess;
     }
-    for (auto& s : io.segs()) std::memcpy((double*)pin_ + s.off, s.host, s.count * sizeof(double));
+    char* to = pin_;
+    for (size_t k = first; k < last; to += io.segs()[k++].count * sizeof(double))
+      std::memcpy(to, io.segs()[k].host, io.segs()[k].count * sizeof(double));
     return hipMemcpyAsync(dev_, pin_, total, hipMemcpyHostToDevice, stream);
   }
   while ((int)lanes_.size() < nthreads) {
@@ -168,13 +183,16 @@ hipError_t RowBuffers::copy(const RowIO& io, bool to_host, int device, hipStream
     if (e != hipSuccess) return e;
     lanes_.push_back(st);
   }
-  hipError_t first = hipStreamSynchronize(stream);
-  if (first != hipSuccess) return first;
+  const hipError_t drained = hipStreamSynchronize(stream);
+  if (drained != hipSuccess) return drained;
   std::vector<Chunk> chunks;
-  for (auto& s : io.segs())
-    for (size_t o = 0; o < s.count * sizeof(double); o += kChunk)
-      chunks.push_back(Chunk{(char*)s.host + o, s.off * sizeof(double) + o,
-                             std::min(kChunk, s.count * sizeof(double) - o)});
+  size_t off = 0;
+  for (size_t k = first; k < last; ++k) {
+    const size_t bytes = io.segs()[k].count * sizeof(double);
+    for (size_t o = 0; o < bytes; o += kChunk)
+      chunks.push_back(Chunk{(char*)io.segs()[k].host + o, off + o, std::min(kChunk, bytes - o)});
+    off += bytes;
+  }
   std::atomic<int> next{0};
   std::atomic<int> error{(int)hipSuccess};
   const int nc = (int)chunks.size();
@@ -219,21 +237,53 @@ hipError_t RowBuffers::copy(const RowIO& io, bool to_host, int device, hipStream
   return (hipError_t)error.load();
 }
 
+hipError_t RowBuffers::plain(const RowIO& io, size_t first, bool to_host, const int* id, int n, hipStream_t stream) {
+  (void)hipGetLastError();  // the allocation that failed
+  hipError_t e = hipStreamSynchronize(stream);
+  std::vector<int> ids((size_t)n);
+  std::vector<double> buf((size_t)n);
+  if (e == hipSuccess) e = hipMemcpy(ids.data(), id, sizeof(int) * n, hipMemcpyDeviceToHost);
+  for (size_t k = first; e == hipSuccess && k < io.segs().size(); ++k) {
+    const RowIO::Seg& s = io.segs()[k];
+    for (int c = 0; c < s.width && e == hipSuccess; ++c) {
+      auto row = [&](int i) -> double& { return s.host[(size_t)s.width * (ids[i] - 1) + c]; };
+      if (to_host) {
+        e = hipMemcpy(buf.data(), s.comp[c], sizeof(double) * n, hipMemcpyDeviceToHost);
+        if (e == hipSuccess)
+          for (int i = 0; i < n; ++i) row(i) = buf[i];
+      } else {
+        for (int i = 0; i < n; ++i) buf[i] = row(i);
+        e = hipMemcpy(s.comp[c], buf.data(), sizeof(double) * n, hipMemcpyHostToDevice);
+      }
+    }
+  }
+  return e;
+}
+
 hipError_t RowBuffers::down(const RowIO& io, const int* id, int n, int device, hipStream_t stream) {
-  if (io.doubles() == 0) return hipStreamSynchronize(stream);
-  hipError_t e = reserve(io.doubles());
-  if (e == hipSuccess) e = launch_rows_out(io.map(), id, n, dev_, stream);
-  if (e == hipSuccess) e = copy(io, true, device, stream);
+  if (io.segs().empty()) return hipStreamSynchronize(stream);
+  hipError_t e = hipSuccess;
+  for (size_t k = 0, l; k < io.segs().size() && e == hipSuccess; k = l) {
+    l = io.part(k);
+    e = reserve(io, k, l, stream);
+    if (e == hipErrorOutOfMemory) return plain(io, k, true, id, n, stream);
+    if (e == hipSuccess) e = launch_rows_out(io.map(k, l), id, n, dev_, stream);
+    if (e == hipSuccess) e = copy(io, k, l, true, device, stream);
+  }
   return e;
 }
 
 hipError_t RowBuffers::up(const RowIO& io, const int* id, int n, int device, hipStream_t stream) {
-  if (io.doubles() == 0) return hipSuccess;
-  // the buffers may still be read by what an earlier call enqueued
-  hipError_t e = hipStreamSynchronize(stream);
-  if (e == hipSuccess) e = reserve(io.doubles());
-  if (e == hipSuccess) e = copy(io, false, device, stream);
-  if (e == hipSuccess) e = launch_rows_in(io.map(), id, n, dev_, stream);
+  hipError_t e = hipSuccess;
+  for (size_t k = 0, l; k < io.segs().size() && e == hipSuccess; k = l) {
+    l = io.part(k);
+    // the buffers may still be read by what an earlier call or part enqueued
+    e = hipStreamSynchronize(stream);
+    if (e == hipSuccess) e = reserve(io, k, l, stream);
+    if (e == hipErrorOutOfMemory) return plain(io, k, false, id, n, stream);
+    if (e == hipSuccess) e = copy(io, k, l, false, device, stream);
+    if (e == hipSuccess) e = launch_rows_in(io.map(k, l), id, n, dev_, stream);
+  }
   return e;
 }
 

@@ -31,40 +31,66 @@ constexpr int kPermuteGroup = 4;
 hipError_t launch_permute(const std::vector<double*>& a8, const std::vector<int*>& a4, const int* order, int n,
                           double* tmp, hipStream_t stream);
 
-// The rows of one call (rows of `width` doubles per particle in the caller's
-// array; a null array is left out) and the buffers they pass through: a device
-// buffer in row layout and pinned host slices, both kept for the next call
-// and freed with the system.
+// The rows of one call: rows of `width` doubles per particle in the caller's
+// array (a null array is left out).  They pass through the buffers below in
+// parts of whole arrays, each as long as fits in kPart bytes (one array at
+// least), so that what is kept on the device stays small beside a large state
+// (64 MB, three parts, cost 2 % of a pass of the 1M gas).
 class RowIO {
  public:
-  explicit RowIO(int n) : n_(n) {}
+  static constexpr size_t kPart = (size_t)192 << 20;
+  explicit RowIO(int n) : n_((size_t)n) {}
   void add(double* host, double* const* comps, int width) {
     if (!host || n_ == 0) return;
-    for (int c = 0; c < width; ++c) {
-      map_.comp[map_.nc] = comps[c];
-      map_.base[map_.nc] = off_ + c;
-      map_.stride[map_.nc] = width;
-      ++map_.nc;
-    }
-    segs_.push_back(Seg{host, off_, (size_t)width * n_});
-    off_ += (size_t)width * n_;
+    Seg s{host, (size_t)width * n_, {}, width};
+    for (int c = 0; c < width; ++c) s.comp[c] = comps[c];
+    segs_.push_back(s);
   }
   void add(const double* host, double* const* comps, int width) { add(const_cast<double*>(host), comps, width); }
-  const RowMap& map() const { return map_; }
-  size_t doubles() const { return off_; }
   struct Seg {
     double* host;
-    size_t off, count;
+    size_t count;  // doubles
+    double* comp[9];
+    int width;
   };
   const std::vector<Seg>& segs() const { return segs_; }
+  // the part that begins with array `first` ends before the one returned
+  size_t part(size_t first) const {
+    size_t last = first, bytes = 0;
+    int nc = 0;
+    while (last < segs_.size()) {
+      bytes += segs_[last].count * sizeof(double);
+      nc += segs_[last].width;
+      if (last > first && (bytes > kPart || nc > RowMap::kMax)) break;
+      ++last;
+    }
+    return last;
+  }
+  // its rows one array after the other, from 0
+  RowMap map(size_t first, size_t last) const {
+    RowMap m;
+    size_t at = 0;
+    for (size_t k = first; k < last; ++k) {
+      for (int c = 0; c < segs_[k].width; ++c) {
+        m.comp[m.nc] = segs_[k].comp[c];
+        m.base[m.nc] = at + c;
+        m.stride[m.nc] = segs_[k].width;
+        ++m.nc;
+      }
+      at += segs_[k].count;
+    }
+    return m;
+  }
 
  private:
-  int n_;
-  size_t off_ = 0;
-  RowMap map_;
+  size_t n_;
   std::vector<Seg> segs_;
 };
 
+// The buffers the rows pass through: a device buffer in row layout and pinned
+// host slices, both kept for the next call and freed with the system.  Where
+// the card or the host has no room for them, the components cross one by one
+// and are put in their rows here on the host (plain).
 class RowBuffers {
  public:
   ~RowBuffers() { release(); }
@@ -77,10 +103,11 @@ class RowBuffers {
   hipError_t up(const RowIO& io, const int* id, int n, int device, hipStream_t stream);
 
  private:
-  hipError_t reserve(size_t doubles);
-  hipError_t copy(const RowIO& io, bool to_host, int device, hipStream_t stream);
+  hipError_t reserve(const RowIO& io, size_t first, size_t last, hipStream_t stream);
+  hipError_t copy(const RowIO& io, size_t first, size_t last, bool to_host, int device, hipStream_t stream);
+  hipError_t plain(const RowIO& io, size_t first, bool to_host, const int* id, int n, hipStream_t stream);
   double* dev_ = nullptr;
-  size_t dev_cap_ = 0;
+  size_t dev_cap_ = 0;  // bytes
   char* pin_ = nullptr;
   size_t pin_cap_ = 0;
   std::vector<hipStream_t> lanes_;  // one per copying thread

@@ -5,6 +5,9 @@ block that just fits the single pinned slice (2 MB: 11,915 particles with all
 end; and with every combination of arrays left out.  Values come back bit for
 bit, wb as q and w say."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -87,3 +90,62 @@ def test_basis_rows(gpu, n):
     assert np.array_equal(g.basis().reshape(n, 9), B)
     g.set_basis(B[::-1])
     assert np.array_equal(g.basis().reshape(n, 9), B[::-1])
+
+
+# hipMalloc and hipHostMalloc as the library finds them: they have no room for
+# requests of `room` bytes or more once told so
+SHIM = r"""
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stddef.h>
+int refused = 0;
+static size_t room[2] = {(size_t)-1, (size_t)-1};
+void leave(size_t device, size_t host) { room[0] = device; room[1] = host; }
+int hipMalloc(void** p, size_t n) {
+  if (n >= room[0]) { ++refused; *p = 0; return 2; }
+  return ((int (*)(void**, size_t))dlsym(RTLD_NEXT, "hipMalloc"))(p, n);
+}
+int hipHostMalloc(void** p, size_t n, unsigned flags) {
+  if (n >= room[1]) { ++refused; *p = 0; return 2; }
+  return ((int (*)(void**, size_t, unsigned))dlsym(RTLD_NEXT, "hipHostMalloc"))(p, n, flags);
+}
+"""
+
+NO_ROOM = """
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+shim.leave.argtypes = [ctypes.c_size_t] * 2
+import numpy as np
+from tests.test_gpu_rows import sparse
+n, every = int(sys.argv[2]), 2 ** 64 - 1
+g, x = sparse(n)
+h, _ = sparse(n)
+rng = np.random.default_rng(n)
+q = rng.normal(size=(n, 4))
+new = dict(x=x + 1e-5, v=rng.normal(size=(n, 3)), w=rng.normal(size=(n, 3)), q=q / np.linalg.norm(q, axis=1)[:, None])
+shim.leave(0 if sys.argv[3] == "device" else every, 0 if sys.argv[3] == "host" else every)
+g.set_state(**new)
+g.set_state(v=new["v"][::-1])
+a = g.state()
+assert ctypes.c_int.in_dll(shim, "refused").value >= 3
+shim.leave(every, every)
+h.set_state(**new)
+h.set_state(v=new["v"][::-1])
+for s in (h.state(), g.state()):
+    for k in a:
+        assert np.array_equal(a[k], s[k]), k
+print("same")
+"""
+
+
+@pytest.mark.parametrize("n,where", [(257, "device"), (257, "host"), (100003, "device"), (100003, "host")])
+def test_no_room_for_buffers(gpu, tmp_path, n, where):
+    # transfers need no memory: on a full card, or host, they take longer
+    (tmp_path / "shim.c").write_text(SHIM)
+    so = str(tmp_path / "shim.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", so, str(tmp_path / "shim.c"), "-Wl,--no-as-needed,-rpath,/opt/rocm/lib",
+                    "-L/opt/rocm/lib", "-lamdhip64", "-ldl"], check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", NO_ROOM, so, str(n), where], cwd=root, stdout=subprocess.PIPE,
+                         stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert out.returncode == 0 and out.stdout.endswith("same\n"), out.stdout[-2000:]

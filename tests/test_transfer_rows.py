@@ -20,8 +20,13 @@ int main(int argc, char** argv) {
   double* const comps[4] = {comp, comp + 1, comp + 2, comp + 3};
   dem::RowIO io(std::atoi(argv[1]));
   for (int w : widths) io.add(&host, comps, w);
-  const dem::RowMap& m = io.map();
-  for (int c = 0; c < m.nc; ++c) std::printf("%zu %d\n", (size_t)m.base[c], m.stride[c]);
+  if (argc == 2) {
+    const dem::RowMap m = io.map(0, io.segs().size());
+    for (int c = 0; c < m.nc; ++c) std::printf("%zu %d\n", (size_t)m.base[c], m.stride[c]);
+  } else {
+    for (size_t k = 0; k < io.segs().size(); k = io.part(k))
+      std::printf("%zu %zu\n", io.part(k) - k, (size_t)io.map(k, io.part(k)).base[0]);
+  }
 }
 """
 
@@ -36,8 +41,8 @@ def offsets(tmp_path_factory):
     subprocess.run([cxx, "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I", CSRC, "-o",
                     str(d / "rows"), str(d / "rows.cpp")], check=True)
 
-    def run(n):
-        out = subprocess.run([str(d / "rows"), str(n)], check=True, stdout=subprocess.PIPE, text=True).stdout
+    def run(*args):
+        out = subprocess.run([str(d / "rows")] + [str(a) for a in args], check=True, stdout=subprocess.PIPE, text=True).stdout
         return [tuple(map(int, line.split())) for line in out.splitlines()]
 
     return run
@@ -50,3 +55,10 @@ def test_offsets(offsets, n):
         want += [(at + c, w) for c in range(w)]
         at += w * n
     assert offsets(n) == want
+
+
+@pytest.mark.parametrize("n,arrays", [(1, [7]), (1143901, [7]), (1143902, [6, 1]), (3000000, [2, 2, 2, 1]),
+                                      (10000000, [1] * 7), (230000000, [1] * 7)])
+def test_parts(offsets, n, arrays):
+    # whole arrays up to 192 MB, the rows of each part from 0
+    assert offsets(n, "parts") == [(k, 0) for k in arrays]
