@@ -383,7 +383,7 @@ int grains_gpu_adjoint_backward(grains_gpu_system* s, int matA, int matB, const 
   in.add(dJ_dx, A.xb, 3);
   in.add(dJ_dv, A.vb, 3);
   in.add(dJ_dw, A.wb, 3);
-  ACHECK(s, s->rows.up(in, s->P.id, N, s->device, s->stream));
+  ACHECK(s, s->rows->up(in, s->P.id, N, s->stream));
   for (int c = 0; c < 3; ++c) {
     if (!dJ_dx) ACHECK(s, hipMemsetAsync(A.xb[c], 0, n * sizeof(double), s->stream));
     if (!dJ_dv) ACHECK(s, hipMemsetAsync(A.vb[c], 0, n * sizeof(double), s->stream));
@@ -437,11 +437,12 @@ int grains_gpu_adjoint_backward(grains_gpu_system* s, int matA, int matB, const 
                      (int)s->obstacles.size(), s->d_models, A, N, 0, matA, matB, h, dt, 1., 1, s->d_status);
   ACHECK(s, hipGetLastError());
   // results
+  ACHECK(s, hipStreamSynchronize(s->stream));
   RowIO out(N);
   out.add(grad_x0, A.xb, 3);
   out.add(grad_v0, A.vb, 3);
   out.add(grad_w0, A.wb, 3);
-  ACHECK(s, s->rows.down(out, s->P.id, N, s->device, s->stream));
+  ACHECK(s, s->rows->down(out, s->P.id, N, s->stream));
   if (grad_params) {
     std::vector<double> gth(3 * n);
     ACHECK(s, hipMemcpy(gth.data(), A.gth, 3 * n * sizeof(double), hipMemcpyDeviceToHost));

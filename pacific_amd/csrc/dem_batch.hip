@@ -394,7 +394,7 @@ struct grains_gpu_batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::vector<void*> allocations;
-  RowBuffers rows;                // buffers of the state transfers
+  std::shared_ptr<RowBuffers> rows;  // buffers of the state transfers
   DevStatus* h_status = nullptr;  // pinned
   ~grains_gpu_batch();
   int launch(int mode, int nsteps);
@@ -439,8 +439,7 @@ grains_gpu_batch::~grains_gpu_batch() {
   if (exec) (void)hipGraphExecDestroy(exec);
   if (graph) (void)hipGraphDestroy(graph);
   for (void* p : allocations) (void)hipFree(p);
-  rows.release();
-  if (h_status) (void)hipHostFree(h_status);
+  if (h_status) rows->give_back(h_status);
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
   if (stream) (void)hipStreamDestroy(stream);
@@ -693,7 +692,8 @@ int grains_gpu_batch_create(grains_gpu_system* const* systems, int nsys, int pre
   BCHECK(b, balloc(b, &b->d_models, hmod.size()));
   BCHECK(b, up(b->d_models, hmod));
   BCHECK(b, balloc(b, &b->d_status, 1));
-  BCHECK(b, hipHostMalloc((void**)&b->h_status, sizeof(DevStatus), hipHostMallocDefault));
+  b->rows = RowBuffers::of(b->device);
+  b->h_status = b->rows->status_block();
   BCHECK(b, hipMemset(b->d_status, 0, sizeof(DevStatus)));
   b->time = systems[0]->cfg.t_start;
   int e = b->launch(0, 0);  // bin + initial forces
@@ -847,7 +847,7 @@ int grains_gpu_batch_get_state(grains_gpu_batch* b, int isys, double* x, double*
   io.add(T, at(b->P.T, 3, o), 3);
   int e = b->fetch();
   if (e) return e;
-  BCHECK(b, b->rows.down(io, b->P.id + p0, n, b->device, b->stream));
+  BCHECK(b, b->rows->down(io, b->P.id + p0, n, b->stream));
   return b->read();
 }
 

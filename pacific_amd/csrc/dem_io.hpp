@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "dem_types.hpp"
@@ -87,30 +89,48 @@ class RowIO {
   std::vector<Seg> segs_;
 };
 
-// The buffers the rows pass through: a device buffer in row layout and pinned
-// host slices, both kept for the next call and freed with the system.  Where
-// the card or the host has no room for them, the components cross one by one
-// and are put in their rows here on the host (plain).
+// What the transfers of one device pass through, shared by its systems and
+// batches: a device buffer in row layout and pinned host slices, each as large
+// as the largest part so far, and pinned blocks that a status block comes back
+// to.  Made with the first system and freed with the last: allocating them
+// costs 0.3 ms each above 2 MB, as long as a state of 27,000 takes.  A call holds
+// the lock while it uses the buffers, and therefore comes with a stream that
+// has little left to do.  Where the card or the host has no room for
+// them, the components cross one by one and are put in their rows here on the
+// host (plain).
 class RowBuffers {
  public:
-  ~RowBuffers() { release(); }
-  void release();
+  static std::shared_ptr<RowBuffers> of(int device);
+  explicit RowBuffers(int device) : device_(device) {}
+  RowBuffers(const RowBuffers&) = delete;
+  ~RowBuffers();
   // device state (storage order, ids at id) -> the host arrays of io; the
   // stream has drained on return
-  hipError_t down(const RowIO& io, const int* id, int n, int device, hipStream_t stream);
+  hipError_t down(const RowIO& io, const int* id, int n, hipStream_t stream);
   // the host arrays of io -> device state; enqueued on the stream after the
   // rows have left the host arrays
-  hipError_t up(const RowIO& io, const int* id, int n, int device, hipStream_t stream);
+  hipError_t up(const RowIO& io, const int* id, int n, hipStream_t stream);
+  // a block for a DevStatus, to be given back
+  DevStatus* status_block();
+  void give_back(DevStatus* p);
 
  private:
-  hipError_t reserve(const RowIO& io, size_t first, size_t last, hipStream_t stream);
-  hipError_t copy(const RowIO& io, size_t first, size_t last, bool to_host, int device, hipStream_t stream);
+  hipError_t reserve(const RowIO& io, size_t first, size_t last);
+  hipError_t copy(const RowIO& io, size_t first, size_t last, bool to_host, hipStream_t stream);
   hipError_t plain(const RowIO& io, size_t first, bool to_host, const int* id, int n, hipStream_t stream);
+  const int device_;
+  std::mutex use_;  // the buffers
   double* dev_ = nullptr;
   size_t dev_cap_ = 0;  // bytes
   char* pin_ = nullptr;
   size_t pin_cap_ = 0;
-  std::vector<hipStream_t> lanes_;  // one per copying thread
+  std::vector<hipEvent_t> copied_;  // one per copying thread
+  std::vector<hipStream_t> lanes_;
+  hipEvent_t read_ = nullptr;  // after the kernel that last read rows from the device buffer
+  bool in_use_ = false;
+  std::mutex blocks_;
+  std::vector<DevStatus*> pages_, free_;
+  std::vector<std::unique_ptr<DevStatus[]>> plain_;
 };
 
 }  // namespace dem

@@ -50,8 +50,7 @@ void grains_gpu_system::free_device() {
   drop_graphs();
   for (void* p : allocations) (void)hipFree(p);
   allocations.clear();
-  rows.release();
-  if (h_status) (void)hipHostFree(h_status);
+  if (h_status) rows->give_back(h_status);
   h_status = nullptr;
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
@@ -135,7 +134,8 @@ int grains_gpu_system::allocate() {
   HIPCHECK(this, track(this, &d_obs, obstacles.size()));
   HIPCHECK(this, track(this, &d_models, (size_t)kMaxMaterials * kMaxMaterials));
   HIPCHECK(this, track(this, &d_status, 1));
-  HIPCHECK(this, hipHostMalloc((void**)&h_status, sizeof(DevStatus), hipHostMallocDefault));
+  rows = RowBuffers::of(device);
+  h_status = rows->status_block();
   if (verlet)
     for (int a = 0; a < 3; ++a) HIPCHECK(this, track(this, &V.xb[a], n));
   V.sync = nullptr;
@@ -1253,7 +1253,7 @@ int grains_gpu_set_hydro_ft(grains_gpu_system* s, const double* ft, size_t m) {
   for (int c = 0; c < 6; ++c) comps[c] = s->d_hyd + (size_t)c * n;
   RowIO io(n);
   io.add(ft, comps, 6);
-  HIPCHECK(s, s->rows.up(io, s->P.id, n, s->device, s->stream));
+  HIPCHECK(s, s->rows->up(io, s->P.id, n, s->stream));
   HIPCHECK(s, hipStreamSynchronize(s->stream));
   // step graphs captured before hold StepParams without the fluid forces
   if (fresh) s->drop_graphs();
@@ -1296,7 +1296,7 @@ int grains_gpu_get_state(grains_gpu_system* s, double* x, double* v, double* w, 
   // the status comes back with the rows
   int e = s->fetch_status();
   if (e) return e;
-  HIPCHECK(s, s->rows.down(io, s->P.id, n, s->device, s->stream));
+  HIPCHECK(s, s->rows->down(io, s->P.id, n, s->stream));
   return s->read_status();
 }
 
@@ -1307,7 +1307,7 @@ int grains_gpu_get_basis(grains_gpu_system* s, double* B) {
   const int n = s->nparticles;
   RowIO io(n);
   io.add(B, s->P.B[s->cur & 1], 9);
-  HIPCHECK(s, s->rows.down(io, s->P.id, n, s->device, s->stream));
+  HIPCHECK(s, s->rows->down(io, s->P.id, n, s->stream));
   return s->check_status();
 }
 
@@ -1318,7 +1318,7 @@ int grains_gpu_set_basis(grains_gpu_system* s, const double* B) {
   const int n = s->nparticles;
   RowIO io(n);
   io.add(B, s->P.B[s->cur & 1], 9);
-  HIPCHECK(s, s->rows.up(io, s->P.id, n, s->device, s->stream));
+  HIPCHECK(s, s->rows->up(io, s->P.id, n, s->stream));
   HIPCHECK(s, hipStreamSynchronize(s->stream));
   return GRAINS_OK;
 }
@@ -1334,7 +1334,7 @@ int grains_gpu_set_state(grains_gpu_system* s, const double* x, const double* v,
   io.add(v, s->P.v[cv], 3);
   io.add(w, s->P.w[cv], 3);
   io.add(q, s->P.q, 4);
-  HIPCHECK(s, s->rows.up(io, s->P.id, n, s->device, s->stream));
+  HIPCHECK(s, s->rows->up(io, s->P.id, n, s->stream));
   // the body-fixed angular velocity follows w and q, given or kept
   HIPCHECK(s, launch_body_spin(s->P, n, cv, s->stream));
   int e = s->bin_current();

@@ -147,7 +147,7 @@ struct grains_gpu_system {
     v.stamp = verlet ? st : 0;
     return v;
   }
-  dem::RowBuffers rows;               // buffers of the state transfers
+  std::shared_ptr<dem::RowBuffers> rows;  // buffers of the state transfers
   dem::DevStatus* h_status = nullptr;  // pinned: the status block comes back without a staging copy
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -8,6 +8,7 @@ import ctypes
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -92,6 +93,26 @@ def test_basis_rows(gpu, n):
     assert np.array_equal(g.basis().reshape(n, 9), B[::-1])
 
 
+def test_systems_of_several_threads(gpu):
+    # the buffers are shared: transfers of one chunk and of many, set and
+    # fetched from threads at once, the first of them growing the buffers
+    sizes = (40, 5000, 30000, 120000)
+
+    def work(n):
+        g, x = sparse(n)
+        rng = np.random.default_rng(n)
+        for _ in range(10):
+            v, w = rng.normal(size=(n, 3)), rng.normal(size=(n, 3))
+            g.set_state(v=v, w=w)
+            s = g.state()
+            if not (np.array_equal(s["v"], v) and np.array_equal(s["w"], w) and np.array_equal(s["x"], x)):
+                return n
+        return 0
+
+    with ThreadPoolExecutor(4) as pool:
+        assert list(pool.map(work, sizes)) == [0] * 4
+
+
 # hipMalloc and hipHostMalloc as the library finds them: they have no room for
 # requests of `room` bytes or more once told so
 SHIM = r"""
@@ -118,6 +139,8 @@ shim.leave.argtypes = [ctypes.c_size_t] * 2
 import numpy as np
 from tests.test_gpu_rows import sparse
 n, every = int(sys.argv[2]), 2 ** 64 - 1
+if sys.argv[3] == "host":
+    shim.leave(every, 0)
 g, x = sparse(n)
 h, _ = sparse(n)
 rng = np.random.default_rng(n)
