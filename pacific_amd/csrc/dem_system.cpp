@@ -391,6 +391,7 @@ int grains_gpu_system::bin_current() {
     HIPCHECK(this, launch_key(P, S, grid, sp, d_status, vstate(-1), stream));
     HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), touch.count, false,
                                        stream));
+    list_current = true;
     return GRAINS_OK;
   }
   HIPCHECK(this, launch_key(P, S, grid, sp, d_status, vstate(0), stream));
@@ -503,6 +504,7 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     HIPCHECK(this, launch_forces_solo(mode, cfg.precision == GRAINS_MIXED, P, S, grid, d_obs, d_models, sp, d_status,
                                       d_pairs, L, vstate(1), stream));
     if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
+    list_current = mode != kModeFused;
     if (commit && mem.cap) mem.cur ^= 1;
     if (mode == kModeForcesKick) cur ^= 2;
     if (mode == kModeFused) {
@@ -511,7 +513,8 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     }
     return GRAINS_OK;
   }
-  if (solo)  // an evaluation of the general sweep: the list must be current
+  // an evaluation of the general sweep: the list must be current
+  if (solo && !list_current)
     HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, L, touch.count, true, stream));
   const dem::NbrList CL = contact_list();
   // (not for evaluations outside the step loop, nor with extras)
@@ -527,6 +530,7 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
                                d_pairs, L, vstate(1), CL, TL, stream));
   if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
   if (sp.stats) HIPCHECK(this, launch_stats_fold(d_stat_part, nparticles, d_stat_tot, force_time, stream));
+  list_current = mode != kModeFused;
   // the evaluation wrote the other memory buffer: it becomes current
   if (commit && mem.cap) mem.cur ^= 1;
   if (mode == kModeForcesKick) cur ^= 2;
@@ -567,6 +571,7 @@ int grains_gpu_system::enqueue_steps_impl(int nsteps) {
     force_time = time;
     HIPCHECK(this, launch_move(P, S, grid, sp, d_status, 0.5 * cfg.dt, cfg.dt, vstate(1), ++step_number,
                                stream));
+    list_current = false;
     if ((e = bin_launch())) return e;
     if (recording && (e = record_state())) return e;
     int i = 1;

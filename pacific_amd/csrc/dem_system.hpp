@@ -139,6 +139,9 @@ struct grains_gpu_system {
   // neighbours and 64 obstacles
   static constexpr int kSoloMax = 65536;
   bool solo = false;
+  // no drift since the list was built or found current (systems whose force
+  // sweep rebuilds it: an evaluation of the general sweep rebuilds it unless)
+  bool list_current = false;
   // the number of the last positions written (DevStatus::seq counts along on
   // the device, so that captured steps need no new arguments)
   int step_number = 0;
