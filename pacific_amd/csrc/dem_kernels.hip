@@ -249,12 +249,13 @@ __global__ __launch_bounds__(256) void k_canon(Particles P, Sorted S, int cx, in
 // every neighbour candidate of each sorted particle that passes the
 // conservative distance reject of the narrow phase, in the order the force
 // sweep visits them, written to the candidate list; the force sweep then reads
-// a short list instead of 27 cells.  kDetectLanes lanes share a particle and
-// test that many consecutive candidates at once (the accepted ones numbered by
-// a ballot): one lane alone waits for its candidates' loads one after the
-// other (46.8 us per launch for 343 polyhedra, whose 27 cells hold about 96
-// bodies each; 21.6 us with eight, work list included, and 101 us instead of
-// 123 for 200,000 -- a launch of its own wrote the work list in 59 us).
+// a short list instead of 27 cells.  LANES lanes share a particle and test that
+// many consecutive candidates at once (the accepted ones numbered by a ballot):
+// one lane alone waits for its candidates' loads one after the other, which few
+// particles have nothing to fill with (46.8 us per launch for 343 polyhedra,
+// whose 27 cells hold about 96 bodies each; 21.6 us with eight, work list
+// included; a launch of its own wrote the work list of 200,000 in 59 us).  The
+// rule and its figures stand at launch_detect.
 // ITEMS (systems with non-spherical bodies): each listed slot's contact
 // record starts as kNoFeat, so that the narrow phase writes only contacts, and
 // the evaluations the narrow phase has to make are appended to its work list:
@@ -264,11 +265,10 @@ __global__ __launch_bounds__(256) void k_canon(Particles P, Sorted S, int cx, in
 // After an error raised on the device (which ends the run) the contact
 // searches return at once, so that the rest of a batch of steps costs
 // little whatever the state has become.
-constexpr int kDetectLanes = 8;
 constexpr int kItemBuf = 1024;  // items a workgroup collects before it appends them
 
-template <bool ITEMS>
-__global__ __launch_bounds__(kDetectLanes * kDetectBodies) void k_detect(Particles P, Sorted S, Grid G,
+template <bool ITEMS, int LANES>
+__global__ __launch_bounds__(kDetectThreads) void k_detect(Particles P, Sorted S, Grid G,
                                                                          const BoxObstacle* __restrict__ obs,
                                                                          StepParams sp, NbrList L,
                                                                          const DevStatus* st) {
@@ -276,9 +276,9 @@ __global__ __launch_bounds__(kDetectLanes * kDetectBodies) void k_detect(Particl
   __shared__ int nbuf, base;
   if (st->code) return;
   const int n = sp.n;
-  const int lane = threadIdx.x & (kDetectLanes - 1);
-  const int gshift = threadIdx.x & 63 & ~(kDetectLanes - 1);
-  const int k = xcd_tile(blockIdx.x, gridDim.x) * kDetectBodies + threadIdx.x / kDetectLanes;
+  const int lane = threadIdx.x & (LANES - 1);
+  const int gshift = threadIdx.x & 63 & ~(LANES - 1);
+  const int k = xcd_tile(blockIdx.x, gridDim.x) * (kDetectThreads / LANES) + threadIdx.x / LANES;
   if (ITEMS) {
     if (threadIdx.x == 0) nbuf = 0;
     __syncthreads();
@@ -301,8 +301,26 @@ __global__ __launch_bounds__(kDetectLanes * kDetectBodies) void k_detect(Particl
       else items[atomicAdd(nitems, 1)] = it;
     };
     int c = 0;
+    if constexpr (LANES == 1 && !ITEMS) {
+      // one candidate at a time: at this register count eight waves per SIMD
+      // overlap the loads better than wider batches of loads per thread do
+      for_each_candidate(S, G, 0, 0, n, x, [&](int k2, int ix, int iy, int iz) {
+        if (k2 == k) return;
+        const double* q2 = S.posr + 4 * (size_t)k2;
+        const d3 xo{ix ? q2[0] + image_shift(G, 0, ix) : q2[0], iy ? q2[1] + image_shift(G, 1, iy) : q2[1],
+                    iz ? q2[2] + image_shift(G, 2, iz) : q2[2]};
+        const d3 AB = xo - x;
+        const double s2 = AB.x * AB.x + AB.y * AB.y + AB.z * AB.z;
+        const double R = r + q2[3];
+        if (s2 > R * R * 1.000000000001) return;
+        if (c < L.cap) L.ent[(size_t)c * n + k] = nbr_entry(k2, ix, iy, iz);
+        ++c;
+      });
+      L.count[k] = c;
+      return;
+    }
     for_each_run(S, G, 0, 0, n, x, [&](int b, int e, int ix, int iy, int iz) {
-      for (int k0 = b; k0 < e; k0 += kDetectLanes) {
+      for (int k0 = b; k0 < e; k0 += LANES) {
         const int k2 = k0 + lane;
         bool hit = k2 < e && k2 != k;
         if (hit) {
@@ -314,7 +332,7 @@ __global__ __launch_bounds__(kDetectLanes * kDetectBodies) void k_detect(Particl
           const double R = r + q2[3];
           hit = !(s2 > R * R * 1.000000000001);
         }
-        const unsigned hits = (unsigned)(__ballot(hit) >> gshift) & ((1u << kDetectLanes) - 1u);
+        const unsigned hits = LANES == 1 ? (unsigned)hit : (unsigned)(__ballot(hit) >> gshift) & ((1u << LANES) - 1u);
         const int j = c + __popc(hits & ((1u << lane) - 1u));
         if (hit && j < L.cap) {
           const unsigned e2 = nbr_entry(k2, ix, iy, iz);
@@ -336,7 +354,7 @@ __global__ __launch_bounds__(kDetectLanes * kDetectBodies) void k_detect(Particl
     if (ITEMS) {
       int last = -1;
       if (body && c <= L.cap)
-        for (int o0 = 0; o0 < sp.nobs; o0 += kDetectLanes) {
+        for (int o0 = 0; o0 < sp.nobs; o0 += LANES) {
           const int o = o0 + lane;
           bool met = false;
           if (o < sp.nobs) {
@@ -344,12 +362,12 @@ __global__ __launch_bounds__(kDetectLanes * kDetectBodies) void k_detect(Particl
             met = fabs(B.aabb_c[0] - x.x) <= B.aabb_e[0] + r && fabs(B.aabb_c[1] - x.y) <= B.aabb_e[1] + r &&
                   fabs(B.aabb_c[2] - x.z) <= B.aabb_e[2] + r;
           }
-          const unsigned hits = (unsigned)(__ballot(met) >> gshift) & ((1u << kDetectLanes) - 1u);
+          const unsigned hits = LANES == 1 ? (unsigned)met : (unsigned)(__ballot(met) >> gshift) & ((1u << LANES) - 1u);
           if (met && c + o < sp.cf.cap) append((unsigned)(c + o) | ((unsigned)kNbrNoShift << kNbrSlotBits), -1 - o);
           if (hits) last = o0 + 31 - __builtin_clz(hits);
         }
       // every obstacle slot the force sweep will read, met or not, starts empty
-      for (int o = lane; o <= last; o += kDetectLanes)
+      for (int o = lane; o <= last; o += LANES)
         if (c + o < sp.cf.cap) sp.cf.ent[(size_t)(c + o) * n + k] = kNoFeat;
       // a body without a usable list: -1, k_narrow_full searches its cells
       if (lane == 0) sp.cf.count[k] = !body ? 0 : (c > L.cap ? -1 : c + last + 1);
@@ -360,7 +378,7 @@ __global__ __launch_bounds__(kDetectLanes * kDetectBodies) void k_detect(Particl
     const int m = min(nbuf, kItemBuf);
     if (threadIdx.x == 0) base = m ? atomicAdd(nitems, m) : 0;
     __syncthreads();
-    for (int i = threadIdx.x; i < m; i += kDetectLanes * kDetectBodies) items[base + i] = buf[i];
+    for (int i = threadIdx.x; i < m; i += kDetectThreads) items[base + i] = buf[i];
   }
 }
 
@@ -619,12 +637,29 @@ hipError_t launch_vfilter(const Particles& P, const Sorted& S, const Grid& G, co
   return hipGetLastError();
 }
 
+template <int LANES>
+static void launch_detect_lanes(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
+                                const StepParams& sp, const NbrList& L, const DevStatus* st, hipStream_t stream) {
+  const dim3 grid(nblk(sp.n, kDetectThreads / LANES)), block(kDetectThreads);
+  if (P.shape) hipLaunchKernelGGL((k_detect<true, LANES>), grid, block, 0, stream, P, S, G, obs, sp, L, st);
+  else hipLaunchKernelGGL((k_detect<false, LANES>), grid, block, 0, stream, P, S, G, obs, sp, L, st);
+}
+
 hipError_t launch_detect(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
                          const StepParams& sp, const NbrList& L, const DevStatus* st, hipStream_t stream) {
   if (sp.n == 0) return hipSuccess;
-  const dim3 grid(nblk(sp.n, kDetectBodies)), block(kDetectLanes * kDetectBodies);
-  if (P.shape) hipLaunchKernelGGL(k_detect<true>, grid, block, 0, stream, P, S, G, obs, sp, L, st);
-  else hipLaunchKernelGGL(k_detect<false>, grid, block, 0, stream, P, S, G, obs, sp, L, st);
+  // lanes per particle by the number of particles, as measured (us per launch;
+  // 1, 2, 4, 8 lanes): packed polyhedra 343 75, 44, 30, 22; 27,000 45, 29, 22, 20;
+  // 200,000 94, 88, 83, 101; polyhedra on a loose lattice 20,000 17, 16, 14, 15;
+  // 60,000 18, 18, 17, 26; 200,000 23, 33, 40, 66; packed spheres 60,000 21, 18,
+  // 17, 21, 200,000 25, 26, 32, 52; gas of 27,000 23, 23, 22, 22, of 60,000
+  // at solid fraction 0.05 18, 18, 19, 22, of 1,000,000 74, 108, 151, 258.  More
+  // lanes overlap the loads of few particles; once there are particles enough,
+  // every lane repeats the search for the cells' runs for little.
+  const bool items = P.shape != nullptr;
+  if (sp.n <= 32768) launch_detect_lanes<8>(P, S, G, obs, sp, L, st, stream);
+  else if (sp.n <= (items ? 65536 : 49152)) launch_detect_lanes<4>(P, S, G, obs, sp, L, st, stream);
+  else launch_detect_lanes<1>(P, S, G, obs, sp, L, st, stream);
   return hipGetLastError();
 }
 

@@ -38,8 +38,9 @@ hipError_t launch_stats_fold(const double* part, int n, double* tot, double time
 // with non-spherical bodies, the narrow phase's work list into sp.cf
 hipError_t launch_detect(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
                          const StepParams& sp, const NbrList& L, const DevStatus* st, hipStream_t stream);
-// bodies per workgroup of the detection that writes a work list
-constexpr int kDetectBodies = 32;
+// threads of a workgroup of the contact search, and bodies at most (its work
+// list is sized for any number of lanes per body)
+constexpr int kDetectThreads = 256;
 // narrow phase of a system with non-spherical bodies: the contacts of every
 // sorted particle (candidates of L, or its 27 cells when L.count is null)
 // into sp.cf, and the contact statistics when sp.stats is set

@@ -172,8 +172,8 @@ int grains_gpu_system::allocate() {
     HIPCHECK(this, hipMemsetAsync(cf.count, 0, sizeof(int) * n, stream));
     cf.cap = (int)fcap;
     cf.n = (int)n;
-    const size_t blocks = (n + kDetectBodies - 1) / kDetectBodies;
-    cf.item_stride = (int)((blocks + kItemLists - 1) / kItemLists * kDetectBodies * fcap);
+    const size_t blocks = (n + kDetectThreads - 1) / kDetectThreads;
+    cf.item_stride = (int)((blocks + kItemLists - 1) / kItemLists * kDetectThreads * fcap);
     HIPCHECK(this, track(this, &cf.items, (size_t)kItemLists * cf.item_stride));
     HIPCHECK(this, track(this, &cf.nitems, (size_t)kItemLists * kItemPad));
     HIPCHECK(this, hipMemsetAsync(cf.nitems, 0, sizeof(int) * kItemLists * kItemPad, stream));
