@@ -37,16 +37,36 @@ constexpr int kSoloBodies = 64;
 // pieces taken earlier, whose workgroups are running and wait for still earlier
 // ones, so the first piece not yet done never waits and all end, whatever share
 // of the launch is resident.
+// A piece is published by one wave for the workgroup, and its predecessors'
+// are taken up by one wave, once per phase: every agent-scope fence writes back
+// or invalidates the XCD's L2, and with a fence per wave and piece they were
+// what a rebuild waited for (a step of a gas of 64,000 that rebuilds every
+// fourth or fifth time 87 us, 70 with one).  The stores of all waves have reached the L2
+// (s_waitcnt) before the barrier, so the one write-back covers them; the count
+// is raised when it has ended, which is waited for explicitly: with no store
+// of this wave outstanding the compiler leaves that wait out.
+__device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void wait_pieces(int* done, int count) {
-  if (threadIdx.x == 0)
-    while (__hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < count) __builtin_amdgcn_s_sleep(2);
+  if (threadIdx.x == 0) {
+    // (hundreds of waiting workgroups that ask often hold up the counts)
+    while (__hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < count) {
+      if (gridDim.x > 256) __builtin_amdgcn_s_sleep(16);
+      else __builtin_amdgcn_s_sleep(2);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    drain();
+  }
   __syncthreads();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 __device__ __forceinline__ void piece_done(int* done) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  drain();
   __syncthreads();
-  if (threadIdx.x == 0) __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    drain();
+    __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // inclusive sum over the workgroup (kSoloThreads lanes); total of all lanes
@@ -68,10 +88,14 @@ __device__ __forceinline__ int block_sum_scan(int v, int* lds, int& total) {
   return incl;
 }
 
-constexpr int kPieceBodies = 4 * kSoloThreads;   // phases over particles
-constexpr int kPieceCells = 8 * kSoloThreads;    // phases over cells
-constexpr int kSearchLanes = 8;                  // lanes per particle of the neighbour phase
-constexpr int kPieceSearch = 4 * kSoloThreads / kSearchLanes;
+// Small pieces fill the chip, but each is published with a write-back of its
+// XCD's L2: about 250 pieces of the neighbour phase at most (us per step that
+// rebuilds every fourth or fifth time, of a gas of 8,000, 27,000 and 64,000: 25,
+// 37 and 59; four times as many 25, 42 and 79; 1,024 particles to every piece of
+// the other phases and 128 to those of this one 33, 47 and 70).
+constexpr int kPieceStep = 16384;              // particles per round of a piece's threads
+constexpr int kPieceCells = 8 * kSoloThreads;  // phases over cells
+constexpr int kSearchLanes = 4;                // lanes per particle of the neighbour phase
 
 __device__ __forceinline__ void solo_rebuild(const Particles& P, const Sorted& S, const VerletState& V, const NbrList& L,
                                           int n, int cx, DevStatus* st) {
@@ -79,8 +103,10 @@ __device__ __forceinline__ void solo_rebuild(const Particles& P, const Sorted& S
   RebuildSync* const rs = V.sync + cx;
   const Grid& G = V.Gv;
   const int tid = threadIdx.x;
-  const int nb = (n + kPieceBodies - 1) / kPieceBodies, nc = (G.ncells + kPieceCells - 1) / kPieceCells;
-  const int count[6] = {nb, nc, nc, nb, nb, (n + kPieceSearch - 1) / kPieceSearch};
+  const int rounds = 1 + n / kPieceStep, bodies = rounds * kSoloThreads, search = bodies / kSearchLanes;
+  const int nb = (n + bodies - 1) / bodies, nc = (G.ncells + kPieceCells - 1) / kPieceCells;
+  const int count[6] = {nb, nc, nc, nb, nb, (n + search - 1) / search};
+  int seen = 0;  // pieces of this phase were waited for
   for (;;) {
     __syncthreads();
     if (tid == 0) ticket = __hip_atomic_fetch_add(&rs->ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -88,11 +114,14 @@ __device__ __forceinline__ void solo_rebuild(const Particles& P, const Sorted& S
     int i = ticket, phase = 0;
     while (phase < 6 && i >= count[phase]) i -= count[phase++];
     if (phase == 6) break;
-    if (phase > 0) wait_pieces(&rs->done[phase - 1], count[phase - 1]);
+    if (phase > seen) {
+      wait_pieces(&rs->done[phase - 1], count[phase - 1]);
+      seen = phase;
+    }
     if (phase == 0) {
       // cell keys on the list's grid, build positions
       if (i == 0 && tid == 0) atomicAdd(&st->n_rebuild, 1);
-      for (int s = i * kPieceBodies + tid; s < min((i + 1) * kPieceBodies, n); s += kSoloThreads) {
+      for (int s = i * bodies + tid; s < min((i + 1) * bodies, n); s += kSoloThreads) {
         const double x[3] = {P.x[cx][0][s], P.x[cx][1][s], P.x[cx][2][s]};
         int c[3];
 #pragma unroll
@@ -134,18 +163,18 @@ __device__ __forceinline__ void solo_rebuild(const Particles& P, const Sorted& S
         if (i == 0 && tid == 0) S.start[G.ncells] = n;
       }
     } else if (phase == 3) {
-      for (int s = i * kPieceBodies + tid; s < min((i + 1) * kPieceBodies, n); s += kSoloThreads) {
+      for (int s = i * bodies + tid; s < min((i + 1) * bodies, n); s += kSoloThreads) {
         const int dst = S.start[S.key[s]] + S.slot[s];
         if ((unsigned)dst < (unsigned)n) S.tmp_order[dst] = s;
       }
     } else if (phase == 4) {
-      for (int j = i * kPieceBodies + tid; j < min((i + 1) * kPieceBodies, n); j += kSoloThreads)
+      for (int j = i * bodies + tid; j < min((i + 1) * bodies, n); j += kSoloThreads)
         rank_particle(P, S, j, cx, n);
     } else {
       // neighbours within the contact distance plus the skin, kSearchLanes
       // candidates at a time in the order of the cells
       const int lane = tid & (kSearchLanes - 1), gshift = tid & 63 & ~(kSearchLanes - 1);
-      for (int k = i * kPieceSearch + tid / kSearchLanes; k < min((i + 1) * kPieceSearch, n);
+      for (int k = i * search + tid / kSearchLanes; k < min((i + 1) * search, n);
            k += kSoloThreads / kSearchLanes) {
         const int s = S.order[k];
         if ((unsigned)s >= (unsigned)n) continue;
