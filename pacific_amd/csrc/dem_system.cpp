@@ -139,7 +139,9 @@ int grains_gpu_system::allocate() {
   if (verlet)
     for (int a = 0; a < 3; ++a) HIPCHECK(this, track(this, &V.xb[a], n));
   V.sync = nullptr;
-  solo = verlet && n > 0 && n <= (size_t)kSoloMax && nbr_cap <= 64 && obstacles.size() <= 64;
+  solo = verlet && n > 0 && n <= (size_t)kSoloMax && nbr_cap >= kSoloCap && nbr_cap <= 64 &&
+         obstacles.size() <= 64;
+  busy = false;
   if (solo) {
     HIPCHECK(this, track(this, &V.sync, 2));
     HIPCHECK(this, hipMemsetAsync(V.sync, 0, 2 * sizeof(RebuildSync), stream));
@@ -392,6 +394,7 @@ int grains_gpu_system::bin_current() {
     HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), touch.count, false,
                                        stream));
     list_current = true;
+    ++builds_seen;
     return GRAINS_OK;
   }
   HIPCHECK(this, launch_key(P, S, grid, sp, d_status, vstate(0), stream));
@@ -416,6 +419,20 @@ bool grains_gpu_system::scattered() const {
     far += f;
   }
   return 2 * far > seen;
+}
+
+// Whether velocities v (by id) make the Verlet list of a system near the size
+// limit stale so often that the general launches rebuild it: some particle of a
+// sample crosses half the skin in fewer than kBusyRate steps.  Measured rates
+// take over once steps have been made (read_status).
+void grains_gpu_system::expect_rebuilds(const double* v) {
+  if (!solo || nparticles <= kBusyMin) return;
+  const double reach = 0.5 * V.skin / (kBusyRate * cfg.dt);
+  busy = false;
+  for (int i = 0; i < nparticles && !busy; i += std::max(1, nparticles / 2048)) {
+    const double* u = v + 3 * (size_t)i;
+    busy = u[0] * u[0] + u[1] * u[1] + u[2] * u[2] > reach * reach;
+  }
 }
 
 // Stores the particles in the order of the cells they were just binned in
@@ -461,12 +478,13 @@ int grains_gpu_system::mark(std::vector<hipEvent_t>& evs, size_t& n) {
 int grains_gpu_system::bin_launch() {
   int e;
   if (prof && (e = mark(prof->bin_ev, prof->nbin))) return e;
-  if (solo)
-    ;  // the force sweep rebuilds the list itself
-  else if (verlet)
+  if (one_launch()) {
+    // the force sweep rebuilds the list itself
+  } else if (verlet) {
     HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), touch.count, true,
                                        stream));
-  else
+    list_current = true;
+  } else
     HIPCHECK(this, launch_bin(P, S, grid, nparticles, cur & 1, stream));
   if (prof && (e = mark(prof->bin_ev, prof->nbin))) return e;
   return GRAINS_OK;
@@ -498,7 +516,7 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     HIPCHECK(this, launch_narrow(P, S, grid, d_obs, sp, d_status, L, stream));
     if (prof && (e = mark(prof->narrow_ev, prof->nnarrow))) return e;
   }
-  if (solo && !sp.stats && !sp.fsum) {
+  if (one_launch() && !sp.stats && !sp.fsum) {
     // one launch: list rebuild if stale, contacts, forces, integration
     if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
     HIPCHECK(this, launch_forces_solo(mode, cfg.precision == GRAINS_MIXED, P, S, grid, d_obs, d_models, sp, d_status,
@@ -514,7 +532,7 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     return GRAINS_OK;
   }
   // an evaluation of the general sweep: the list must be current
-  if (solo && !list_current)
+  if (verlet && !list_current)
     HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, L, touch.count, true, stream));
   const dem::NbrList CL = contact_list();
   // (not for evaluations outside the step loop, nor with extras)
@@ -634,7 +652,7 @@ int grains_gpu_system::graph_chunk(bool& done) {
     drop_graphs();
     graph_dt = cfg.dt;
   }
-  const int key = (cur & 3) | ((mem.cur & 1) << 2);
+  const int key = (cur & 3) | ((mem.cur & 1) << 2) | (one_launch() ? 8 : 0);
   for (auto& g : graphs)
     if (g.first == key) {
       for (int j = 0; j < kGraphSteps; ++j) force_time += cfg.dt;
@@ -693,6 +711,11 @@ int grains_gpu_system::check_status() {
 int grains_gpu_system::read_status() {
   const DevStatus st = *h_status;
   last_status = st;
+  if (solo && steps_done - steps_seen >= kBusySteps) {
+    busy = kBusyRate * (st.n_rebuild - builds_seen) > steps_done - steps_seen;
+    builds_seen = st.n_rebuild;
+    steps_seen = steps_done;
+  }
   if (st.code) {
     static const char* names[] = {"", "ContactError", "MotionError", "SimulationError"};
     char buf[160];
@@ -744,6 +767,7 @@ int grains_gpu_system::initialize() {
   if ((e = upload())) return e;
   if ((e = bin_current())) return e;
   if (scattered() && (e = sort_storage())) return e;
+  expect_rebuilds(h_v.data());
   initialized = true;
   // LeapFrog: accelerations at the initial time (Grains.cpp:169-174)
   if (cfg.scheme == GRAINS_LEAPFROG) {
@@ -1342,6 +1366,7 @@ int grains_gpu_set_state(grains_gpu_system* s, const double* x, const double* v,
   HIPCHECK(s, s->rows->up(io, s->P.id, n, s->stream));
   // the body-fixed angular velocity follows w and q, given or kept
   HIPCHECK(s, launch_body_spin(s->P, n, cv, s->stream));
+  if (v) s->expect_rebuilds(v);
   int e = s->bin_current();
   if (e) return e;
   if (recompute_forces) {

@@ -134,13 +134,28 @@ struct grains_gpu_system {
   double* d_stat_tot = nullptr;
   double force_time = 0.;
   // systems whose force sweep also rebuilds the Verlet list and finds the
-  // contacts in it, one launch per step (k_forces_solo: faster up to this many
-  // spheres in beds and gases alike, figures there); its masks hold 64 listed
-  // neighbours and 64 obstacles
-  static constexpr int kSoloMax = 65536;
+  // contacts in it, one launch per step (k_forces_solo, figures there).  Its
+  // masks hold 64 listed neighbours and 64 obstacles; lists of fewer than
+  // kSoloCap entries, which packings overflow, are searched sooner by the
+  // general launches (three entries, us per step: bed of 1,000 118 against 82,
+  // of 48,000 84 against 72).  Beds gain above kSoloMax as well (100,000: 56
+  // against 71 us), gases do not (110,000: 47.8 against 43.7), and what a system
+  // is may change: one limit, the gases', for both.
+  static constexpr int kSoloMax = 65536, kSoloCap = 16;
   bool solo = false;
-  // no drift since the list was built or found current (systems whose force
-  // sweep rebuilds it: an evaluation of the general sweep rebuilds it unless)
+  // ... unless a list of more than kBusyMin particles goes stale more often
+  // than every kBusyRate steps: the rebuild inside the sweep is the slower one,
+  // with few workgroups (gas that rebuilds every fourth or fifth time, us per
+  // step: 27,000 37 against 46, 48,000 56 against 50, 64,000 59 against 50; every
+  // 28th: 48,000 22 against 37, 64,000 28 against 37)
+  static constexpr int kBusyMin = 32768, kBusyRate = 10, kBusySteps = 32;
+  bool busy = false;
+  int builds_seen = 0;
+  long steps_seen = 0;
+  bool one_launch() const { return solo && !(busy && nparticles > kBusyMin); }
+  void expect_rebuilds(const double* v);
+  // no drift since the Verlet list was built or found current (an evaluation of
+  // the general sweep finds out unless)
   bool list_current = false;
   // the number of the last positions written (DevStatus::seq counts along on
   // the device, so that captured steps need no new arguments)

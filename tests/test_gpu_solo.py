@@ -196,3 +196,47 @@ def test_general_evaluation_between_one_launch_steps(gpu, scheme):
         h.set_state(**{f: s[f] for f in ("x", "v", "w", "q")})
         b = h.force_sums()
         assert b.max() > 0 and np.max(np.abs(a - b)) <= 1e-12 * b.max()
+
+
+@pytest.mark.parametrize("precision", [0, MIXED])
+@pytest.mark.parametrize("with_memory", [False, True])
+def test_list_too_short_for_some(gpu, precision, with_memory):
+    # large spheres among small ones: more neighbours than a list of 16 holds
+    wl = memory(2000) if with_memory else bed(2000)
+    big = np.arange(50, 2000, 333)
+    near = np.linalg.norm(wl["x"][:, None] - wl["x"][big][None], axis=2) < 3.9e-3
+    keep = ~near.any(1)
+    keep[big] = True
+    for k in ("radius", "density", "crust", "material", "x", "v", "w"):
+        wl[k] = np.asarray(wl[k])[keep]
+    wl["radius"] = np.where(np.isin(np.flatnonzero(keep), big), 2.9995e-3, 1e-3)
+    wl["x"] = wl["x"] + np.array([2e-3, 2e-3, 2e-3])
+    wl["max"] = (0.03, 0.03, 0.3)
+    wl["boxes"] = []
+    a, builds_a = run(wl, precision, 16, False, (40, 1, 2))
+    b, builds_b = run(wl, precision, 16, True, (40, 1, 2))
+    assert builds_a == builds_b
+    for f in ("x", "v", "w", "F", "T"):
+        assert np.array_equal(a[f], b[f]), f
+
+
+@pytest.mark.parametrize("precision", [0, MIXED])
+def test_rebuilds_often_and_seldom(gpu, precision):
+    # near the size limit a system whose list goes stale often steps by the
+    # general launches, as its velocities and then its rebuilds say: slow, made
+    # fast from outside, slow again, over graph replays and single steps
+    wl = gas(40001)
+    slow = dict(wl, v=wl["v"] * 0.05)
+    a, b = make_gpu(slow, precision=precision, record=False), make_gpu(slow, precision=precision, record=False, stats=True)
+    for v in (None, wl["v"], slow["v"]):
+        for k in (70, 1, 2, 70):
+            if v is not None and k == 70:
+                for s in (a, b):
+                    s.set_state(v=v)
+            a.step(k)
+            b.step(k)
+        sa, sb = a.state(), b.state()
+        for f in ("x", "v", "w", "F", "T"):
+            assert np.array_equal(sa[f], sb[f]), f
+        assert a.neighbor_stats() == b.neighbor_stats()
+    assert a.neighbor_stats()[1] > 20
