@@ -630,6 +630,20 @@ static void launch_forces_t(const Particles& P, const Sorted& S, const Grid& G, 
     launch_forces_sph<MODE, MIXED>(P, S, G, obs, models, sp, st, pairs, L, V, CL, TL, stream);
 }
 
+__global__ __launch_bounds__(256) void k_count_touched(const int* __restrict__ count, int n, int* touched) {
+  int c = 0;
+  for (int s = blockIdx.x * 256 + threadIdx.x; s < n; s += gridDim.x * 256) c += count[s] != 0;
+  for (int d = 32; d; d >>= 1) c += __shfl_down(c, d);
+  if ((threadIdx.x & 63) == 0 && c) atomicAdd(touched, c);
+}
+hipError_t launch_count_touched(const NbrList& CL, int n, int* touched, hipStream_t stream) {
+  if (n == 0) return hipSuccess;
+  hipError_t e = launch_clear(touched, 1, stream);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_count_touched, dim3(std::min(nblk(n, 256), 1024)), dim3(256), 0, stream, CL.count, n, touched);
+  return hipGetLastError();
+}
+
 hipError_t launch_vfilter(const Particles& P, const Sorted& S, const Grid& G, const VerletState& V, int n, int cx,
                           const NbrList& L, const NbrList& CL, const TouchList& TL, DevStatus* st, hipStream_t stream) {
   if (n == 0) return hipSuccess;

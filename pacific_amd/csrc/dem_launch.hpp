@@ -34,6 +34,8 @@ hipError_t launch_vfilter(const Particles& P, const Sorted& S, const Grid& G, co
 // folds the per-block contact statistics of the last force launch over n
 // particles into the running totals (6 doubles), at the given time
 hipError_t launch_stats_fold(const double* part, int n, double* tot, double time, hipStream_t stream);
+// particles with a contact in CL (of n) into *touched
+hipError_t launch_count_touched(const NbrList& CL, int n, int* touched, hipStream_t stream);
 // neighbour candidates of every sorted particle into L, and, for a system
 // with non-spherical bodies, the narrow phase's work list into sp.cf
 hipError_t launch_detect(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,

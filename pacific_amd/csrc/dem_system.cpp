@@ -187,13 +187,15 @@ int grains_gpu_system::allocate() {
   HIPCHECK(this, track(this, &d_stat_part, 5 * ((n + 255) / 256) + 5));
   HIPCHECK(this, track(this, &d_stat_tot, 8));
   HIPCHECK(this, hipMemsetAsync(d_stat_tot, 0, 8 * sizeof(double), stream));
-  // a touch list where nothing holds the particles together, neither weight
-  // nor walls, so that contacts are collisions and few, and where the state no
-  // longer fits the 256 MB cache, so that the sweep waits for memory and the
-  // wave of a contact holds up the others (us per step without and with it:
-  // gas of 110,000 32 and 41, of 400,000 63.5 and 64.8, of 600,000 87 and 81, of
-  // 1M 142 and 132; a settled bed of 200,000 80 and 95)
+  // a touch list where neither weight nor walls hold the particles together,
+  // so that contacts may be collisions and few, and where the state no longer
+  // fits the 256 MB cache, so that the sweep waits for memory and the wave of a
+  // contact holds up the others (us per step without and with it: gas of 110,000
+  // 32 and 41, of 400,000 63.5 and 64.8, of 600,000 87 and 81, of 1M 142 and 132).
+  // Whether contacts are few is counted (touch_few): 1M particles of which 1.5 %
+  // touch 112 and 108, 6 % 143 and 132, 12 % 186 and 195, all 246 and 395
   touch = dem::TouchList{};
+  touch_few = true;
   const bool gas = cfg.gravity[0] == 0. && cfg.gravity[1] == 0. && cfg.gravity[2] == 0. && obstacles.empty();
   if (verlet && gas && n > (size_t)kTouchMin && cfg.precision != GRAINS_MIXED) {
     const size_t blocks = (n + 255) / 256;
@@ -421,6 +423,13 @@ bool grains_gpu_system::scattered() const {
   return 2 * far > seen;
 }
 
+// The particles of the last evaluation that have a contact, for the choice of
+// the next batch's sweep (read_status).
+int grains_gpu_system::count_touched() {
+  if (touch.idx) HIPCHECK(this, launch_count_touched(contact_list(), nparticles, &d_status->n_touched, stream));
+  return GRAINS_OK;
+}
+
 // Whether velocities v (by id) make the Verlet list of a system near the size
 // limit stale so often that the general launches rebuild it: some particle of a
 // sample crosses half the skin in fewer than kBusyRate steps.  Measured rates
@@ -536,7 +545,8 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, L, touch.count, true, stream));
   const dem::NbrList CL = contact_list();
   // (not for evaluations outside the step loop, nor with extras)
-  const dem::TouchList TL = mode == kModeForcesOnly || sp.stats || sp.fsum || sp.mem.cap ? dem::TouchList{} : touch;
+  const dem::TouchList TL =
+      mode == kModeForcesOnly || sp.stats || sp.fsum || sp.mem.cap || !touch_few ? dem::TouchList{} : touch;
   if (CL.count) {
     // this step's contacts from the Verlet list
     if (prof && (e = mark(prof->detect_ev, prof->ndetect))) return e;
@@ -549,6 +559,7 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
   if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
   if (sp.stats) HIPCHECK(this, launch_stats_fold(d_stat_part, nparticles, d_stat_tot, force_time, stream));
   list_current = mode != kModeFused;
+  if (mode != kModeFused && (e = count_touched())) return e;
   // the evaluation wrote the other memory buffer: it becomes current
   if (commit && mem.cap) mem.cur ^= 1;
   if (mode == kModeForcesKick) cur ^= 2;
@@ -613,6 +624,7 @@ int grains_gpu_system::enqueue_steps_impl(int nsteps) {
       if ((e = forces(kModeFused, first))) return e;
       if ((e = bin_launch())) return e;
     }
+    if ((e = count_touched())) return e;
   }
   steps_done += nsteps;
   for (int i = 0; i < nsteps; ++i) time += cfg.dt;
@@ -652,7 +664,7 @@ int grains_gpu_system::graph_chunk(bool& done) {
     drop_graphs();
     graph_dt = cfg.dt;
   }
-  const int key = (cur & 3) | ((mem.cur & 1) << 2) | (one_launch() ? 8 : 0);
+  const int key = (cur & 3) | ((mem.cur & 1) << 2) | (one_launch() ? 8 : 0) | (touch_few ? 16 : 0);
   for (auto& g : graphs)
     if (g.first == key) {
       for (int j = 0; j < kGraphSteps; ++j) force_time += cfg.dt;
@@ -711,6 +723,7 @@ int grains_gpu_system::check_status() {
 int grains_gpu_system::read_status() {
   const DevStatus st = *h_status;
   last_status = st;
+  if (touch.idx) touch_few = (long)kTouchShare * st.n_touched < nparticles;
   if (solo && steps_done - steps_seen >= kBusySteps) {
     busy = kBusyRate * (st.n_rebuild - builds_seen) > steps_done - steps_seen;
     builds_seen = st.n_rebuild;

@@ -103,7 +103,9 @@ struct grains_gpu_system {
   // contacts of the current step filtered from the Verlet list
   static constexpr int kContactCap = 16;
   dem::TouchList touch{};  // the particles of a large gas that have a contact
-  static constexpr int kTouchMin = 500000;
+  static constexpr int kTouchMin = 500000, kTouchShare = 12;
+  bool touch_few = true;  // fewer than one in kTouchShare have one: the sweep goes by the list
+  int count_touched();
   int* d_ct_count = nullptr;
   unsigned* d_ct = nullptr;
   dem::NbrList contact_list() const {

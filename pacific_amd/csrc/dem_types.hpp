@@ -209,6 +209,7 @@ struct DevStatus {
   // that reads it, in which errors may be raised while workgroups start
   int stop[2];
   int n_rebuild;     // Verlet list builds
+  int n_touched;     // particles with a contact, as last counted (systems that may keep a touch list)
 };
 static_assert(offsetof(DevStatus, rebuild) / 128 != offsetof(DevStatus, npairs) / 128, "");
 

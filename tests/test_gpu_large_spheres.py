@@ -3,8 +3,9 @@ the general sweep, which a system that collects contact statistics runs: same
 lists, same order of the sums, so the same bits.  Packings with walls and
 weight, a last tile that is not full, uniform crust and coupling factor and
 not, both precisions, every scheme; a gas with a touch list, just above the
-size at which it is kept, with batches that end in a half kick and with a list
-too short for its neighbours (searched in their cells)."""
+size at which it is kept, with batches that end in a half kick, with a list
+too short for its neighbours (searched in their cells) and with as many
+particles in contact, later or from the start, as the list is not used for."""
 import numpy as np
 import pytest
 
