@@ -664,8 +664,8 @@ def main():
                    "contacts_per_particle": cbar, "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": "k_verlet32<fused>" if headline == MIXED else
-                     "k_forces_gas<fused>" if args.n > 500000 else "k_verlet64<fused>", "kernel_ms": force_ms,
+                     "kernel": "k_forces_solo<fused>" if args.n <= 65536 else "k_verlet32<fused>" if headline == MIXED
+                     else "k_forces_gas<fused>" if args.n > 500000 else "k_verlet64<fused>", "kernel_ms": force_ms,
                      "bytes_alg_per_launch": b_alg, "contacts_per_particle": cbar, "binning_ms": bin_ms,
                      "contact_filter_ms": detect_ms, "verlet_skin_m": skin, "verlet_builds": builds},
     }

@@ -29,8 +29,10 @@
 #include "dem_forces.hpp"
 #include "dem_launch.hpp"
 
-constexpr int kFilterGroup = 4;  // list entries in flight per particle (2: the same, 1: 33 us instead of 30.6 for the 1M gas)
 namespace dem {
+
+// list entries in flight per particle (2: the same, 1: 33 us instead of 30.6 for the 1M gas)
+constexpr int kFilterGroup = 4;
 
 // ---------------------------------------------------------------------------
 // First half kick + drift over storage indices (in place): Grains.cpp:353

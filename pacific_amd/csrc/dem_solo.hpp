@@ -18,14 +18,16 @@ namespace dem {
 // particle: the listed neighbours of a workgroup's particles are spread over
 // its lanes, one per lane, the force and torque of each contact left in LDS and
 // summed by the particle's thread in the list's order -- the sum of the general
-// sweep.  Pairs first, then obstacles, as there, each kind in waves of its own.
+// sweep, but for a law with a rolling moment, which joins its contact's torque
+// before that sum and not after it (one rounding of the torque per contact).
+// Pairs first, then obstacles, as there, each kind in waves of its own.
 // Bound by the latency of one contact and of the phases' barriers.  Per step,
-// general launches -> this one: bed of 1,000 41 -> 18.9 us, of 48,611 (mixed)
-// 39 -> 21, 5,003 with contact memory 72 -> 29, gas of 27,000 (mixed) 25.5 ->
-// 16.7, of 60,000 35.6 -> 29.4.  The general launches, with more waves on the
-// streaming part, are as fast or faster above (gas of 110,000 43.7 against
-// 47.8 us, of 200,000 49 against 73; bed of 100,000 71 against 56, of 200,000
-// 80 against 93), hence the limit grains_gpu_system::kSoloMax.
+// general launches -> this one: bed of 1,000 41 -> 18.8 us, of 48,611 (mixed)
+// 39 -> 20, 5,003 with contact memory 72 -> 29, gas of 27,000 37 -> 18, of 64,000
+// 37 -> 25.  Above, gases are as fast or faster by the general launches, with
+// more waves on the streaming part (110,000 43.7 against 47.8 us, 200,000 49
+// against 73), beds from somewhere above 100,000 (100,000 71 against 56, 200,000
+// 80 against 93); the rule stands at grains_gpu_system::kSoloMax.
 constexpr int kSoloThreads = 256;
 constexpr int kSoloBodies = 64;
 
@@ -41,9 +43,10 @@ constexpr int kSoloBodies = 64;
 // are taken up by one wave, once per phase: every agent-scope fence writes back
 // or invalidates the XCD's L2, and with a fence per wave and piece they were
 // what a rebuild waited for (a step of a gas of 64,000 that rebuilds every
-// fourth or fifth time 87 us, 70 with one).  The stores of all waves have reached the L2
-// (s_waitcnt) before the barrier, so the one write-back covers them; the count
-// is raised when it has ended, which is waited for explicitly: with no store
+// fourth or fifth time 87 us, 70 with one).  The stores of all waves have
+// reached the L2 (s_waitcnt) before the barrier, so the one write-back covers
+// them; the count is raised when it has ended, which is waited for explicitly:
+// with no store
 // of this wave outstanding the compiler leaves that wait out.
 __device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void wait_pieces(int* done, int count) {
@@ -460,9 +463,26 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
   sphere_tail<MODE>(P, S, G, sp, st, VS, s, cx, cv, kin, self[10][tid], P.crust[s], P.cfac[s], P.inertia[s], F, Tq);
 }
 
+template <int MODE, bool MIXED>
+static void launch_solo_mode(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
+                             const HookeModel* models, const StepParams& sp, DevStatus* st, int* pairs,
+                             const NbrList& L, const VerletState& V, hipStream_t stream) {
+  const dim3 grid((sp.n + kSoloBodies - 1) / kSoloBodies), block(kSoloThreads);
+  if (sp.mem.cap)
+    hipLaunchKernelGGL((k_forces_solo<MODE, MIXED, true>), grid, block, 0, stream, P, S, G, obs, models, sp, st, pairs, L, V);
+  else
+    hipLaunchKernelGGL((k_forces_solo<MODE, MIXED, false>), grid, block, 0, stream, P, S, G, obs, models, sp, st, pairs, L, V);
+}
+
+// (instantiated once per precision, each in a translation unit of its own)
 template <bool MIXED>
 hipError_t launch_solo_t(int mode, const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
                          const HookeModel* models, const StepParams& sp, DevStatus* st, int* pairs, const NbrList& L,
-                         const VerletState& V, hipStream_t stream);
+                         const VerletState& V, hipStream_t stream) {
+  if (mode == kForcesOnly) launch_solo_mode<kForcesOnly, MIXED>(P, S, G, obs, models, sp, st, pairs, L, V, stream);
+  else if (mode == kForcesKick) launch_solo_mode<kForcesKick, MIXED>(P, S, G, obs, models, sp, st, pairs, L, V, stream);
+  else launch_solo_mode<kFused, MIXED>(P, S, G, obs, models, sp, st, pairs, L, V, stream);
+  return hipGetLastError();
+}
 
 }  // namespace dem

@@ -3,26 +3,10 @@
 
 namespace dem {
 
-template <int MODE>
-static void launch_mode(const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
-                        const HookeModel* models, const StepParams& sp, DevStatus* st, int* pairs, const NbrList& L,
-                        const VerletState& V, hipStream_t stream) {
-  const dim3 grid((sp.n + kSoloBodies - 1) / kSoloBodies), block(kSoloThreads);
-  if (sp.mem.cap)
-    hipLaunchKernelGGL((k_forces_solo<MODE, true, true>), grid, block, 0, stream, P, S, G, obs, models, sp, st, pairs, L, V);
-  else
-    hipLaunchKernelGGL((k_forces_solo<MODE, true, false>), grid, block, 0, stream, P, S, G, obs, models, sp, st, pairs, L, V);
-}
-
-template <>
-hipError_t launch_solo_t<true>(int mode, const Particles& P, const Sorted& S, const Grid& G, const BoxObstacle* obs,
-                             const HookeModel* models, const StepParams& sp, DevStatus* st, int* pairs,
-                             const NbrList& L, const VerletState& V, hipStream_t stream) {
-  if (mode == kForcesOnly) launch_mode<kForcesOnly>(P, S, G, obs, models, sp, st, pairs, L, V, stream);
-  else if (mode == kForcesKick) launch_mode<kForcesKick>(P, S, G, obs, models, sp, st, pairs, L, V, stream);
-  else launch_mode<kFused>(P, S, G, obs, models, sp, st, pairs, L, V, stream);
-  return hipGetLastError();
-}
+template hipError_t launch_solo_t<true>(int, const Particles&, const Sorted&, const Grid&, const BoxObstacle*, const HookeModel*,
+    const StepParams&, DevStatus*, int*, const NbrList&, const VerletState&, hipStream_t);
+extern template hipError_t launch_solo_t<false>(int, const Particles&, const Sorted&, const Grid&, const BoxObstacle*, const HookeModel*,
+    const StepParams&, DevStatus*, int*, const NbrList&, const VerletState&, hipStream_t);
 
 hipError_t launch_forces_solo(int mode, bool mixed, const Particles& P, const Sorted& S, const Grid& G,
                               const BoxObstacle* obs, const HookeModel* models, const StepParams& sp, DevStatus* st,

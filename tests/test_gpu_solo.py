@@ -78,10 +78,23 @@ def test_rolling_resistance(gpu, precision, model):
 
 
 def test_many_obstacles(gpu):
-    # more walls than the one-launch step keeps as bits: the general launches
+    # more walls than the one-launch step keeps as bits: the general launches.
+    # The six that are touched come last, behind 70 that are not
     wl = bed(300)
-    wl["boxes"] = wl["boxes"] + [((1e-4,) * 3, (0.5e-3 + 1e-3 * (i % 19), 0.5e-3 + 1e-3 * (i // 19), 0.25), None, 5e-5, 0)
-                                 for i in range(70)]
+    wl["boxes"] = [((1e-4,) * 3, (0.5e-3 + 1e-3 * (i % 19), 0.5e-3 + 1e-3 * (i // 19), 0.25), None, 5e-5, 0)
+                   for i in range(70)] + wl["boxes"]
+    g, o = make_gpu(wl), make_oracle(wl)
+    touched = set()
+    for k in (0, 1, 49):
+        g.step(k)
+        o.step(k)
+        po = pair_set(o.pairs())
+        assert pair_set(g.pairs()) == po
+        touched |= {-b - 1 for _, b in po if b < 0}
+        scale = contact_scale(o.state(), o.masses()[2])
+        if k < 2:
+            assert rel_force_error(g.state()["F"], o.state()["F"], scale) <= 1e-12
+    assert len(touched) >= 4 and min(touched) >= 70
     a, _ = run(wl, 0, 32, False, (50,))
     b, _ = run(wl, 0, 32, True, (50,))
     assert np.array_equal(a["x"], b["x"]) and np.array_equal(a["F"], b["F"])
