@@ -106,8 +106,10 @@ namespace {
 // writing the caller's (often fresh) pages is what takes the time, and threads
 // share it.  The copies go through the system's stream and kLanes of the
 // buffers' own, which the first calls make one by one: a stream costs 0.7 ms
-// until its first copy is done, against 0.35 ms for a whole state of 27,000
-// (a state of 1M: 5.5 ms through the system's stream alone, 4.8 with four).
+// until its first copy is done, 3 early in a process, against 0.35 ms for a
+// whole state of 27,000 (a state of 1M: 5.5 ms through the system's stream
+// alone, 4.8 with four; one stream and chunks of 2 MB are as fast there, but 3 %
+// of a pass of 200,000 slower).
 constexpr size_t kSingle = (size_t)2 << 20;
 constexpr size_t kChunk = (size_t)1 << 20;
 constexpr int kThreads = 8;
