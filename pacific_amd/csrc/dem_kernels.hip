@@ -667,14 +667,17 @@ hipError_t launch_detect(const Particles& P, const Sorted& S, const Grid& G, con
   // lanes per particle by the number of particles, as measured (us per launch;
   // 1, 2, 4, 8 lanes): packed polyhedra 343 75, 44, 30, 22; 27,000 45, 29, 22, 20;
   // 200,000 94, 88, 83, 101; polyhedra on a loose lattice 20,000 17, 16, 14, 15;
-  // 60,000 18, 18, 17, 26; 200,000 23, 33, 40, 66; packed spheres 60,000 21, 18,
-  // 17, 21, 200,000 25, 26, 32, 52; gas of 27,000 23, 23, 22, 22, of 60,000
-  // at solid fraction 0.05 18, 18, 19, 22, of 1,000,000 74, 108, 151, 258.  More
-  // lanes overlap the loads of few particles; once there are particles enough,
-  // every lane repeats the search for the cells' runs for little.
+  // 60,000 18, 18, 17, 26; 200,000 24, 35, 42, 67, and as a hopper fills with them
+  // 57, 43, 49, 69, then 84, 55, 55, 74 (where the work list is another launch,
+  // one lane and that launch 29, 67 and 84); packed spheres 60,000 21, 18, 17, 21,
+  // 200,000 25, 26, 32, 52; gas of 27,000 23, 23, 22, 22, of 60,000 at solid
+  // fraction 0.05 18, 18, 19, 22, of 1,000,000 74, 108, 151, 258.  More lanes
+  // overlap the loads of few particles; once there are particles enough, every
+  // lane repeats the search for the cells' runs for little.
   const bool items = P.shape != nullptr;
   if (sp.n <= 32768) launch_detect_lanes<8>(P, S, G, obs, sp, L, st, stream);
   else if (sp.n <= (items ? 65536 : 49152)) launch_detect_lanes<4>(P, S, G, obs, sp, L, st, stream);
+  else if (items) launch_detect_lanes<2>(P, S, G, obs, sp, L, st, stream);
   else launch_detect_lanes<1>(P, S, G, obs, sp, L, st, stream);
   return hipGetLastError();
 }

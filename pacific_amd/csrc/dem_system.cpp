@@ -135,7 +135,7 @@ int grains_gpu_system::allocate() {
   HIPCHECK(this, track(this, &d_models, (size_t)kMaxMaterials * kMaxMaterials));
   HIPCHECK(this, track(this, &d_status, 1));
   rows = RowBuffers::of(device);
-  h_status = rows->status_block();
+  if (!h_status) h_status = rows->status_block();
   if (verlet)
     for (int a = 0; a < 3; ++a) HIPCHECK(this, track(this, &V.xb[a], n));
   V.sync = nullptr;
