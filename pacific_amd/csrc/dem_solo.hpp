@@ -240,7 +240,7 @@ __global__ __launch_bounds__(kSoloThreads) __attribute__((amdgpu_waves_per_eu(2)
   // after an error (which ends the run) the rest of a batch of steps neither
   // rebuilds nor searches, so that it costs little whatever the state has become
   const bool stop = st->stop[cx] != 0;
-  if (!stop && st->rebuild[cx] == st->seq[cx] + 1) solo_rebuild(P, S, VS, L, sp.n, cx, st);
+  if (!stop && VS.stamp == 1 && st->rebuild[cx] == st->seq[cx] + 1) solo_rebuild(P, S, VS, L, sp.n, cx, st);
   if (MODE == kFused) number_next(sp, st, VS);
   const bool mine = tid < B && t0 + tid < sp.n;
   const int s = t0 + tid;

@@ -423,6 +423,14 @@ bool grains_gpu_system::scattered() const {
   return 2 * far > seen;
 }
 
+// Rebuilds the Verlet list if a drift since it was built has found it stale.
+int grains_gpu_system::current_list() {
+  if (!verlet || list_current) return GRAINS_OK;
+  HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), touch.count, true, stream));
+  list_current = true;
+  return GRAINS_OK;
+}
+
 // The particles of the last evaluation that have a contact, for the choice of
 // the next batch's sweep (read_status).
 int grains_gpu_system::count_touched() {
@@ -466,6 +474,9 @@ int grains_gpu_system::sort_storage() {
   }
   // (posr, written anew by the binning, holds what is on its way)
   HIPCHECK(this, launch_permute(a8, a4, S.order, nparticles, S.posr, stream));
+  // the list in the given order does not count as a build
+  HIPCHECK(this, launch_clear(&d_status->n_rebuild, 1, stream));
+  builds_seen = 0;
   return bin_current();
 }
 
@@ -490,9 +501,7 @@ int grains_gpu_system::bin_launch() {
   if (one_launch()) {
     // the force sweep rebuilds the list itself
   } else if (verlet) {
-    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, nbr_list(), touch.count, true,
-                                       stream));
-    list_current = true;
+    if ((e = current_list())) return e;
   } else
     HIPCHECK(this, launch_bin(P, S, grid, nparticles, cur & 1, stream));
   if (prof && (e = mark(prof->bin_ev, prof->nbin))) return e;
@@ -529,7 +538,7 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     // one launch: list rebuild if stale, contacts, forces, integration
     if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
     HIPCHECK(this, launch_forces_solo(mode, cfg.precision == GRAINS_MIXED, P, S, grid, d_obs, d_models, sp, d_status,
-                                      d_pairs, L, vstate(1), stream));
+                                      d_pairs, L, vstate(list_current ? 2 : 1), stream));
     if (prof && (e = mark(prof->force_ev, prof->nforce))) return e;
     list_current = mode != kModeFused;
     if (commit && mem.cap) mem.cur ^= 1;
@@ -541,8 +550,7 @@ int grains_gpu_system::forces(int mode, int first_step, bool commit) {
     return GRAINS_OK;
   }
   // an evaluation of the general sweep: the list must be current
-  if (verlet && !list_current)
-    HIPCHECK(this, launch_verlet_build(P, S, V, nparticles, cur & 1, d_status, L, touch.count, true, stream));
+  if ((e = current_list())) return e;
   const dem::NbrList CL = contact_list();
   // (not for evaluations outside the step loop, nor with extras)
   const dem::TouchList TL =
@@ -1422,7 +1430,10 @@ int grains_gpu_set_neighbor_list(grains_gpu_system* s, int capacity, double skin
 
 int grains_gpu_neighbor_stats(grains_gpu_system* s, double* skin, long* builds) {
   if (!s || !s->initialized) return GRAINS_ARGUMENT_ERROR;
-  int e = s->check_status();
+  HIPCHECK(s, hipSetDevice(s->device));
+  // a build that the next step's launch would make counts from the drift on
+  int e = s->current_list();
+  if (!e) e = s->check_status();
   if (e) return e;
   if (skin) *skin = s->verlet ? s->V.skin : 0.;
   if (builds) *builds = s->verlet ? s->last_status.n_rebuild : 0;

@@ -159,6 +159,7 @@ struct grains_gpu_system {
   // no drift since the Verlet list was built or found current (an evaluation of
   // the general sweep finds out unless)
   bool list_current = false;
+  int current_list();
   // the number of the last positions written (DevStatus::seq counts along on
   // the device, so that captured steps need no new arguments)
   int step_number = 0;

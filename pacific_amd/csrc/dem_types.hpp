@@ -179,7 +179,7 @@ struct VerletState {
   double* xb[3];  // positions at the last build (storage order)
   double skin;
   double half2;   // (skin / 2)^2
-  int stamp;      // > 0: the staleness check is on; 0 = no Verlet list; < 0 wrap only
+  int stamp;      // > 0: the staleness check is on (2: the list is current); 0 = no Verlet list; < 0 wrap only
   int pad;
   RebuildSync* sync;  // [2], of a system whose force sweep rebuilds the list itself
 };

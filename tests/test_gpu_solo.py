@@ -253,3 +253,32 @@ def test_rebuilds_often_and_seldom(gpu, precision):
             assert np.array_equal(sa[f], sb[f]), f
         assert a.neighbor_stats() == b.neighbor_stats()
     assert a.neighbor_stats()[1] > 20
+
+
+@pytest.mark.parametrize("precision", [0, MIXED])
+@pytest.mark.parametrize("scheme", [0, 1, 2, 3])
+def test_list_builds_are_counted_as_by_general_launches(gpu, scheme, precision):
+    # steps, states set and evaluations in between; a list of 8 entries takes
+    # the general launches, which rebuild right after the drift (after an
+    # explicit step also where a state set next builds it again: left out)
+    wl = gas(700)
+    a = make_gpu(wl, scheme=scheme, precision=precision, record=False)
+    b = make_gpu(wl, scheme=scheme, precision=precision, record=False, nbr=8)
+    rng = np.random.default_rng(scheme)
+    for k in range(24):
+        op, m = int(rng.integers(0, 5)), int(rng.choice([1, 2, 5]))
+        for g in (a, b):
+            g.step(m)
+            if op == 1:
+                g.compute_forces()
+            if op == 2:
+                g.force_sums()
+            if op == 3 and scheme == 0:
+                s = g.state()
+                g.set_state(x=s["x"], v=0.9 * s["v"], recompute=bool(k % 2))
+        assert a.neighbor_stats() == b.neighbor_stats(), k
+        if k % 3 == 0:
+            sa, sb = a.state(), b.state()
+            for f in ("x", "v", "w", "F", "T"):
+                assert np.array_equal(sa[f], sb[f]), (k, f)
+    assert a.neighbor_stats()[1] > 5

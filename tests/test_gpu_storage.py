@@ -59,3 +59,21 @@ def test_random_order_against_oracle(gpu, kind, skin):
     g.set_hydro_ft(ft)
     g.compute_forces()
     assert np.max(np.abs(g.state()["F"] - f0 - ft[:, :3])) <= 1e-15 * np.max(np.abs(f0))
+
+
+@pytest.mark.parametrize("skin", [None, 0.0])
+def test_list_builds_are_counted_as_in_the_given_order(gpu, skin):
+    # the list built to find the order is no build of the run
+    rng = np.random.default_rng(4)
+    wl = workloads.periodic_gas(5000, sigma=0.6, phi=0.25)
+    order = rng.permutation(5000)
+    other = dict(wl)
+    for k in ("radius", "density", "crust", "material", "x", "v", "w"):
+        other[k] = np.asarray(wl[k])[order]
+    a, b = make_gpu(wl, skin=skin, record=False), make_gpu(other, skin=skin, record=False)
+    for steps in (0, 40):
+        a.step(steps)
+        b.step(steps)
+        builds = a.neighbor_stats()[1]
+        assert b.neighbor_stats()[1] == builds
+        assert builds == 0 if skin == 0.0 else builds >= (1 if steps == 0 else 3)
