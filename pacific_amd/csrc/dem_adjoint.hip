@@ -445,7 +445,7 @@ int grains_gpu_adjoint_backward(grains_gpu_system* s, int matA, int matB, const 
   ACHECK(s, s->rows->down(out, s->P.id, N, s->stream));
   if (grad_params) {
     std::vector<double> gth(3 * n);
-    ACHECK(s, hipMemcpy(gth.data(), A.gth, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
+    ACHECK(s, dem::copy_sync(gth.data(), A.gth, 3 * n * sizeof(double), hipMemcpyDeviceToHost));
     double gkn = 0., gbeta = 0., gmu = 0.;
     for (size_t i = 0; i < n; ++i) {
       gkn += gth[3 * i];

@@ -429,7 +429,7 @@ hipError_t balloc(grains_gpu_batch* b, T** p, size_t n) {
 template <typename T>
 hipError_t up(T* dst, const std::vector<T>& v) {
   if (v.empty()) return hipSuccess;
-  return hipMemcpy(dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+  return dem::copy_sync(dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
 }
 
 }  // namespace
@@ -656,10 +656,10 @@ int grains_gpu_batch_create(grains_gpu_system* const* systems, int nsys, int pre
   BCHECK(b, balloc(b, &S.sid, n));
   BCHECK(b, balloc(b, &S.posr, 4 * n));
   S.block_sums = nullptr;
-  BCHECK(b, hipMemset(S.count, 0, sizeof(int) * (size_t)std::max<long>(cells, 1)));
-  BCHECK(b, hipMemset(S.start, 0, sizeof(int) * ((size_t)cells + nsys)));
-  BCHECK(b, hipMemset(S.tmp_order, 0, sizeof(int) * n));
-  BCHECK(b, hipMemset(S.order, 0, sizeof(int) * n));
+  BCHECK(b, dem::fill_sync(S.count, 0, sizeof(int) * (size_t)std::max<long>(cells, 1)));
+  BCHECK(b, dem::fill_sync(S.start, 0, sizeof(int) * ((size_t)cells + nsys)));
+  BCHECK(b, dem::fill_sync(S.tmp_order, 0, sizeof(int) * n));
+  BCHECK(b, dem::fill_sync(S.order, 0, sizeof(int) * n));
   BCHECK(b, balloc(b, &b->d_sys, (size_t)nsys));
   BCHECK(b, up(b->d_sys, hs));
   // flat mode
@@ -676,7 +676,7 @@ int grains_gpu_batch_create(grains_gpu_system* const* systems, int nsys, int pre
     b->ncells = (int)cells;
     b->Sf = S;
     BCHECK(b, balloc(b, &b->Sf.start, (size_t)cells + 1));
-    BCHECK(b, hipMemset(b->Sf.start, 0, sizeof(int) * ((size_t)cells + 1)));
+    BCHECK(b, dem::fill_sync(b->Sf.start, 0, sizeof(int) * ((size_t)cells + 1)));
     BCHECK(b, balloc(b, &b->Sf.block_sums, (size_t)scan_blocks((int)cells) + 1));
     for (int a = 0; a < 3; ++a) {
       BCHECK(b, balloc(b, &P.v[1][a], n));
@@ -694,7 +694,7 @@ int grains_gpu_batch_create(grains_gpu_system* const* systems, int nsys, int pre
   BCHECK(b, balloc(b, &b->d_status, 1));
   b->rows = RowBuffers::of(b->device);
   b->h_status = b->rows->status_block();
-  BCHECK(b, hipMemset(b->d_status, 0, sizeof(DevStatus)));
+  BCHECK(b, dem::fill_sync(b->d_status, 0, sizeof(DevStatus)));
   b->time = systems[0]->cfg.t_start;
   int e = b->launch(0, 0);  // bin + initial forces
   if (e) return e;
@@ -729,10 +729,12 @@ int grains_gpu_batch_step(grains_gpu_batch* b, int nsteps, int chunk) {
         (void)hipGraphDestroy(b->graph);
         b->exec = nullptr;
       }
+      std::unique_lock<std::mutex> hold(capture_lock());
       BCHECK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
       int e = b->launch(1, chunk);
       hipGraph_t g = nullptr;
       hipError_t ec = hipStreamEndCapture(b->stream, &g);
+      hold.unlock();
       if (e) return e;
       BCHECK(b, ec);
       b->graph = g;
@@ -756,10 +758,12 @@ int grains_gpu_batch_step_timed(grains_gpu_batch* b, int nsteps, int chunk, doub
   if (chunk > 0 && nsteps >= chunk && (!b->exec || b->graph_steps != chunk)) {
     int e = grains_gpu_batch_step(b, 0, chunk);
     if (e) return e;
+    std::unique_lock<std::mutex> hold(capture_lock());
     BCHECK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     e = b->launch(1, chunk);
     hipGraph_t g = nullptr;
     hipError_t ec = hipStreamEndCapture(b->stream, &g);
+    hold.unlock();
     if (e) return e;
     BCHECK(b, ec);
     if (b->exec) {

@@ -19,6 +19,19 @@
 
 namespace dem {
 
+std::mutex& capture_lock() {
+  static std::mutex m;
+  return m;
+}
+hipError_t copy_sync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+  std::lock_guard<std::mutex> hold(capture_lock());
+  return hipMemcpy(dst, src, bytes, kind);
+}
+hipError_t fill_sync(void* dst, int value, size_t bytes) {
+  std::lock_guard<std::mutex> hold(capture_lock());
+  return hipMemset(dst, value, bytes);
+}
+
 __global__ __launch_bounds__(256) void k_rows_out(RowMap m, const int* __restrict__ id, int n,
                                                   double* __restrict__ out) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -296,18 +309,18 @@ hipError_t RowBuffers::plain(const RowIO& io, size_t first, bool to_host, const 
   std::vector<int> ids((size_t)n);
   std::vector<double> buf((size_t)n);
   hipError_t e = hipStreamSynchronize(stream);
-  if (e == hipSuccess) e = hipMemcpy(ids.data(), id, sizeof(int) * n, hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = dem::copy_sync(ids.data(), id, sizeof(int) * n, hipMemcpyDeviceToHost);
   for (size_t k = first; e == hipSuccess && k < io.segs().size(); ++k) {
     const RowIO::Seg& s = io.segs()[k];
     for (int c = 0; c < s.width && e == hipSuccess; ++c) {
       auto row = [&](int i) -> double& { return s.host[(size_t)s.width * (ids[i] - 1) + c]; };
       if (to_host) {
-        e = hipMemcpy(buf.data(), s.comp[c], sizeof(double) * n, hipMemcpyDeviceToHost);
+        e = dem::copy_sync(buf.data(), s.comp[c], sizeof(double) * n, hipMemcpyDeviceToHost);
         if (e == hipSuccess)
           for (int i = 0; i < n; ++i) row(i) = buf[i];
       } else {
         for (int i = 0; i < n; ++i) buf[i] = row(i);
-        e = hipMemcpy(s.comp[c], buf.data(), sizeof(double) * n, hipMemcpyHostToDevice);
+        e = dem::copy_sync(s.comp[c], buf.data(), sizeof(double) * n, hipMemcpyHostToDevice);
       }
     }
   }

@@ -13,6 +13,13 @@
 
 namespace dem {
 
+// Synchronous copies and fills go through the legacy stream, which ends the
+// capture that another thread has under way on a stream of its own, and fails
+// itself: captures hold this lock, and so does each of these.
+std::mutex& capture_lock();
+hipError_t copy_sync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind);
+hipError_t fill_sync(void* dst, int value, size_t bytes);
+
 // Component c of the particle in storage index s <-> element
 // base[c] + stride[c] * (id[s] - 1) of one buffer of rows.
 struct RowMap {

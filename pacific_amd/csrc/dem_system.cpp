@@ -310,28 +310,28 @@ int grains_gpu_system::upload() {
   std::vector<double> buf((size_t)n);
   auto up = [&](double* dst, const std::vector<double>& src, int stride, int comp) -> hipError_t {
     for (int i = 0; i < n; ++i) buf[i] = src[(size_t)stride * i + comp];
-    return hipMemcpy(dst, buf.data(), sizeof(double) * n, hipMemcpyHostToDevice);
+    return dem::copy_sync(dst, buf.data(), sizeof(double) * n, hipMemcpyHostToDevice);
   };
   for (int a = 0; a < 3; ++a) {
     HIPCHECK(this, up(P.x[0][a], h_x, 3, a));
     HIPCHECK(this, up(P.v[0][a], h_v, 3, a));
     HIPCHECK(this, up(P.w[0][a], h_w, 3, a));
     HIPCHECK(this, up(P.wb[a], h_wb, 3, a));
-    HIPCHECK(this, hipMemset(P.F[a], 0, sizeof(double) * n));
-    HIPCHECK(this, hipMemset(P.T[a], 0, sizeof(double) * n));
+    HIPCHECK(this, dem::fill_sync(P.F[a], 0, sizeof(double) * n));
+    HIPCHECK(this, dem::fill_sync(P.T[a], 0, sizeof(double) * n));
     if (P.v_nm2[a]) {
-      HIPCHECK(this, hipMemset(P.v_nm2[a], 0, sizeof(double) * n));
-      HIPCHECK(this, hipMemset(P.dUdt_nm2[a], 0, sizeof(double) * n));
-      HIPCHECK(this, hipMemset(P.wb_nm2[a], 0, sizeof(double) * n));
-      HIPCHECK(this, hipMemset(P.dWdt_nm2[a], 0, sizeof(double) * n));
+      HIPCHECK(this, dem::fill_sync(P.v_nm2[a], 0, sizeof(double) * n));
+      HIPCHECK(this, dem::fill_sync(P.dUdt_nm2[a], 0, sizeof(double) * n));
+      HIPCHECK(this, dem::fill_sync(P.wb_nm2[a], 0, sizeof(double) * n));
+      HIPCHECK(this, dem::fill_sync(P.dWdt_nm2[a], 0, sizeof(double) * n));
     }
   }
   for (int a = 0; a < 4; ++a) HIPCHECK(this, up(P.q[a], h_q, 4, a));
-  HIPCHECK(this, hipMemcpy(P.rad, h_rad.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-  HIPCHECK(this, hipMemcpy(P.mass, h_mass.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-  HIPCHECK(this, hipMemcpy(P.inertia, h_inertia.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-  HIPCHECK(this, hipMemcpy(P.crust, h_crust.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-  HIPCHECK(this, hipMemcpy(P.wfac, h_wfac.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.rad, h_rad.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.mass, h_mass.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.inertia, h_inertia.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.crust, h_crust.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.wfac, h_wfac.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   auto uniform = [&](const std::vector<double>& a) {
     for (int i = 1; i < n; ++i)
       if (a[i] != a[0]) return -1.;
@@ -339,26 +339,26 @@ int grains_gpu_system::upload() {
   };
   crust_all = uniform(h_crust);
   cfac_all = uniform(h_cfac);
-  HIPCHECK(this, hipMemcpy(P.cfac, h_cfac.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-  HIPCHECK(this, hipMemcpy(P.req, h_req.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.cfac, h_cfac.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.req, h_req.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   std::vector<int> ids((size_t)n);
   for (int i = 0; i < n; ++i) ids[i] = i + 1;
-  HIPCHECK(this, hipMemcpy(P.id, ids.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  HIPCHECK(this, hipMemcpy(P.mat, h_mat.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.id, ids.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(P.mat, h_mat.data(), sizeof(int) * n, hipMemcpyHostToDevice));
   if (!obstacles.empty())
-    HIPCHECK(this, hipMemcpy(d_obs, obstacles.data(), sizeof(BoxObstacle) * obstacles.size(),
+    HIPCHECK(this, dem::copy_sync(d_obs, obstacles.data(), sizeof(BoxObstacle) * obstacles.size(),
                              hipMemcpyHostToDevice));
-  HIPCHECK(this, hipMemcpy(d_models, models, sizeof(models), hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(d_models, models, sizeof(models), hipMemcpyHostToDevice));
   if (has_shapes()) {
-    HIPCHECK(this, hipMemcpy(P.shape, h_shape.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+    HIPCHECK(this, dem::copy_sync(P.shape, h_shape.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     for (int j = 0; j < 9; ++j) {
       HIPCHECK(this, up(P.B[0][j], h_B, 9, j));
       HIPCHECK(this, up(P.B[1][j], h_B, 9, j));
     }
     for (int a = 0; a < 3; ++a) HIPCHECK(this, up(P.I3[a], h_I3, 3, a));
-    HIPCHECK(this, hipMemcpy(d_shapes, shapes.data(), sizeof(ShapeDesc) * shapes.size(), hipMemcpyHostToDevice));
+    HIPCHECK(this, dem::copy_sync(d_shapes, shapes.data(), sizeof(ShapeDesc) * shapes.size(), hipMemcpyHostToDevice));
     if (!shape_verts.empty())
-      HIPCHECK(this, hipMemcpy(d_verts, shape_verts.data(), sizeof(double) * shape_verts.size(),
+      HIPCHECK(this, dem::copy_sync(d_verts, shape_verts.data(), sizeof(double) * shape_verts.size(),
                                hipMemcpyHostToDevice));
   }
   cur = 0;
@@ -684,6 +684,7 @@ int grains_gpu_system::graph_chunk(bool& done) {
     }
   const int cur0 = cur, mem0 = mem.cur, number0 = step_number;
   const double ft0 = force_time;
+  std::unique_lock<std::mutex> hold(capture_lock());
   HIPCHECK(this, hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
   int e = GRAINS_OK;
   for (int j = 0; j < kGraphSteps && !e; ++j) {
@@ -693,6 +694,7 @@ int grains_gpu_system::graph_chunk(bool& done) {
   }
   hipGraph_t graph = nullptr;
   const hipError_t ce = hipStreamEndCapture(stream, &graph);
+  hold.unlock();
   hipGraphExec_t exec = nullptr;
   hipError_t ie = hipErrorUnknown;
   if (!e && ce == hipSuccess && graph && cur == cur0 && mem.cur == mem0)
@@ -818,8 +820,8 @@ int grains_gpu_system::grow(const std::function<int()>& add) {
   }
   double stat[8];
   DevStatus st;
-  HIPCHECK(this, hipMemcpy(stat, d_stat_tot, sizeof(stat), hipMemcpyDeviceToHost));
-  HIPCHECK(this, hipMemcpy(&st, d_status, sizeof(st), hipMemcpyDeviceToHost));
+  HIPCHECK(this, dem::copy_sync(stat, d_stat_tot, sizeof(stat), hipMemcpyDeviceToHost));
+  HIPCHECK(this, dem::copy_sync(&st, d_status, sizeof(st), hipMemcpyDeviceToHost));
   const double ft = force_time;
   free_adjoint();
   free_device();
@@ -834,19 +836,19 @@ int grains_gpu_system::grow(const std::function<int()>& add) {
   // weight of the evaluation at initialisation (it touches nothing)
   const size_t m = (size_t)nparticles;
   std::vector<int> ids(m);
-  HIPCHECK(this, hipMemcpy(ids.data(), P.id, sizeof(int) * m, hipMemcpyDeviceToHost));
+  HIPCHECK(this, dem::copy_sync(ids.data(), P.id, sizeof(int) * m, hipMemcpyDeviceToHost));
   std::vector<double> buf(m);
   for (int a = 0; a < 3; ++a)
     for (int k = 0; k < 2; ++k) {
       double* dev = k ? P.T[a] : P.F[a];
       const std::vector<double>& old = k ? T : F;
-      HIPCHECK(this, hipMemcpy(buf.data(), dev, sizeof(double) * m, hipMemcpyDeviceToHost));
+      HIPCHECK(this, dem::copy_sync(buf.data(), dev, sizeof(double) * m, hipMemcpyDeviceToHost));
       for (size_t i = 0; i < m; ++i)
         if ((size_t)(ids[i] - 1) < n) buf[i] = old[3 * (size_t)(ids[i] - 1) + a];
-      HIPCHECK(this, hipMemcpy(dev, buf.data(), sizeof(double) * m, hipMemcpyHostToDevice));
+      HIPCHECK(this, dem::copy_sync(dev, buf.data(), sizeof(double) * m, hipMemcpyHostToDevice));
     }
-  HIPCHECK(this, hipMemcpy(d_stat_tot, stat, sizeof(stat), hipMemcpyHostToDevice));
-  HIPCHECK(this, hipMemcpy(d_status, &st, sizeof(st), hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(d_stat_tot, stat, sizeof(stat), hipMemcpyHostToDevice));
+  HIPCHECK(this, dem::copy_sync(d_status, &st, sizeof(st), hipMemcpyHostToDevice));
   force_time = ft;
   return GRAINS_OK;
 }
@@ -887,7 +889,7 @@ static int set_model(grains_gpu_system* s, int matA, int matB, const HookeModel&
     s->models[matB * kMaxMaterials + matA] = m;
   }
   if (s->initialized)
-    HIPCHECK(s, hipMemcpy(s->d_models, s->models, sizeof(s->models), hipMemcpyHostToDevice));
+    HIPCHECK(s, dem::copy_sync(s->d_models, s->models, sizeof(s->models), hipMemcpyHostToDevice));
   return GRAINS_OK;
 }
 
@@ -1323,8 +1325,8 @@ int grains_gpu_force_sums(grains_gpu_system* s, double* out) {
   if ((e = s->check_status())) return e;
   std::vector<int> ids((size_t)n);
   std::vector<double> buf((size_t)n);
-  HIPCHECK(s, hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost));
-  HIPCHECK(s, hipMemcpy(buf.data(), s->d_fsum, sizeof(double) * n, hipMemcpyDeviceToHost));
+  HIPCHECK(s, dem::copy_sync(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost));
+  HIPCHECK(s, dem::copy_sync(buf.data(), s->d_fsum, sizeof(double) * n, hipMemcpyDeviceToHost));
   for (int i = 0; i < n; ++i) out[ids[i] - 1] = buf[i];
   return GRAINS_OK;
 }
@@ -1480,7 +1482,7 @@ int grains_gpu_get_pairs(grains_gpu_system* s, int* buf, size_t cap, size_t* n) 
   *n = np;
   if (buf && cap) {
     size_t m = std::min(np, cap);
-    HIPCHECK(s, hipMemcpy(buf, s->d_pairs, sizeof(int) * 2 * m, hipMemcpyDeviceToHost));
+    HIPCHECK(s, dem::copy_sync(buf, s->d_pairs, sizeof(int) * 2 * m, hipMemcpyDeviceToHost));
   }
   return GRAINS_OK;
 }

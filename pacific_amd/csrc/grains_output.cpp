@@ -122,7 +122,7 @@ int grains_gpu_coordination_at_state(grains_gpu_system* s, int* out) {
   if (hipStreamSynchronize(s->stream) != hipSuccess) return fail(s, GRAINS_DEVICE_ERROR, "stream sync failed");
   for (int c = 0; c < 6 && n; ++c) {
     double* src = c < 3 ? s->P.F[c] : s->P.T[c - 3];
-    if (hipMemcpy(ft.data() + c * n, src, sizeof(double) * n, hipMemcpyDeviceToHost) != hipSuccess)
+    if (dem::copy_sync(ft.data() + c * n, src, sizeof(double) * n, hipMemcpyDeviceToHost) != hipSuccess)
       return fail(s, GRAINS_DEVICE_ERROR, "torsor copy failed");
   }
   const int rec0 = s->record_pairs;
@@ -132,7 +132,7 @@ int grains_gpu_coordination_at_state(grains_gpu_system* s, int* out) {
   grains_gpu_set_record_pairs(s, rec0);
   for (int c = 0; c < 6 && n; ++c) {
     double* dst = c < 3 ? s->P.F[c] : s->P.T[c - 3];
-    if (hipMemcpy(dst, ft.data() + c * n, sizeof(double) * n, hipMemcpyHostToDevice) != hipSuccess)
+    if (dem::copy_sync(dst, ft.data() + c * n, sizeof(double) * n, hipMemcpyHostToDevice) != hipSuccess)
       return fail(s, GRAINS_DEVICE_ERROR, "torsor copy failed");
   }
   return e;

@@ -123,13 +123,13 @@ int download(grains_gpu_system* s, HostState& h) {
     for (size_t i = 0; i < n; ++i) quat_matrix(&h.q[4 * i], &h.B[9 * i]);
   }
   std::vector<int> ids(n);
-  if (n && hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost) != hipSuccess)
+  if (n && dem::copy_sync(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost) != hipSuccess)
     return fail(s, GRAINS_DEVICE_ERROR, "reload: id download failed");
   std::vector<double> buf(n);
   auto down3 = [&](double* const* src, std::vector<double>& dst) -> bool {
     dst.assign(3 * n, 0.);
     for (int a = 0; a < 3; ++a) {
-      if (hipMemcpy(buf.data(), src[a], sizeof(double) * n, hipMemcpyDeviceToHost) != hipSuccess) return false;
+      if (dem::copy_sync(buf.data(), src[a], sizeof(double) * n, hipMemcpyDeviceToHost) != hipSuccess) return false;
       for (size_t i = 0; i < n; ++i) dst[3 * (size_t)(ids[i] - 1) + a] = buf[i];
     }
     return true;
@@ -145,13 +145,13 @@ int download(grains_gpu_system* s, HostState& h) {
     const int c = cm.cur;
     std::vector<int> cnt(n), key((size_t)cm.cap * n);
     std::vector<double> f[9];
-    bool ok = hipMemcpy(cnt.data(), cm.n[c], sizeof(int) * n, hipMemcpyDeviceToHost) == hipSuccess &&
-              hipMemcpy(key.data(), cm.key[c], sizeof(int) * key.size(), hipMemcpyDeviceToHost) == hipSuccess;
+    bool ok = dem::copy_sync(cnt.data(), cm.n[c], sizeof(int) * n, hipMemcpyDeviceToHost) == hipSuccess &&
+              dem::copy_sync(key.data(), cm.key[c], sizeof(int) * key.size(), hipMemcpyDeviceToHost) == hipSuccess;
     for (int a = 0; a < 3 && ok; ++a) {
       const double* srcs[3] = {cm.kd[c][a], cm.pn[c][a], cm.sr[c][a]};
       for (int k = 0; k < 3 && ok; ++k) {
         f[3 * k + a].resize(key.size());
-        ok = hipMemcpy(f[3 * k + a].data(), srcs[k], sizeof(double) * key.size(), hipMemcpyDeviceToHost) ==
+        ok = dem::copy_sync(f[3 * k + a].data(), srcs[k], sizeof(double) * key.size(), hipMemcpyDeviceToHost) ==
              hipSuccess;
       }
     }
@@ -531,13 +531,13 @@ int grains_gpu_load_reload(grains_gpu_system* s, const char* file_c) {
   if (s->has_shapes() && (e = grains_gpu_set_basis(s, h.B.data()))) return e;
   if ((e = grains_gpu_set_state(s, h.x.data(), h.v.data(), h.w.data(), h.q.data(), 0))) return e;
   std::vector<int> ids(n);
-  if (n && hipMemcpy(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost) != hipSuccess)
+  if (n && dem::copy_sync(ids.data(), s->P.id, sizeof(int) * n, hipMemcpyDeviceToHost) != hipSuccess)
     return fail(s, GRAINS_DEVICE_ERROR, "reload: id download failed");
   std::vector<double> buf(n);
   auto up3 = [&](double* const* dst, const std::vector<double>& src) -> bool {
     for (int a = 0; a < 3; ++a) {
       for (size_t si = 0; si < n; ++si) buf[si] = src[3 * (size_t)(ids[si] - 1) + a];
-      if (hipMemcpy(dst[a], buf.data(), sizeof(double) * n, hipMemcpyHostToDevice) != hipSuccess) return false;
+      if (dem::copy_sync(dst[a], buf.data(), sizeof(double) * n, hipMemcpyHostToDevice) != hipSuccess) return false;
     }
     return true;
   };
@@ -569,12 +569,12 @@ int grains_gpu_load_reload(grains_gpu_system* s, const char* file_c) {
         }
       }
     }
-    bool ok = hipMemcpy(cm.n[c], cnt.data(), sizeof(int) * n, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(cm.key[c], key.data(), sizeof(int) * key.size(), hipMemcpyHostToDevice) == hipSuccess;
+    bool ok = dem::copy_sync(cm.n[c], cnt.data(), sizeof(int) * n, hipMemcpyHostToDevice) == hipSuccess &&
+              dem::copy_sync(cm.key[c], key.data(), sizeof(int) * key.size(), hipMemcpyHostToDevice) == hipSuccess;
     for (int a = 0; a < 3 && ok; ++a) {
       double* dsts[3] = {cm.kd[c][a], cm.pn[c][a], cm.sr[c][a]};
       for (int k = 0; k < 3 && ok; ++k)
-        ok = hipMemcpy(dsts[k], fv[3 * k + a].data(), sizeof(double) * key.size(), hipMemcpyHostToDevice) ==
+        ok = dem::copy_sync(dsts[k], fv[3 * k + a].data(), sizeof(double) * key.size(), hipMemcpyHostToDevice) ==
              hipSuccess;
     }
     if (!ok) return fail(s, GRAINS_DEVICE_ERROR, "reload: contact memory upload failed");

@@ -7,6 +7,7 @@ contacts than lanes, lists too short for their neighbours (searched in their
 cells), contact memory, and the size above which the general launches run
 anyway."""
 import ctypes
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -282,3 +283,23 @@ def test_list_builds_are_counted_as_by_general_launches(gpu, scheme, precision):
             for f in ("x", "v", "w", "F", "T"):
                 assert np.array_equal(sa[f], sb[f]), (k, f)
     assert a.neighbor_stats()[1] > 5
+
+
+def test_systems_stepping_at_once(gpu):
+    # one-launch steps with rebuilds of several systems on their own streams,
+    # from four threads: the same bits as one after the other
+    sizes = (700, 4097, 8000, 20000)
+
+    def work(n):
+        g = make_gpu(gas(n), precision=MIXED if n == 8000 else 0, record=False)
+        for k in (1, 70, 2, 70):
+            g.step(k)
+        return g.state(), g.neighbor_stats()
+
+    alone = [work(n) for n in sizes]
+    with ThreadPoolExecutor(4) as pool:
+        together = list(pool.map(work, sizes))
+    for (a, na), (b, nb) in zip(alone, together):
+        assert na == nb and na[1] >= 3
+        for f in ("x", "v", "w", "F", "T"):
+            assert np.array_equal(a[f], b[f]), f
